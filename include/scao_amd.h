@@ -38,7 +38,7 @@
 extern "C" {
 #endif
 
-#define SCAO_ABI_VERSION 12
+#define SCAO_ABI_VERSION 13
 
 enum scao_status { SCAO_OK = 0, SCAO_ERR_INVALID = 1, SCAO_ERR_HIP = 2 };
 enum scao_dtype { SCAO_F32 = 0, SCAO_BF16 = 1, SCAO_F16 = 2 };
@@ -122,6 +122,16 @@ typedef struct scao_leaf_desc {
                                block-diagonal split): Sl is its m*n diag EMA, no
                                U/S/T/Delta/W, k = 0; it takes delta tasks (its
                                norm partials) and masked apply tasks only      */
+/* Row parts of the projection (bits 8..15, 0 or 1: whole rows) and column
+ * chunks of the delta stage, k rounded up to 64 columns each (bits 16..23, 0:
+ * one task per 64x64 tile; else tiles of 16 rows x 64 columns).  With parts >
+ * 1, T is followed by that many planes of k x n floats (rounded up to 4) and
+ * the delta stage is chunked; with chunks > 0, Delta is followed by that many
+ * planes of k x k floats (rounded up to 4).                                   */
+#define SCAO_LF_NSPLIT_SHIFT 8
+#define SCAO_LF_DCHUNK_SHIFT 16
+#define SCAO_LF_GET_NSPLIT(f) ((((f) >> 8) & 255) > 1 ? (((f) >> 8) & 255) : 1)
+#define SCAO_LF_GET_DCHUNK(f) (((f) >> 16) & 255)
 
 /* A unit of work: (leaf or param, two tile coordinates, reduction slot). */
 typedef struct scao_task {
@@ -203,19 +213,25 @@ int scao_int8_ema_update(int8_t* q, double scale_in, const float* new_val, doubl
                          int64_t n, double* scale_out, void* scratch, void* stream);
 
 /* ---- batched step: Phase 2 (preconditioned Adan) ---------------------- */
-/* A1  T = U_l^T G for (leaf, 256-column strip, 64-row chunk of T); also
- *     ||g||^2 (chunk 0) and ||p*decay||^2 (chunk 0 of LARS params) into slots.
- *     variant = (fast ? 1 : 0) | (p norm ? 2 : 0) | (tall ? 4 : 0)
- *     | (wide ? 8 : 0): "fast" tasks promise fp32 data, SCAO_LF_VEC4, a full
- *     256-column strip, a full 64-row chunk of T and m % 32 == 0, and run on
- *     the bf16 matrix cores with fp32 products (three-way bf16 splits); "p
- *     norm" tasks are the chunk-0 tasks of LARS params; "tall" tasks (fast
- *     only) cover 128 rows of T from b = c0, a multiple of 128, with
- *     c0 + 128 <= k; "wide" tasks (fast only, not tall) cover 256 rows of T
- *     from b = c0, a multiple of 256, with c0 + 256 <= k. */
+/* A1  T = U_l^T G for (leaf, 256-column strip a, row of T and part b); also
+ *     ||g||^2 (c0 = 0) and ||p*decay||^2 (c0 = 0 of LARS params) into slots.
+ *     b = c0 + (part << 16): rows c0 .. of T over the part's rows of G
+ *     (SCAO_LF_NSPLIT_SHIFT: rows 32 ceil(m / (32 parts)) at a time).
+ *     variant = (whole ? 1 : 0) | (p norm ? 2 : 0) | (128 rows of T ? 4 : 0)
+ *     | (256 rows of T ? 8 : 0) | (bf16 ? 16 : 0) | (fp16 ? 32 : 0).  "whole"
+ *     tasks promise that type (fp32 without bits 16 and 32) for parameter and
+ *     gradient, a full 256-column strip, a part whose rows are a multiple of
+ *     32, a full chunk of T (c0 a multiple of 64, 128 or 256 and that many
+ *     rows) and a row stride under 2^25 elements; other tasks are masked, 64
+ *     rows of T, any type.  "p norm" tasks are the c0 = 0 tasks of LARS
+ *     params.  All run on the bf16 matrix cores with fp32 products (three-way
+ *     bf16 splits). */
 int scao_kron_project(const scao_task* tasks, int ntasks, const scao_leaf_desc* leaves,
                       const scao_param_desc* params, double* slots, int variant, void* stream);
-/* A2  P = T U_r, Delta = (s_l s_r^T - 1) P and nu^2 partial per 64x64 tile of P. */
+/* A2  P = T U_r, Delta = (s_l s_r^T - 1) P and nu^2 partial per 64x64 tile of P.
+ *     A leaf with column chunks takes two launches: first, with slots NULL
+ *     (params is not read), a task per chunk and 64x64 tile, (leaf, a, b +
+ *     (chunk << 16)), each forming its share of the tile of P; then its tiles. */
 int scao_kron_delta(const scao_task* tasks, int ntasks, const scao_leaf_desc* leaves,
                     const scao_param_desc* params, double* slots, void* stream);
 /* A3  W = U_l Delta per 64-row strip. */

@@ -21,7 +21,7 @@ import torch  # noqa: F401  -- loads torch's HIP runtime before ours
 HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.environ.get("SCAO_AMD_LIB", os.path.join(HERE, "_lib", "libscao_amd.so"))
 
-ABI_VERSION = 12
+ABI_VERSION = 13
 SLOT_WIDTH = 3
 FLAT_CHUNK = 4096
 PROJ_COLS = 256
@@ -30,6 +30,7 @@ APPLY_WIDE_ROWS = 16
 APPLY_WIDE_COLS = 256
 APPLY_GROUP = 8
 GRAM_TILE = 128
+LF_NSPLIT_SHIFT, LF_DCHUNK_SHIFT = 8, 16
 NOALLOC_SCRATCH_BYTES = 16 << 20
 EIG_BAND = 16
 EIG_BANDW = 2 * EIG_BAND + 1

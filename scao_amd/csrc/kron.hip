@@ -19,6 +19,7 @@
 //   * reduction index: K-step s of a 16-wide chunk uses index
 //     kb + 4*(l/16) + s, so one float4 per lane feeds four K-steps.
 // Both only reorder an exact sum, so they change rounding order, never terms.
+#include <algorithm>
 #include <mutex>
 
 #include "scao_common.hpp"
@@ -28,209 +29,107 @@ using namespace scao;
 namespace {
 
 // ----------------------------------------------------------- project ---
-// T[c0:c0+CR, j0:j0+256] = U_l^T G over all m rows.  Wave w owns 64 columns.
-// Rows are consumed in chunks of PR=32: each chunk of G (32 x 256) and U_l
-// (32 x CR) is loaded into registers one chunk ahead (coalesced float4: one
-// wave reads one 1 KB row of G), written to LDS, and all four waves run
-// 2*CR MFMAs on it.  CR = 64, or 128 for whole tiles of k % 128 == 0 blocks
-// (every G chunk staged then feeds twice the MFMAs, and each strip of G is
-// read by half as many blocks).  Chunk-0 tasks also reduce ||g||^2 and
-// ||p*decay||^2 from the staged registers (every element of the strip passes
-// through exactly one thread).
-constexpr int PR = 32;           // rows per chunk
-// Whole fp32 tiles (the FAST variants) run on the bf16 matrix cores
-// (project_tile_x6) with 256 threads for 64 rows of T and 512 for 128 or 256.
-constexpr int X6_NT128 = 512;
-constexpr int GP = SCAO_PROJ_COLS + 4;  // LDS pitch of the G chunk
-
-template <bool FAST, bool DO_P, int CR = 64>
-__device__ __forceinline__ void project_tile(const scao_leaf_desc& L, const scao_param_desc& P,
-                                             int j0, int c0, int slot, double* slots) {
-  static_assert(CR == 64 || (CR == 128 && FAST), "CR");
-  constexpr int UP = CR + 4;       // LDS pitch of the U_l chunk
-  constexpr int NQ = CR / 16;      // MFMA tiles down T
-  constexpr int NU = CR / 32;      // float4 of U_l per thread and chunk
-  __shared__ __attribute__((aligned(16))) float Gs[PR][GP];
-  __shared__ __attribute__((aligned(16))) float Us[PR][UP];
-  __shared__ double red[16];
-  const int tid = threadIdx.x;
-  const int w = tid / 64, l = tid % 64;
-  const int m = L.m, n = L.n, k = L.k;
-  const int64_t ld = L.ld;
-  const int dt = FAST ? SCAO_F32 : P.dtype;
-  const int kk = l / 16;
-  const bool do_norms = (c0 == 0) && slot >= 0;
-  constexpr bool do_p = DO_P;
-  const bool decay = P.flags & SCAO_PF_DECAY;
-  const bool gvec_leaf = FAST || (L.flags & SCAO_LF_VEC4) != 0;
-  const bool kvec = FAST || (k % 4) == 0;
-
-  // loader geometry (fixed per thread): G row gr_h = idx/64, 4 columns at gc
-  const int gc = (tid % 64) * 4;         // column offset inside the strip
-  int gmask = 15;
-  if (!FAST)
-    for (int t = 0; t < 4; ++t) gmask = (j0 + gc + t < n) ? gmask : (gmask & ~(1 << t));
-  const bool gvec = gvec_leaf && gmask == 15;
-  const int uc = (tid % (CR / 4)) * 4;   // c offset inside the CR-wide chunk
-  int umask = 15;
-  if (!FAST)
-    for (int t = 0; t < 4; ++t) umask = (c0 + uc + t < k) ? umask : (umask & ~(1 << t));
-  const bool uvec = kvec && umask == 15;
-
-  v4f acc[NQ][4];
-#pragma unroll
-  for (int q = 0; q < NQ; ++q)
-#pragma unroll
-    for (int t = 0; t < 4; ++t) acc[q][t] = v4f{0.f, 0.f, 0.f, 0.f};
-  double g2 = 0.0, p2 = 0.0;
-
-  v4f rg[8], ru[NU], rp[8];
-  auto load_chunk = [&](int i0) {
-#pragma unroll
-    for (int h = 0; h < 8; ++h) {
-      const int i = i0 + tid / 64 + 4 * h;     // rows i0 + (0..31)
-      const int64_t e = L.off + (int64_t)i * ld + j0 + gc;
-      if (FAST) {
-        rg[h] = gld4_nt((const float*)P.graw + e);
-        if (do_p) rp[h] = gld4_nt((const float*)P.p + e);
-      } else {
-        const bool ok = i < m && gmask;
-        rg[h] = ok ? ld4(P.graw, dt, e, gvec, gmask) : v4f{0.f, 0.f, 0.f, 0.f};
-        if (do_p) rp[h] = ok ? ld4(P.p, dt, e, gvec, gmask) : v4f{0.f, 0.f, 0.f, 0.f};
-      }
-    }
-#pragma unroll
-    for (int h = 0; h < NU; ++h) {
-      const int i = i0 + tid / (CR / 4) + (1024 / CR) * h;
-      if (FAST)
-        ru[h] = gld4(L.Ul + (int64_t)i * k + c0 + uc);
-      else
-        ru[h] = (i < m && umask) ? ldf4(L.Ul, (int64_t)i * k + c0 + uc, uvec, umask)
-                                 : v4f{0.f, 0.f, 0.f, 0.f};
-    }
-  };
-  auto store_chunk = [&]() {
-#pragma unroll
-    for (int h = 0; h < 8; ++h) *(v4f*)&Gs[tid / 64 + 4 * h][gc] = rg[h];
-#pragma unroll
-    for (int h = 0; h < NU; ++h) *(v4f*)&Us[tid / (CR / 4) + (1024 / CR) * h][uc] = ru[h];
-    if (do_norms) {
-      float a = 0.f, b = 0.f;
-#pragma unroll
-      for (int h = 0; h < 8; ++h)
-#pragma unroll
-        for (int t = 0; t < 4; ++t) {
-          a = fmaf(rg[h][t], rg[h][t], a);
-          if (do_p) {
-            const float x = decay ? round_to(dt, rp[h][t] * P.decay) : rp[h][t];
-            b = fmaf(x, x, b);
-          }
-        }
-      g2 += (double)a;
-      p2 += (double)b;
-    }
-  };
-
-  load_chunk(0);
-  for (int i0 = 0; i0 < m; i0 += PR) {
-    if (i0) __syncthreads();              // previous chunk fully consumed
-    store_chunk();
-    __syncthreads();
-    if (i0 + PR < m) load_chunk(i0 + PR); // in flight during the MFMAs below
-    // operands of step s + 1 are read from LDS while step s's MFMAs run
-    v4f b[2];
-    float a[2][NQ];
-    b[0] = *(const v4f*)&Gs[kk][64 * w + 4 * (l % 16)];
-#pragma unroll
-    for (int q = 0; q < NQ; ++q) a[0][q] = Us[kk][16 * q + (l % 16)];
-#pragma unroll
-    for (int s = 0; s < PR / 4; ++s) {
-      const int cur = s & 1;
-      if (s + 1 < PR / 4) {
-        b[cur ^ 1] = *(const v4f*)&Gs[4 * (s + 1) + kk][64 * w + 4 * (l % 16)];
-#pragma unroll
-        for (int q = 0; q < NQ; ++q) a[cur ^ 1][q] = Us[4 * (s + 1) + kk][16 * q + (l % 16)];
-      }
-#pragma unroll
-      for (int q = 0; q < NQ; ++q)
-#pragma unroll
-        for (int t = 0; t < 4; ++t) acc[q][t] = mfma16(a[cur][q], b[cur][t], acc[q][t]);
-    }
-    if (FAST && CR == 64) {
-      // the schedule: step 0's reads, then per step the next step's reads
-      // ahead of its 16 MFMAs (a G float4 and four U_l values: three LDS
-      // instructions).  Measured faster at CR = 64 only: the 128-wide tile
-      // runs slower with it.
-      __builtin_amdgcn_sched_group_barrier(0x100, 3, 0);
-#pragma unroll
-      for (int s = 0; s < PR / 4; ++s) {
-        if (s + 1 < PR / 4) __builtin_amdgcn_sched_group_barrier(0x100, 3, 0);
-        __builtin_amdgcn_sched_group_barrier(0x008, 16, 0);
-      }
-    }
-  }
-  // T[c][j] for c = c0 + 16q + 4*(l/16) + r, j = jl + t
-  const int jl = j0 + 64 * w + 4 * (l % 16);
-  int cmask = 15;
-  if (!FAST)
-    for (int t = 0; t < 4; ++t) cmask = (jl + t < n) ? cmask : (cmask & ~(1 << t));
-  const bool tvec = gvec_leaf && cmask == 15;
-#pragma unroll
-  for (int q = 0; q < NQ; ++q)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int c = c0 + 16 * q + 4 * kk + r;
-      if (FAST || (c < k && cmask)) {
-        v4f o = {acc[q][0][r], acc[q][1][r], acc[q][2][r], acc[q][3][r]};
-        stf4(L.T, (int64_t)c * n + jl, o, tvec, cmask);
-      }
-    }
-  if (do_norms) {
-    double x[2] = {g2, p2};
-    block_sum<2>(x, red);
-    if (threadIdx.x == 0) {
-      slots[(int64_t)slot * SCAO_SLOT_WIDTH + 0] = x[0];
-      slots[(int64_t)slot * SCAO_SLOT_WIDTH + 1] = x[1];
-      slots[(int64_t)slot * SCAO_SLOT_WIDTH + 2] = 0.0;
-    }
-  }
-}
-
-// The same tile for whole fp32 tiles (FAST) on the bf16 matrix cores, with
-// fp32 products through three-way splits (mfma_x6): one v_mfma_f32_16x16x32
-// covers a whole 32-row chunk, so a chunk costs 6 * 16 cycles per output
-// tile against 8 * 32 for the fp32 16x16x4 form.  NT threads (NT / 64
-// waves) share the CR x 256 tile; wave w owns CW = 256 / (NT / 64) columns
-// (NJ = CW / 16 output tiles across) and all CR rows of T.
+// T[c0:c0+CR, j0:j0+256] = U_l^T G over rows [i_beg, i_end), on the bf16
+// matrix cores with fp32 products through three-way splits (mfma_x6).  Rows
+// are consumed in chunks of PR = 32, one v_mfma_f32_16x16x32 deep.  NT
+// threads (NT / 64 waves) share the CR x 256 tile; wave w owns
+// CW = 256 / (NT / 64) columns (NJ = CW / 16 output tiles across) and all CR
+// rows of T.
 //   * G does not pass through LDS: lane (jj, g) of wave w loads rows
 //     8g..8g+7 of the chunk at the NJ columns j0 + CW*w + NJ*jj + t, which is
 //     exactly its B operand of the NJ output tiles t (the column permutation
-//     of the fp32 form), and splits it in registers.
+//     of the fp32 form), and splits it in registers.  bf16 gradients are
+//     their own split (the two remainders are zero), so their products take
+//     three MFMAs instead of six and no split.
 //   * U_l (shared by the waves) is split by its loader and stored as three
 //     bf16 planes, column-major inside the chunk (column pitch 80 B: the 16
 //     lanes of one A-operand read hit 16 disjoint bank quads).
 // The next chunk's G, p and U_l are loaded while the current one's MFMAs run.
-template <bool DO_P, int CR, int NT>
-__device__ __forceinline__ void project_tile_x6(const scao_leaf_desc& L, const scao_param_desc& P,
-                                                int j0, int c0, int slot, double* slots) {
+// Chunk-0 tasks also reduce ||g||^2 and ||p*decay||^2 of their rows and strip
+// from the loaded registers (every element passes through exactly one lane).
+//
+// EDGE: the strip may end past column n and the rows past i_end (those count
+// as zero); every load is masked and G may have any of the three types (dt).
+// KEDGE: c0 + CR may lie past k, so U_l's loads and T's stores are masked.
+// Loads need element alignment only, in every form.
+//
+// When the whole tiles of a step are too few to fill 256 CUs the rows are
+// split (SCAO_LF_NSPLIT_SHIFT): each part writes a plane of its own and the
+// delta stage adds the planes in order.
+//
+// HBM bounds the projection of a step that fills the chip (5.4 TB/s at 323 M
+// parameters, k = 64), latency a smaller one.  Against fp32 MFMAs over tiles
+// staged through LDS with masked scalar loads, for all but aligned whole fp32
+// tiles: one Llama-1B layer in bf16 866 -> 75 us, odd sizes (7 M elements) 596
+// -> 66 us; row parts: one GPT-2-small layer 80 -> 19 us.
+constexpr int PR = 32;           // rows per chunk
+// a lane's rows are addressed by 32-bit byte offsets: 24 row strides and a
+// strip stay below 2^32 for strides under 2^25 elements
+constexpr int64_t SHORT_ROWS = 1 << 25;
+
+// rows of one part of a block's row split, and the part's plane of T: plane
+// 0 (T itself) when the rows are whole, else plane 1 + part
+__host__ __device__ inline int split_rows(int m, int parts) {
+  return ((m + PR * parts - 1) / (PR * parts)) * PR;
+}
+__host__ __device__ inline int64_t plane_floats(int64_t n) { return (n + 3) & ~(int64_t)3; }
+
+// The values one lane holds of a chunk of G or p: eight rows of NJ columns,
+// as loaded (DT = SCAO_F32: floats, also in EDGE tiles of any type;
+// SCAO_BF16 / SCAO_F16: packed 16-bit pairs).
+template <int DT, int NJ> struct lane_rows {
+  static constexpr int W = DT == SCAO_F32 ? NJ : NJ / 2;   // 32-bit words per row
+  typedef uint32_t vw __attribute__((ext_vector_type(W)));
+  typedef vw vwu __attribute__((aligned(DT == SCAO_F32 ? 4 : 2)));
+  typedef __attribute__((address_space(1))) vwu gvw;
+  vw x[8];
+  __device__ __forceinline__ void load(int e, const char* at) {
+    x[e] = __builtin_nontemporal_load((const gvw*)at);
+  }
+  __device__ __forceinline__ float get(int e, int t) const {
+    if constexpr (DT == SCAO_F32) return __uint_as_float(x[e][t]);
+    const uint32_t u = x[e][t / 2];
+    if constexpr (DT == SCAO_BF16) return __uint_as_float(t & 1 ? u & 0xffff0000u : u << 16);
+    return f16_to_f((uint16_t)(t & 1 ? u >> 16 : u));
+  }
+  // column t's bf16 values of all eight rows, as the MFMA takes them
+  __device__ __forceinline__ v8bf column(int t) const {
+    v4u_t r;
+#pragma unroll
+    for (int p = 0; p < 4; ++p)
+      r[p] = __builtin_amdgcn_perm(x[2 * p + 1][t / 2], x[2 * p][t / 2],
+                                   t & 1 ? 0x07060302u : 0x05040100u);
+    return __builtin_bit_cast(v8bf, r);
+  }
+};
+
+constexpr int UCP = 40;   // bf16 per U_l column in LDS (32 rows + pad)
+template <int CR> struct project_lds {
+  __bf16 U[2][3][CR][UCP];   // by chunk parity
+  double red[16];
+};
+
+template <bool DO_P, int CR, int NT, int DT, bool EDGE, bool KEDGE = EDGE>
+__device__ __forceinline__ void project_tile(project_lds<CR>& lds, const scao_leaf_desc& L, const scao_param_desc& P,
+                                             int j0, int c0, int i_beg, int i_end, float* T,
+                                             int slot, double* slots) {
   static_assert(CR == 64 || CR == 128 || CR == 256, "CR");
   static_assert(NT == 256 || NT == 512, "NT");
+  static_assert(!EDGE || (DT == SCAO_F32 && (KEDGE || CR == 64)), "EDGE tiles convert on load");
   constexpr int NQ = CR / 16;        // MFMA tiles down T
   constexpr int CW = 256 / (NT / 64);
   constexpr int NJ = CW / 16;        // MFMA tiles across, G columns per lane
-  constexpr int UCP = 40;            // bf16 per U_l column in LDS (32 rows + pad)
   constexpr int UG = NT / 8;         // U_l loader threads per 4-row group
   constexpr int UW = CR / UG;        // U_l columns per loader thread
+  constexpr int ES = DT == SCAO_F32 ? 4 : 2;   // bytes per element (EDGE: not used)
   static_assert(UW == 2 || UW == 4, "U_l loader width");
-  typedef float vj __attribute__((ext_vector_type(NJ)));
-  typedef __attribute__((address_space(1))) vj gvj;
-  __shared__ __attribute__((aligned(16))) __bf16 Us[2][3][CR][UCP];   // by chunk parity
-  __shared__ double red[2 * NT / 64];
+  __bf16 (*Us)[3][CR][UCP] = lds.U;
   const int tid = threadIdx.x;
   const int w = tid / 64, l = tid % 64;
   const int jj = l % 16, g = l / 16;
-  const int m = L.m, n = L.n, k = L.k;
+  const int n = L.n, k = L.k;
   const int64_t ld = L.ld;
+  const int dt = EDGE ? P.dtype : DT;
   const bool do_norms = (c0 == 0) && slot >= 0;
   // x * 1.0f == x bit for bit, so no per-element select on the decay flag
   const float dec = (P.flags & SCAO_PF_DECAY) ? P.decay : 1.0f;
@@ -241,9 +140,9 @@ __device__ __forceinline__ void project_tile_x6(const scao_leaf_desc& L, const s
   // registers) plus a 32-bit lane offset fixed for the whole tile: lane
   // (jj, g) reads rows 8g.. of the chunk at column gcol, the U_l loader rows
   // 4ua.. at column c0 + ub*UW.
-  const uint32_t g_lane = (uint32_t)((8 * g * ld + (gcol - j0)) * (int64_t)sizeof(float));
+  const uint32_t g_lane = (uint32_t)((8 * g * ld + (gcol - j0)) * (int64_t)ES);
   const uint32_t u_lane = (uint32_t)((4 * ua * (int64_t)k + ub * UW) * (int64_t)sizeof(float));
-  const int64_t ldb = ld * (int64_t)sizeof(float), kb = k * (int64_t)sizeof(float);
+  const int64_t ldb = ld * (int64_t)ES, kb = k * (int64_t)sizeof(float);
 
   v4f acc[NQ][NJ];
 #pragma unroll
@@ -252,31 +151,88 @@ __device__ __forceinline__ void project_tile_x6(const scao_leaf_desc& L, const s
     for (int t = 0; t < NJ; ++t) acc[q][t] = v4f{0.f, 0.f, 0.f, 0.f};
   double g2 = 0.0, p2 = 0.0;
 
-  vj rg[8], rp[8];
+  lane_rows<DT, NJ> rg, rp;
   float ru[4][UW];
-  auto load_g = [&](int i0) {
-    const int64_t o = L.off + (int64_t)i0 * ld + j0;
-    const char* gb = (const char*)((const float*)P.graw + o);
-    const char* pb = (const char*)((const float*)P.p + o);
+  // Masked rows: every address is clamped into the tile and what lies outside
+  // becomes zero afterwards, so the loads of a chunk go out together.
+  auto load_edge = [&](lane_rows<DT, NJ>& r, const void* base, int i0) {
+    if constexpr (EDGE) {
+      const int64_t first = L.off + gcol;
+      auto row = [&](int e) { return (int64_t)min(i0 + 8 * g + e, i_end - 1) * ld; };
+      if (gcol + NJ <= n && dt == SCAO_F32) {
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      rg[e] = __builtin_nontemporal_load((const gvj*)(gb + e * ldb + g_lane));
-      if (DO_P) rp[e] = __builtin_nontemporal_load((const gvj*)(pb + e * ldb + g_lane));
+        for (int e = 0; e < 8; ++e) r.load(e, (const char*)((const float*)base + first + row(e)));
+      } else if (gcol + NJ <= n) {
+        v2u h[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) h[e] = gld2w((const uint16_t*)base + first + row(e));
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+#pragma unroll
+          for (int t = 0; t < NJ; ++t) {
+            const uint16_t x = (uint16_t)(t & 1 ? h[e][t / 2] >> 16 : h[e][t / 2]);
+            r.x[e][t] = __float_as_uint(dt == SCAO_BF16 ? bf16_to_f(x) : f16_to_f(x));
+          }
+      } else {
+        int64_t col[NJ];
+#pragma unroll
+        for (int t = 0; t < NJ; ++t) col[t] = L.off + min(gcol + t, n - 1);
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+#pragma unroll
+          for (int t = 0; t < NJ; ++t)
+            r.x[e][t] = __float_as_uint(ld1(base, dt, col[t] + row(e)));
+      }
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+#pragma unroll
+        for (int t = 0; t < NJ; ++t)
+          if (i0 + 8 * g + e >= i_end || gcol + t >= n) r.x[e][t] = 0u;
+    }
+  };
+  auto load_g = [&](int i0) {
+    if constexpr (EDGE) {
+      load_edge(rg, P.graw, i0);
+      if (DO_P) load_edge(rp, P.p, i0);
+    } else {
+      const int64_t o = (L.off + (int64_t)i0 * ld + j0) * ES;
+      const char* gb = (const char*)P.graw + o;
+      const char* pb = (const char*)P.p + o;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        rg.load(e, gb + e * ldb + g_lane);
+        if (DO_P) rp.load(e, pb + e * ldb + g_lane);
+      }
     }
   };
   auto load_u = [&](int i0) {
-    const char* ubase = (const char*)(L.Ul + (int64_t)i0 * k + c0);
+    if constexpr (EDGE || KEDGE) {
+      const int col = c0 + ub * UW;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const float* src = (const float*)(ubase + r * kb + u_lane);
-      if constexpr (UW == 4) {
-        const v4f x = gld4(src);
+      for (int r = 0; r < 4; ++r) {
+        const float* src = L.Ul + (int64_t)min(i0 + 4 * ua + r, i_end - 1) * k;
 #pragma unroll
-        for (int c = 0; c < 4; ++c) ru[r][c] = x[c];
-      } else {
-        const v2u x = *(const gv2u*)src;
-        ru[r][0] = __uint_as_float(x[0]);
-        ru[r][1] = __uint_as_float(x[1]);
+        for (int c = 0; c < UW; ++c) ru[r][c] = gld1(src + (KEDGE ? min(col + c, k - 1) : col + c));
+      }
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int c = 0; c < UW; ++c)
+          if (i0 + 4 * ua + r >= i_end || (KEDGE && col + c >= k)) ru[r][c] = 0.f;
+    } else {
+      const char* ubase = (const char*)(L.Ul + (int64_t)i0 * k + c0);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const float* src = (const float*)(ubase + r * kb + u_lane);
+        if constexpr (UW == 4) {
+          const v4f x = gld4(src);
+#pragma unroll
+          for (int c = 0; c < 4; ++c) ru[r][c] = x[c];
+        } else {
+          const v2u x = gld2w(src);
+          ru[r][0] = __uint_as_float(x[0]);
+          ru[r][1] = __uint_as_float(x[1]);
+        }
       }
     }
   };
@@ -303,27 +259,32 @@ __device__ __forceinline__ void project_tile_x6(const scao_leaf_desc& L, const s
     }
   };
   // CR = 256: the prefetches are unconditional, clamped to the last chunk
-  // (m % PR == 0 for these tiles), and pinned ahead of the MFMAs: behind a
-  // branch, the join makes the compiler wait for every load in flight, the
-  // next chunk's G included, and the scheduler sinks them among the MFMAs.
-  // The narrower tiles have half or a quarter of the MFMAs per chunk to hide
-  // loads behind and measured faster with the branch (the last chunk loads
-  // nothing).
-  const int last = m - PR;
-  load_g(0);
-  load_u(0);
+  // ((i_end - i_beg) % PR == 0 for these tiles), and pinned ahead of the
+  // MFMAs: behind a branch, the join makes the compiler wait for every load in
+  // flight, the next chunk's G included, and the scheduler sinks them among
+  // the MFMAs.  The narrower tiles have half or a quarter of the MFMAs per
+  // chunk to hide loads behind and measured faster with the branch (the last
+  // chunk loads nothing).
+  constexpr bool PIN = CR == 256 && !EDGE && !KEDGE;
+  const int last = i_end - PR;
+  load_g(i_beg);
+  load_u(i_beg);
   write_u(0);
-  if (CR == 256 || PR < m) load_u(PR < last ? PR : last);
+  if (PIN || i_beg + PR < i_end) load_u(PIN && i_beg + PR > last ? last : i_beg + PR);
   __syncthreads();
-  for (int i0 = 0, cur = 0; i0 < m; i0 += PR, cur ^= 1) {
+  for (int i0 = i_beg, cur = 0; i0 < i_end; i0 += PR, cur ^= 1) {
     // this chunk's G operands, split in registers
     bf3 bg[NJ];
 #pragma unroll
     for (int t = 0; t < NJ; ++t) {
-      float x[8];
+      if constexpr (DT == SCAO_BF16) {
+        bg[t].h = rg.column(t);
+      } else {
+        float x[8];
 #pragma unroll
-      for (int e = 0; e < 8; ++e) x[e] = rg[e][t];
-      bg[t] = split_bf3(x);
+        for (int e = 0; e < 8; ++e) x[e] = rg.get(e, t);
+        bg[t] = split_bf3(x);
+      }
     }
     if (do_norms) {
       float a = 0.f, b = 0.f;
@@ -331,16 +292,18 @@ __device__ __forceinline__ void project_tile_x6(const scao_leaf_desc& L, const s
       for (int e = 0; e < 8; ++e)
 #pragma unroll
         for (int t = 0; t < NJ; ++t) {
-          a = fmaf(rg[e][t], rg[e][t], a);
+          const float y = rg.get(e, t);
+          a = fmaf(y, y, a);
           if (DO_P) {
-            const float x = rp[e][t] * dec;
+            float x = rp.get(e, t) * dec;
+            if (EDGE || DT != SCAO_F32) x = round_to(dt, x);
             b = fmaf(x, x, b);
           }
         }
       g2 += (double)a;
       p2 += (double)b;
     }
-    if constexpr (CR == 256) {
+    if constexpr (PIN) {
       write_u(cur ^ 1);                   // chunk i+1's planes, read after the barrier below
       // the loads go out after the split (measured faster than letting the
       // scheduler hoist them above it)
@@ -348,10 +311,10 @@ __device__ __forceinline__ void project_tile_x6(const scao_leaf_desc& L, const s
       load_g(i0 + PR < last ? i0 + PR : last);   // in flight during the MFMAs below
       load_u(i0 + 2 * PR < last ? i0 + 2 * PR : last);
       __builtin_amdgcn_sched_barrier(0);
-    } else if (i0 + PR < m) {
+    } else if (i0 + PR < i_end) {
       write_u(cur ^ 1);
       load_g(i0 + PR);
-      if (i0 + 2 * PR < m) load_u(i0 + 2 * PR);
+      if (i0 + 2 * PR < i_end) load_u(i0 + 2 * PR);
     }
 #pragma unroll
     for (int q = 0; q < NQ; ++q) {
@@ -360,7 +323,9 @@ __device__ __forceinline__ void project_tile_x6(const scao_leaf_desc& L, const s
       au.m = *(const v8bf*)&Us[cur][1][16 * q + jj][8 * g];
       au.l = *(const v8bf*)&Us[cur][2][16 * q + jj][8 * g];
 #pragma unroll
-      for (int t = 0; t < NJ; ++t) acc[q][t] = mfma_x6(au, bg[t], acc[q][t]);
+      for (int t = 0; t < NJ; ++t)
+        acc[q][t] = DT == SCAO_BF16 ? mfma_x3(au, bg[t].h, acc[q][t])
+                                    : mfma_x6(au, bg[t], acc[q][t]);
     }
     __syncthreads();
   }
@@ -370,20 +335,42 @@ __device__ __forceinline__ void project_tile_x6(const scao_leaf_desc& L, const s
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int c = c0 + 16 * q + 4 * g + r;
-      vj o;
+      if constexpr (EDGE || KEDGE) {
+        if (c >= k) continue;
 #pragma unroll
-      for (int t = 0; t < NJ; ++t) o[t] = acc[q][t][r];
-      *(gvj*)(L.T + (int64_t)c * n + gcol) = o;
+        for (int t = 0; t < NJ; ++t)
+          if (gcol + t < n) gst1(T + (int64_t)c * n + gcol + t, acc[q][t][r]);
+      } else {
+        typedef float vj __attribute__((ext_vector_type(NJ)));
+        typedef vj vju __attribute__((aligned(4)));
+        vj o;
+#pragma unroll
+        for (int t = 0; t < NJ; ++t) o[t] = acc[q][t][r];
+        *(__attribute__((address_space(1))) vju*)(T + (int64_t)c * n + gcol) = o;
+      }
     }
   if (do_norms) {
     double x[2] = {g2, p2};
-    block_sum_n<2, NT>(x, red);
+    block_sum_n<2, NT>(x, lds.red);
     if (threadIdx.x == 0) {
       slots[(int64_t)slot * SCAO_SLOT_WIDTH + 0] = x[0];
       slots[(int64_t)slot * SCAO_SLOT_WIDTH + 1] = x[1];
       slots[(int64_t)slot * SCAO_SLOT_WIDTH + 2] = 0.0;
     }
   }
+}
+
+// A task's part of the row split (a step's ranks are whole multiples of 64, so
+// T's rows are): tk.b holds the column origin c0 in its low
+// 16 bits and the part above them.
+template <bool DO_P, int CR, int NT, int DT, bool EDGE>
+__device__ __forceinline__ void project_part(project_lds<CR>& lds, const scao_leaf_desc& L, const scao_param_desc& P,
+                                             int j0, int b, int slot, double* slots) {
+  const int parts = SCAO_LF_GET_NSPLIT(L.flags), part = b >> 16;
+  const int rows = split_rows(L.m, parts);
+  const int i_beg = part * rows, i_end = min(L.m, i_beg + rows);
+  float* T = L.T + (parts > 1 ? (1 + part) * plane_floats((int64_t)L.k * L.n) : 0);
+  project_tile<DO_P, CR, NT, DT, EDGE, false>(lds, L, P, j0, b & 0xffff, i_beg, i_end, T, slot, slots);
 }
 
 // ------------------------------------------------------------- delta ---
@@ -468,8 +455,7 @@ __device__ __forceinline__ void delta_tile(const scao_leaf_desc& L, float eps, i
   int dmask = 15;
   if (!FAST)
     for (int t = 0; t < 4; ++t) dmask = (dl + t < k) ? dmask : (dmask & ~(1 << t));
-  const bool uvec = FAST || ((k % 4) == 0 && dmask == 15);
-  const bool tvec_leaf = FAST || (L.flags & SCAO_LF_VEC4) != 0;
+  const bool uvec = FAST || dmask == 15;
   const int nq = ((n + 63) / 64) * 16;    // per-wave share of n, multiple of 16
   const int jbeg = w * nq, jend = min(n, jbeg + nq);
 
@@ -495,7 +481,7 @@ __device__ __forceinline__ void delta_tile(const scao_leaf_desc& L, float eps, i
         if (FAST)
           a[q] = gld4(T + (int64_t)c * n + j);
         else
-          a[q] = (c < k && jm) ? ldf4(T, (int64_t)c * n + j, tvec_leaf && jm == 15, jm)
+          a[q] = (c < k && jm) ? ldf4(T, (int64_t)c * n + j, jm == 15, jm)
                                : v4f{0.f, 0.f, 0.f, 0.f};
       }
 #pragma unroll
@@ -576,6 +562,170 @@ __device__ __forceinline__ void delta_tile(const scao_leaf_desc& L, float eps, i
     double xs[1] = {nu2};
     block_sum<1>(xs, red);
     if (threadIdx.x == 0) {
+      slots[(int64_t)slot * SCAO_SLOT_WIDTH + 0] = 0.0;
+      slots[(int64_t)slot * SCAO_SLOT_WIDTH + 1] = 0.0;
+      slots[(int64_t)slot * SCAO_SLOT_WIDTH + 2] = xs[0];
+    }
+  }
+}
+
+// One column chunk's share of a 64x64 tile of P = T U_r: with one 64-wide tile
+// per block at k <= 64, a tile per workgroup leaves most CUs idle and walks
+// all n columns in one chain, so few-block steps split n into chunks of k
+// rounded up to 64 columns (the chunks' shares of P then take as much memory
+// as T), one workgroup each.  64 columns of T at a time are staged through LDS
+// as floats: there the planes of a row-split projection are added in order
+// (b0 = 0 tasks also write the sum to T itself).  Wave w takes rows 16w .. +15
+// of the tile on six bf16 products per fp32 product and writes them to the
+// chunk's plane; delta_finish adds the chunks.  tplanes and pplanes: the row
+// parts' planes of T and the chunks' planes of P.
+// 10 blocks of GPT-2 small (k = 64): 36 -> 20 us with delta_finish; one 2048 x
+// 2048 block over 16 row parts: 69 -> 24 us.
+constexpr int TSP = 64 + 4;   // LDS pitch of the staged columns of T
+
+__host__ __device__ inline int delta_cols(int k) { return (k + 63) / 64 * 64; }
+
+__device__ __forceinline__ void delta_part(const scao_leaf_desc& L, int a0, int b0, int chunk,
+                                           const float* tplanes, float* pplanes,
+                                           float (*Ts)[TSP]) {
+  const int tid = threadIdx.x, w = tid / 64, l = tid % 64, i = l % 16, g = l / 16;
+  const int n = L.n, k = L.k;
+  const int parts = SCAO_LF_GET_NSPLIT(L.flags);
+  const int64_t tp = plane_floats((int64_t)k * n);
+  const int jbeg = chunk * delta_cols(k), jend = min(n, jbeg + delta_cols(k));
+  const int dl = b0 + 4 * i;
+  int dm = 0;
+#pragma unroll
+  for (int t = 0; t < 4; ++t) dm |= (dl + t < k) ? (1 << t) : 0;
+  v4f acc[4];
+#pragma unroll
+  for (int t = 0; t < 4; ++t) acc[t] = v4f{0.f, 0.f, 0.f, 0.f};
+  for (int jb = jbeg; jb < jend; jb += 64) {
+    // 64 columns of T, summed over the row parts: thread -> rows tid / 16 + 16q
+    const int col = jb + 4 * (tid % 16);
+    int cm = 0;
+#pragma unroll
+    for (int t = 0; t < 4; ++t) cm |= (col + t < n) ? (1 << t) : 0;
+    // (rows past k repeat row k - 1: they reach only rows of P past k, which
+    // are not stored; no branch between the loads, whose join would wait)
+    const float* first = parts > 1 ? tplanes : L.T;
+    int64_t at[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) at[q] = (int64_t)min(a0 + tid / 16 + 16 * q, k - 1) * n + col;
+    v4f x[4];
+    if (cm == 15) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) x[q] = gld4(first + at[q]);
+#pragma unroll 4
+      for (int s = 1; s < parts; ++s)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) x[q] += gld4(first + s * tp + at[q]);
+    } else {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) x[q] = ldf4(first, at[q], false, cm);
+      for (int s = 1; s < parts; ++s)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) x[q] += ldf4(first + s * tp, at[q], false, cm);
+    }
+    // rows of U_r past n repeat row n - 1 and meet zeros of T
+    v4f cb[2][8];
+    if (dm == 15) {
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+          cb[h][e] = gld4(L.Ur + (int64_t)min(jb + 32 * h + 8 * g + e, n - 1) * k + dl);
+    } else {
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+          cb[h][e] = ldf4(L.Ur, (int64_t)min(jb + 32 * h + 8 * g + e, n - 1) * k + dl, false, dm);
+    }
+    if (jb > jbeg) __syncthreads();   // the previous columns' reads
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int row = tid / 16 + 16 * q, c = a0 + row;
+      *(v4f*)&Ts[row][4 * (tid % 16)] = x[q];
+      if (parts > 1 && b0 == 0 && c < k && cm)
+        stf4(L.T, (int64_t)c * n + col, x[q], cm == 15, cm);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const v4f lo = *(const v4f*)&Ts[16 * w + i][32 * h + 8 * g];
+      const v4f hi = *(const v4f*)&Ts[16 * w + i][32 * h + 8 * g + 4];
+      const float xa[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+      const bf3 aw = split_bf3(xa);
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        float xb[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) xb[e] = cb[h][e][t];
+        acc[t] = mfma_x6(aw, split_bf3(xb), acc[t]);
+      }
+    }
+  }
+  // element (16w + 4g + r, 4i + t) of the tile
+  float* out = pplanes + chunk * plane_floats((int64_t)k * k);
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const int c = a0 + 16 * w + 4 * g + r;
+    if (c < k && dm)
+      stf4(out, (int64_t)c * k + dl, v4f{acc[0][r], acc[1][r], acc[2][r], acc[3][r]}, dm == 15,
+           dm);
+  }
+}
+
+// Delta and the natural-norm partial of 16 rows x 64 columns from the chunks'
+// shares: one float4 per thread and chunk, eight chunks' loads in flight.
+__device__ __forceinline__ void delta_finish(const scao_leaf_desc& L, float eps, int a0, int b0,
+                                             const float* pplanes, int slot, double* slots,
+                                             double* red) {
+  const int tid = threadIdx.x, k = L.k;
+  const int chunks = SCAO_LF_GET_DCHUNK(L.flags);
+  const int64_t pp = plane_floats((int64_t)k * k);
+  const bool sinv4 = L.flags & SCAO_LF_SINV4;
+  const int c = a0 + tid / 16, d = b0 + 4 * (tid % 16);
+  int dm = 0;
+#pragma unroll
+  for (int t = 0; t < 4; ++t) dm |= (c < k && d + t < k) ? (1 << t) : 0;
+  double nu2 = 0.0;
+  if (dm) {
+    const float* src = pplanes + (int64_t)c * k + d;
+    v4f p = {0.f, 0.f, 0.f, 0.f};
+    if (dm == 15) {
+      int s = 0;
+      for (; s + 8 <= chunks; s += 8) {
+        v4f x[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) x[u] = gld4(src + (s + u) * pp);
+#pragma unroll
+        for (int u = 0; u < 8; ++u) p += x[u];
+      }
+      for (; s < chunks; ++s) p += gld4(src + s * pp);
+    } else {
+      for (int s = 0; s < chunks; ++s) p += ldf4(src, s * pp, false, dm);
+    }
+    const float sl = gld1(L.Sl + c);
+    const float sl4 = sinv4 ? sl : inv4(sl);
+    const float il2 = sinv4 ? 0.f : inv2(sl, eps);
+    v4f o;
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      const float sr = d + t < k ? gld1(L.Sr + d + t) : 1.f;
+      o[t] = (sl4 * (sinv4 ? sr : inv4(sr)) - 1.0f) * p[t];
+      if (!sinv4 && d + t < k) {
+        const float y = (il2 * p[t]) * inv2(sr, eps);
+        nu2 += (double)y * (double)y;
+      }
+    }
+    stf4(L.Delta, (int64_t)c * k + d, o, dm == 15, dm);
+  }
+  if (slot >= 0) {
+    double xs[1] = {nu2};
+    block_sum<1>(xs, red);
+    if (tid == 0) {
       slots[(int64_t)slot * SCAO_SLOT_WIDTH + 0] = 0.0;
       slots[(int64_t)slot * SCAO_SLOT_WIDTH + 1] = 0.0;
       slots[(int64_t)slot * SCAO_SLOT_WIDTH + 2] = xs[0];
@@ -830,6 +980,26 @@ __device__ __forceinline__ void corr_tile(const scao_leaf_desc& L, int i0, int j
   const bool kvec = (k % 4) == 0;
 #pragma unroll
   for (int t = 0; t < 4; ++t) acc[t] = v4f{0.f, 0.f, 0.f, 0.f};
+  if (k % 16 == 0) {
+    // no branch between the loads: rows past the block repeat its last one
+    // (they reach only elements past it, which are not stored)
+    const float* wrow = L.W + (int64_t)min(irow, m - 1) * k + 4 * kk;
+    const float* urow[4];
+#pragma unroll
+    for (int t = 0; t < 4; ++t) urow[t] = L.Ur + (int64_t)min(jl + t, n - 1) * k + 4 * kk;
+#pragma unroll 4
+    for (int cb = 0; cb < k; cb += 16) {
+      const v4f a = gld4(wrow + cb);
+      v4f b[4];
+#pragma unroll
+      for (int t = 0; t < 4; ++t) b[t] = gld4(urow[t] + cb);
+#pragma unroll
+      for (int s = 0; s < 4; ++s)
+#pragma unroll
+        for (int t = 0; t < 4; ++t) acc[t] = mfma16(a[s], b[t][s], acc[t]);
+    }
+    return;
+  }
   for (int cb = 0; cb < k; cb += 16) {
     const int c = cb + 4 * kk;
     int cm = 0;
@@ -1821,23 +1991,15 @@ __device__ __forceinline__ void apply_out_tile(const scao_leaf_desc& L, const fl
 }
 
 // ---------------------------------------------------------- kernels ---
-template <bool FAST, bool DO_P, int CR = 64>
-__global__ __launch_bounds__(256) void k_project(const scao_task* __restrict__ tasks,
-                                                 const scao_leaf_desc* __restrict__ leaves,
-                                                 const scao_param_desc* __restrict__ params,
-                                                 double* slots) {
+template <bool DO_P, int CR, int NT, int DT, bool EDGE>
+__global__ __launch_bounds__(NT) void k_project(const scao_task* __restrict__ tasks,
+                                                const scao_leaf_desc* __restrict__ leaves,
+                                                const scao_param_desc* __restrict__ params,
+                                                double* slots) {
   const scao_task tk = tasks[blockIdx.x];
   const scao_leaf_desc L = leaves[tk.idx];
-  project_tile<FAST, DO_P, CR>(L, params[L.param], tk.a, tk.b, tk.slot, slots);
-}
-template <bool DO_P, int CR, int NT>
-__global__ __launch_bounds__(NT) void k_project_x6(const scao_task* __restrict__ tasks,
-                                                   const scao_leaf_desc* __restrict__ leaves,
-                                                   const scao_param_desc* __restrict__ params,
-                                                   double* slots) {
-  const scao_task tk = tasks[blockIdx.x];
-  const scao_leaf_desc L = leaves[tk.idx];
-  project_tile_x6<DO_P, CR, NT>(L, params[L.param], tk.a, tk.b, tk.slot, slots);
+  __shared__ __attribute__((aligned(16))) project_lds<CR> lds;
+  project_part<DO_P, CR, NT, DT, EDGE>(lds, L, params[L.param], tk.a, tk.b, tk.slot, slots);
 }
 // two waves per SIMD: the bf16-product tiles fit 256 registers without spilling
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_delta(
@@ -1851,14 +2013,26 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     diag_leaf_reduce(L, params[L.param], tk.a, tk.b, tk.slot, slots, red);
     return;
   }
-  const bool fast = (L.flags & SCAO_LF_VEC4) && (L.k % 4 == 0) && tk.a + 64 <= L.k &&
-                    tk.b + 64 <= L.k && (L.n % 64 == 0);
+  if (SCAO_LF_GET_DCHUNK(L.flags)) {
+    delta_finish(L, params[L.param].eps, tk.a, tk.b,
+                 L.Delta + plane_floats((int64_t)L.k * L.k), tk.slot, slots, red);
+    return;
+  }
+  const bool fast = tk.a + 64 <= L.k && tk.b + 64 <= L.k && (L.n % 64 == 0);
   if (fast && L.n % 128 == 0)
     delta_tile<true, true>(L, params[L.param].eps, tk.a, tk.b, tk.slot, slots, Ps, red);
   else if (fast)
     delta_tile<true>(L, params[L.param].eps, tk.a, tk.b, tk.slot, slots, Ps, red);
   else
     delta_tile<false>(L, params[L.param].eps, tk.a, tk.b, tk.slot, slots, Ps, red);
+}
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_delta_part(
+    const scao_task* __restrict__ tasks, const scao_leaf_desc* __restrict__ leaves) {
+  __shared__ __attribute__((aligned(16))) float Ts[64][TSP];
+  const scao_task tk = tasks[blockIdx.x];
+  const scao_leaf_desc L = leaves[tk.idx];
+  delta_part(L, tk.a, tk.b & 0xffff, tk.b >> 16, L.T + plane_floats((int64_t)L.k * L.n),
+             L.Delta + plane_floats((int64_t)L.k * L.k), Ts);
 }
 // two waves per SIMD: the bf16-product tiles fit 256 registers without spilling
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_lift(
@@ -1886,10 +2060,24 @@ __global__ __launch_bounds__(256) void k_apply(const scao_task* __restrict__ tas
 }
 
 // single-block reference operator (descriptors by value, tiles from blockIdx)
-__global__ __launch_bounds__(256) void k_project_one(scao_leaf_desc L, scao_param_desc P) {
-  const int strips = (L.n + SCAO_PROJ_COLS - 1) / SCAO_PROJ_COLS;
-  project_tile<false, false>(L, P, (blockIdx.x % strips) * SCAO_PROJ_COLS,
-                             (blockIdx.x / strips) * 64, -1, nullptr);
+template <int CR, int NT>
+__global__ __launch_bounds__(NT) void k_project_one(scao_leaf_desc L, scao_param_desc P,
+                                                    float* tplanes) {
+  __shared__ __attribute__((aligned(16))) project_lds<CR> lds;
+  const int strips = (L.n + SCAO_PROJ_COLS - 1) / SCAO_PROJ_COLS, kt = (L.k + CR - 1) / CR;
+  const int j0 = (int)(blockIdx.x % strips) * SCAO_PROJ_COLS;
+  const int c0 = (int)(blockIdx.x / strips % kt) * CR, part = (int)(blockIdx.x / (strips * kt));
+  const int parts = SCAO_LF_GET_NSPLIT(L.flags), rows = split_rows(L.m, parts);
+  const int i_beg = part * rows, i_end = min(L.m, i_beg + rows);
+  float* T = parts > 1 ? tplanes + part * plane_floats((int64_t)L.k * L.n) : L.T;
+  const bool whole = j0 + SCAO_PROJ_COLS <= L.n && (i_end - i_beg) % PR == 0 &&
+                     L.ld < SHORT_ROWS;
+  if (whole && c0 + CR <= L.k)
+    project_tile<false, CR, NT, SCAO_F32, false>(lds, L, P, j0, c0, i_beg, i_end, T, -1, nullptr);
+  else if (whole)
+    project_tile<false, CR, NT, SCAO_F32, false, true>(lds, L, P, j0, c0, i_beg, i_end, T, -1, nullptr);
+  else
+    project_tile<false, CR, NT, SCAO_F32, true>(lds, L, P, j0, c0, i_beg, i_end, T, -1, nullptr);
 }
 __global__ __launch_bounds__(256) void k_delta_one(scao_leaf_desc L) {
   __shared__ __attribute__((aligned(16))) float Ps[3][64][DP];
@@ -1897,6 +2085,19 @@ __global__ __launch_bounds__(256) void k_delta_one(scao_leaf_desc L) {
   const int tiles = (L.k + 63) / 64;
   delta_tile<false>(L, 1e-8f, (blockIdx.x / tiles) * 64, (blockIdx.x % tiles) * 64, -1, nullptr,
                     Ps, red);
+}
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_delta_part_one(scao_leaf_desc L, const float* tplanes,
+                                                        float* pplanes) {
+  __shared__ __attribute__((aligned(16))) float Ts[64][TSP];
+  const int tiles = (L.k + 63) / 64, tile = (int)blockIdx.x % (tiles * tiles);
+  delta_part(L, (tile / tiles) * 64, (tile % tiles) * 64, (int)blockIdx.x / (tiles * tiles),
+             tplanes, pplanes, Ts);
+}
+__global__ __launch_bounds__(256) void k_delta_finish_one(scao_leaf_desc L, const float* pplanes) {
+  __shared__ double red[16];
+  const int tiles = (L.k + 63) / 64;
+  delta_finish(L, 1e-8f, ((int)blockIdx.x / tiles) * 16, ((int)blockIdx.x % tiles) * 64, pplanes,
+               -1, nullptr, red);
 }
 __global__ __launch_bounds__(256) void k_lift_one(scao_leaf_desc L) {
   const int tiles = (L.k + 63) / 64;
@@ -1908,7 +2109,20 @@ __global__ __launch_bounds__(256) void k_apply_out_one(scao_leaf_desc L, const f
   apply_out_tile(L, G, out, (blockIdx.x / tiles) * 64, (blockIdx.x % tiles) * 64);
 }
 
-bool aligned16(const void* p) { return ((uintptr_t)p & 15u) == 0; }
+// whole projection tiles of the data type: 0 fp32, 1 bf16, 2 fp16
+template <bool DO_P, int CR, int NT>
+void launch_project(int type, dim3 g, hipStream_t s, const scao_task* tasks,
+                    const scao_leaf_desc* leaves, const scao_param_desc* params, double* slots) {
+  if (type == 0)
+    hipLaunchKernelGGL((k_project<DO_P, CR, NT, SCAO_F32, false>), g, dim3(NT), 0, s, tasks,
+                       leaves, params, slots);
+  else if (type == 1)
+    hipLaunchKernelGGL((k_project<DO_P, CR, NT, SCAO_BF16, false>), g, dim3(NT), 0, s, tasks,
+                       leaves, params, slots);
+  else
+    hipLaunchKernelGGL((k_project<DO_P, CR, NT, SCAO_F16, false>), g, dim3(NT), 0, s, tasks,
+                       leaves, params, slots);
+}
 
 }  // namespace
 
@@ -1919,32 +2133,31 @@ extern "C" int scao_kron_project(const scao_task* tasks, int ntasks, const scao_
   SCAO_CHECK_ARG(ntasks >= 0, "scao_kron_project: ntasks < 0");
   if (ntasks == 0) return SCAO_OK;
   SCAO_CHECK_ARG(tasks && leaves && params && slots, "scao_kron_project: null pointer");
-  SCAO_CHECK_ARG(variant >= 0 && variant < 12 && (variant < 4 || (variant & 1)) &&
-                     (variant & 12) != 12,
+  const int width = (variant >> 2) & 3, type = (variant >> 4) & 3;
+  SCAO_CHECK_ARG(variant >= 0 && variant < 64 && width < 3 && type < 3 &&
+                     ((variant & 1) || variant < 4),
                  "scao_kron_project: bad variant %d", variant);
   hipStream_t s = (hipStream_t)stream;
-  dim3 g(ntasks), b(256);
-  if (variant & 1) {
-    const dim3 b512(512), b128(X6_NT128);
-    switch (variant) {
-      case 1: hipLaunchKernelGGL((k_project_x6<false, 64, 256>), g, b, 0, s, tasks, leaves, params, slots); break;
-      case 3: hipLaunchKernelGGL((k_project_x6<true, 64, 256>), g, b, 0, s, tasks, leaves, params, slots); break;
-      case 5: hipLaunchKernelGGL((k_project_x6<false, 128, X6_NT128>), g, b128, 0, s, tasks, leaves, params, slots); break;
-      case 7: hipLaunchKernelGGL((k_project_x6<true, 128, X6_NT128>), g, b128, 0, s, tasks, leaves, params, slots); break;
-      case 9: hipLaunchKernelGGL((k_project_x6<false, 256, 512>), g, b512, 0, s, tasks, leaves, params, slots); break;
-      default: hipLaunchKernelGGL((k_project_x6<true, 256, 512>), g, b512, 0, s, tasks, leaves, params, slots); break;
+  const dim3 g(ntasks);
+  if (!(variant & 1)) {
+    if (variant & 2)
+      hipLaunchKernelGGL((k_project<true, 64, 256, SCAO_F32, true>), g, dim3(256), 0, s, tasks,
+                         leaves, params, slots);
+    else
+      hipLaunchKernelGGL((k_project<false, 64, 256, SCAO_F32, true>), g, dim3(256), 0, s, tasks,
+                         leaves, params, slots);
+  } else if (variant & 2) {
+    switch (width) {
+      case 0: launch_project<true, 64, 256>(type, g, s, tasks, leaves, params, slots); break;
+      case 1: launch_project<true, 128, 512>(type, g, s, tasks, leaves, params, slots); break;
+      default: launch_project<true, 256, 512>(type, g, s, tasks, leaves, params, slots); break;
     }
-    SCAO_LAUNCH_CHECK("scao_kron_project");
-    return SCAO_OK;
-  }
-  SCAO_CHECK_ARG(variant < 8, "scao_kron_project: variant %d needs the bf16 projection", variant);
-  switch (variant) {
-    case 0: hipLaunchKernelGGL((k_project<false, false>), g, b, 0, s, tasks, leaves, params, slots); break;
-    case 1: hipLaunchKernelGGL((k_project<true, false>), g, b, 0, s, tasks, leaves, params, slots); break;
-    case 2: hipLaunchKernelGGL((k_project<false, true>), g, b, 0, s, tasks, leaves, params, slots); break;
-    case 3: hipLaunchKernelGGL((k_project<true, true>), g, b, 0, s, tasks, leaves, params, slots); break;
-    case 5: hipLaunchKernelGGL((k_project<true, false, 128>), g, b, 0, s, tasks, leaves, params, slots); break;
-    default: hipLaunchKernelGGL((k_project<true, true, 128>), g, b, 0, s, tasks, leaves, params, slots); break;
+  } else {
+    switch (width) {
+      case 0: launch_project<false, 64, 256>(type, g, s, tasks, leaves, params, slots); break;
+      case 1: launch_project<false, 128, 512>(type, g, s, tasks, leaves, params, slots); break;
+      default: launch_project<false, 256, 512>(type, g, s, tasks, leaves, params, slots); break;
+    }
   }
   SCAO_LAUNCH_CHECK("scao_kron_project");
   return SCAO_OK;
@@ -1954,7 +2167,14 @@ extern "C" int scao_kron_delta(const scao_task* tasks, int ntasks, const scao_le
                                const scao_param_desc* params, double* slots, void* stream) {
   SCAO_CHECK_ARG(ntasks >= 0, "scao_kron_delta: ntasks < 0");
   if (ntasks == 0) return SCAO_OK;
-  SCAO_CHECK_ARG(tasks && leaves && params && slots, "scao_kron_delta: null pointer");
+  SCAO_CHECK_ARG(tasks && leaves, "scao_kron_delta: null pointer");
+  if (!slots) {
+    hipLaunchKernelGGL(k_delta_part, dim3(ntasks), dim3(256), 0, (hipStream_t)stream, tasks,
+                       leaves);
+    SCAO_LAUNCH_CHECK("scao_kron_delta");
+    return SCAO_OK;
+  }
+  SCAO_CHECK_ARG(params, "scao_kron_delta: null pointer");
   hipLaunchKernelGGL(k_delta, dim3(ntasks), dim3(256), 0, (hipStream_t)stream, tasks, leaves,
                      params, slots);
   SCAO_LAUNCH_CHECK("scao_kron_delta");
@@ -2063,19 +2283,55 @@ int launch_fused_kronecker(const float* U_l, const float* s_l_inv4, const float*
   L.n = (int)n;
   L.k = (int)k;
   L.flags = SCAO_LF_SINV4;
-  if (ldG % 4 == 0 && n % 4 == 0 && aligned16(G) && aligned16(ws) && aligned16(L.T))
-    L.flags |= SCAO_LF_VEC4;
+  L.flags |= SCAO_LF_VEC4;
   scao_param_desc P = {};
   P.g = G;
   P.graw = G;
   P.dtype = SCAO_F32;
-  const int strips = (int)((n + SCAO_PROJ_COLS - 1) / SCAO_PROJ_COLS);
-  const int kt = (int)((k + 63) / 64);
-  hipLaunchKernelGGL(k_project_one, dim3(strips * kt), dim3(256), 0, s, L, P);
+  // One block's strips are far fewer than the CUs, so the rows are split too
+  // (at least 128 per part, up to a workgroup per CU) and P is formed by column
+  // chunks.  Their planes of T and P live in `out`, which the last launch
+  // overwrites, so the scratch stays T, Delta and W.  An `out` that shares
+  // storage with G or has no room for the planes takes fewer parts or none.
+  // 2048 x 2048 at k = 64: projection 337 -> 13 us, P 69 -> 24 us.
+  const int64_t strips = (n + SCAO_PROJ_COLS - 1) / SCAO_PROJ_COLS;
+  const int cr = k > 128 ? 256 : k > 64 ? 128 : 64;
+  const int64_t kt = (k + cr - 1) / cr, pt = (k + 63) / 64;
+  const int64_t tp = plane_floats(k * n), pp = plane_floats(k * k);
+  int64_t chunks = (n + delta_cols((int)k) - 1) / delta_cols((int)k);
+  const bool apart = (uintptr_t)out >= (uintptr_t)(G + (m - 1) * ldG + n) ||
+                     (uintptr_t)(out + m * n) <= (uintptr_t)G;
+  const int64_t room = apart ? m * n : 0;
+  if (chunks > 255 || chunks * pp > room) chunks = 0;
+  int64_t parts = 1;
+  if (chunks) {
+    parts = std::min<int64_t>(std::min<int64_t>(m / 128, 256 / (strips * kt)),
+                              std::min<int64_t>(64, (room - chunks * pp) / tp));
+    parts = parts > 1 ? (m + split_rows((int)m, (int)parts) - 1) / split_rows((int)m, (int)parts) : 1;
+  }
+  L.flags |= (int)(parts << SCAO_LF_NSPLIT_SHIFT) | (int)(chunks << SCAO_LF_DCHUNK_SHIFT);
+  float* tplanes = out;
+  float* pplanes = out + (parts > 1 ? parts * tp : 0);
+  const dim3 gp((unsigned)(strips * kt * parts));
+  if (cr == 256)
+    hipLaunchKernelGGL((k_project_one<256, 512>), gp, dim3(512), 0, s, L, P, tplanes);
+  else if (cr == 128)
+    hipLaunchKernelGGL((k_project_one<128, 512>), gp, dim3(512), 0, s, L, P, tplanes);
+  else
+    hipLaunchKernelGGL((k_project_one<64, 256>), gp, dim3(256), 0, s, L, P, tplanes);
   SCAO_LAUNCH_CHECK("scao_fused_kronecker_precond/project");
-  hipLaunchKernelGGL(k_delta_one, dim3(kt * kt), dim3(256), 0, s, L);
+  if (chunks) {
+    hipLaunchKernelGGL(k_delta_part_one, dim3((unsigned)(pt * pt * chunks)), dim3(256), 0, s, L,
+                       tplanes, pplanes);
+    SCAO_LAUNCH_CHECK("scao_fused_kronecker_precond/delta part");
+    hipLaunchKernelGGL(k_delta_finish_one, dim3((unsigned)((k + 15) / 16 * pt)), dim3(256), 0, s, L,
+                       pplanes);
+  } else {
+    hipLaunchKernelGGL(k_delta_one, dim3((unsigned)(pt * pt)), dim3(256), 0, s, L);
+  }
   SCAO_LAUNCH_CHECK("scao_fused_kronecker_precond/delta");
-  hipLaunchKernelGGL(k_lift_one, dim3((int)((m + 63) / 64) * kt), dim3(256), 0, s, L);
+  const int kt64 = (int)pt;
+  hipLaunchKernelGGL(k_lift_one, dim3((int)((m + 63) / 64) * kt64), dim3(256), 0, s, L);
   SCAO_LAUNCH_CHECK("scao_fused_kronecker_precond/lift");
   hipLaunchKernelGGL(k_apply_out_one, dim3((int)((m + 63) / 64) * (int)((n + 63) / 64)),
                      dim3(256), 0, s, L, G, out);

@@ -83,6 +83,13 @@ __device__ __forceinline__ v4f mfma_x6(const bf3& a, const bf3& b, v4f c) {
   return mfma16bf(a.h, b.h, c);
 }
 
+// c + A b for an fp32 A (bf3 split) and a bf16 b: three exact products.
+__device__ __forceinline__ v4f mfma_x3(const bf3& a, const v8bf& b, v4f c) {
+  c = mfma16bf(a.l, b, c);
+  c = mfma16bf(a.m, b, c);
+  return mfma16bf(a.h, b, c);
+}
+
 // ------------------------------------------------------------- dtypes ---
 __device__ __forceinline__ float bf16_to_f(uint16_t h) {
   return __uint_as_float(((uint32_t)h) << 16);
@@ -115,9 +122,15 @@ __device__ __forceinline__ float round_to(int dt, float x) {
 // and become flat_* accesses).
 typedef __attribute__((address_space(1))) float gfloat;
 typedef __attribute__((address_space(1))) uint16_t gu16;
-typedef __attribute__((address_space(1))) v4f gv4f;
+// The vector accesses promise element alignment only (4 bytes for fp32, 2 for
+// 16-bit types): gfx950's global memory accesses take any address, and the
+// compiler emits the same dwordx4 / dwordx2 instructions as for aligned types.
+// A block's rows may then start anywhere (odd widths, sliced storage).
+typedef v4f v4f_a4 __attribute__((aligned(4)));
+typedef __attribute__((address_space(1))) v4f_a4 gv4f;
 typedef unsigned int v2u __attribute__((ext_vector_type(2)));
-typedef __attribute__((address_space(1))) v2u gv2u;
+typedef v2u v2u_a2 __attribute__((aligned(2)));
+typedef __attribute__((address_space(1))) v2u_a2 gv2u;
 
 __device__ __forceinline__ v4f gld4(const float* p) { return *(const gv4f*)p; }
 __device__ __forceinline__ void gst4(float* p, v4f x) { *(gv4f*)p = x; }
@@ -128,6 +141,7 @@ __device__ __forceinline__ v4f gld4_nt(const float* p) {
 __device__ __forceinline__ void gst4_nt(float* p, v4f x) {
   __builtin_nontemporal_store(x, (gv4f*)p);
 }
+__device__ __forceinline__ v2u gld2w(const void* p) { return *(const gv2u*)p; }
 __device__ __forceinline__ float gld1(const float* p) { return *(const gfloat*)p; }
 __device__ __forceinline__ void gst1(float* p, float x) { *(gfloat*)p = x; }
 // 16-byte alignment for fp32 float4 access, 8-byte for a 16-bit dtype's 4-pack

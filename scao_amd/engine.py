@@ -95,6 +95,7 @@ class PItem:
     diag: bool = False           # diagonal-mode preconditioner in Phase 2
     leaves: list = field(default_factory=list)  # [(leaf, r0, c0)]
     fp32: bool = True            # param and gradient are float32
+    half: int = 0                # param and gradient are both bf16 (1) or fp16 (2)
     aligned: bool = True         # every pointer of the param is 16-byte aligned
     msrc: "MomentSource | None" = None   # filter/noise formed inside the step kernels
     # device addresses, read once per step: p, graw, gmom, filter EMA (0 when
@@ -238,9 +239,10 @@ def _flat_chunks(numel: int) -> int:
     return (numel + L.FLAT_CHUNK - 1) // L.FLAT_CHUNK
 
 
-_LEAF_TASKS = ("delta", "lift")   # with proj* and apply*: idx is a block index
-_TASK_TYPES = (["adam", "delta", "lift", "dred", "dapply", "lars"] +
-               [f"proj{v}" for v in range(12)] + [f"apply{v}" for v in range(64)])
+_LEAF_TASKS = ("dpart", "delta", "lift")   # with proj* and apply*: idx is a block index
+_PROJ_VARIANTS = [0, 2] + [1 | p | w | t for t in (0, 16, 32) for w in (0, 4, 8) for p in (0, 2)]
+_TASK_TYPES = (["adam", "dpart", "delta", "lift", "dred", "dapply", "lars"] +
+               [f"proj{v}" for v in sorted({*range(12), *_PROJ_VARIANTS})] + [f"apply{v}" for v in range(64)])
 
 
 STEP_WIDTHS = (64, 128, 256)   # eigenfactor widths the step kernels are built for
@@ -262,7 +264,63 @@ def _leaf_k(leaf) -> int:
     return -(-k // 64) * 64
 
 
-def _param_tasks(it: PItem):
+class SplitPlan(NamedTuple):
+    """How a step cuts the reductions of its projection and delta stages."""
+    rows: int      # rows per part of the projection (0: whole columns)
+    chunks: bool   # P = T U_r by column chunks of the block's width
+
+
+PROJ_CHUNK = 32         # rows the projection kernel consumes at a time
+SPLIT_MIN_ROWS = 128    # fewest rows of a part
+CUS = 256               # MI355X
+
+
+def _split_plan(leaves) -> SplitPlan:
+    """The cut for a step over ``leaves``.
+
+    A projection task walks all rows of a 256-column strip and a delta task
+    all columns of a 64x64 tile of P, so a step over few blocks has too few of
+    either to fill the chip, each a long serial chain.  The rows are then
+    split into parts (the largest that give every CU work: two workgroups of
+    the 64-row kernel, one of the wider ones), and P is formed by column
+    chunks.  Both write planes that the delta stage adds in order, which costs
+    one more pass over T and P, so a step that fills the chip takes neither."""
+    tasks = []   # (rows, strips, CU share of a task) per block
+    tiles = 0
+    for lf in leaves:
+        if not lf.use_kronecker:
+            continue
+        k = _leaf_k(lf)
+        cr = 256 if k % 256 == 0 else 128 if k % 128 == 0 else 64
+        share = 1.0 if cr > 64 else 0.5
+        tasks.append((lf.m, -(-lf.n // L.PROJ_COLS) * (k // cr), share))
+        tiles += (k // 64) ** 2
+    rows = 0
+    if sum(c * w for _, c, w in tasks) < 0.6 * CUS:
+        for rows in (1024, 512, 256, SPLIT_MIN_ROWS):
+            if sum(-(-m // rows) * c * w for m, c, w in tasks) >= CUS:
+                break
+    return SplitPlan(rows, rows > 0 or tiles < CUS // 2)
+
+
+def _leaf_split(leaf, plan: SplitPlan) -> tuple:
+    """(row parts of the projection, rows of a part, column chunks of P) of a
+    block; the counts fit the 8-bit fields of the block's flags."""
+    parts, rows = 1, leaf.m
+    if not leaf.use_kronecker:
+        return parts, rows, 0
+    if plan.rows:
+        parts = min(255, -(-leaf.m // plan.rows))
+        # the kernel's split_rows(m, parts), then the parts that hold rows
+        rows = -(-leaf.m // (PROJ_CHUNK * parts)) * PROJ_CHUNK
+        parts = -(-leaf.m // rows)
+    chunks = -(-leaf.n // _leaf_k(leaf)) if plan.chunks else 0   # the kernel's delta_cols
+    if chunks > 255:
+        return 1, leaf.m, 0
+    return parts, rows, chunks
+
+
+def _param_tasks(it: PItem, plan: SplitPlan):
     """One parameter's share of a step structure, with local indices: block
     indices from 0 (first block of the parameter), parameter index 0, slots
     from 0.  Returns ({type: int32 array (n, 4)}, local slot ranges, slot
@@ -295,27 +353,28 @@ def _param_tasks(it: PItem):
                 continue
             m, n = leaf.m, leaf.n
             k = _leaf_k(leaf)
-            vec = _leaf_vec(it, leaf, r0, c0l)
-            # the bf16-split tiles address a lane's rows with a 32-bit byte
+            parts, rows, _ = _leaf_split(leaf, plan)
+            # a whole tile's lanes address their rows with a 32-bit byte
             # offset: 24 row strides + a strip, below 2^32 for rows under 2^25
-            short_rows = _cols(it.p) < (1 << 25)
+            typed = (it.fp32 or it.half) and _cols(it.p) < (1 << 25)
             for j0 in range(0, n, L.PROJ_COLS):
-                whole = (vec and it.fp32 and j0 + L.PROJ_COLS <= n and m % 32 == 0
-                         and short_rows)
-                # 128 or 256 rows of T per task where k allows (variant bits 4, 8)
-                cr = 64
-                if whole and k % 128 == 0:
-                    cr = 256 if k % 256 == 0 else 128
-                for c0 in range(0, k, cr):
-                    fast = whole and c0 + 64 <= k
-                    do_p = c0 == 0 and it.lars
-                    var = ((1 if fast else 0) | (2 if do_p else 0) | (4 if cr == 128 else 0)
-                           | (8 if cr == 256 else 0))
-                    if c0 == 0:
-                        add(f"proj{var}", (li, j0, c0, slot))
-                        slot += 1
-                    else:
-                        add(f"proj{var}", (li, j0, c0, -1))
+                for part in range(parts):
+                    nrows = min(rows, m - part * rows)
+                    whole = typed and j0 + L.PROJ_COLS <= n and nrows % PROJ_CHUNK == 0
+                    # 128 or 256 rows of T per task where k allows (variant bits 4, 8)
+                    cr = 64
+                    if whole and k % 128 == 0:
+                        cr = 256 if k % 256 == 0 else 128
+                    for c0 in range(0, k, cr):
+                        do_p = c0 == 0 and it.lars
+                        var = ((1 | (it.half << 4) if whole else 0) | (2 if do_p else 0)
+                               | (4 if cr == 128 else 0) | (8 if cr == 256 else 0))
+                        b = c0 | (part << 16)
+                        if c0 == 0:
+                            add(f"proj{var}", (li, j0, b, slot))
+                            slot += 1
+                        else:
+                            add(f"proj{var}", (li, j0, b, -1))
         for li, (leaf, _, _) in enumerate(leaves):
             if not leaf.use_kronecker:
                 # a diagonal sub-block: its norm partials, 64x64 tiles
@@ -325,8 +384,12 @@ def _param_tasks(it: PItem):
                         slot += 1
                 continue
             k = _leaf_k(leaf)
-            for a in range(0, k, 64):
-                for b in range(0, k, 64):
+            chunks = _leaf_split(leaf, plan)[2]
+            for b in range(0, k, 64):
+                for a in range(0, k, 64):
+                    for ch in range(chunks):
+                        add("dpart", (li, a, b | (ch << 16), -1))
+                for a in range(0, k, 16 if chunks else 64):
                     add("delta", (li, a, b, slot))
                     slot += 1
         pre_end = slot
@@ -380,7 +443,7 @@ def _param_tasks(it: PItem):
 def _item_key(it: PItem) -> tuple:
     """Everything _param_tasks reads from an item."""
     return (id(it.p), it.phase2, it.diag, it.lars, it.mgrad, it.p.numel(), it.fp32, it.aligned,
-            _cols(it.p), tuple((id(lf), r0, c0, _leaf_k(lf)) for lf, r0, c0 in it.leaves)
+            _cols(it.p), it.half, tuple((id(lf), r0, c0, _leaf_k(lf)) for lf, r0, c0 in it.leaves)
             if it.phase2 and not it.diag else ())
 
 
@@ -393,7 +456,9 @@ def _build_structure(items: list[PItem], cache: dict | None = None):
     the item and the module's tiling settings) and placed by offsets, so a
     step whose set of parameters changes (a parameter without a gradient,
     a rank change) costs array arithmetic, not a rebuild of every tile."""
-    knobs = (PIPE_MIN_RANK, L2_OPERANDS, L.APPLY_GROUP)
+    plan = _split_plan([lf for it in items if it.phase2 and not it.diag
+                        for lf, _, _ in it.leaves])
+    knobs = (PIPE_MIN_RANK, L2_OPERANDS, L.APPLY_GROUP, plan)
     if cache is not None and len(cache) > 4 * len(items) + 64:
         cache.clear()
     parts = {k: [] for k in _TASK_TYPES}
@@ -404,7 +469,7 @@ def _build_structure(items: list[PItem], cache: dict | None = None):
         key = (_item_key(it), knobs)
         frag = cache.get(key) if cache is not None else None
         if frag is None:
-            frag = _param_tasks(it)
+            frag = _param_tasks(it, plan)
             if cache is not None:
                 cache[key] = frag
         arrays, rng, nslot, lvs = frag
@@ -567,13 +632,17 @@ def _padded_factors(leaves, ws: Workspace) -> dict:
 
 
 def _leaf_table(leaves, items: list[PItem], ws: Workspace):
-    """Block descriptors plus T/Delta/W scratch for every Phase-2 block."""
+    """Block descriptors plus T/Delta/W scratch for every Phase-2 block (T and
+    Delta followed by the planes of a split reduction, _split_plan)."""
+    plan = _split_plan([lf for lf, *_ in leaves])
     sizes = []
     for (leaf, r0, c0, pi) in leaves:
         k = _leaf_k(leaf)
+        parts, _, chunks = _leaf_split(leaf, plan)
         # W, then (strip-apply ranks) its three bf16 planes: 1.5 floats per element
         wsz = _align4(leaf.m * k) + (_align4((3 * leaf.m * k + 1) // 2) if k in STRIP_RANKS else 0)
-        sizes.append((_align4(k * leaf.n), _align4(k * k), wsz))
+        sizes.append((_align4(k * leaf.n) * (1 + parts if parts > 1 else 1),
+                      _align4(k * k) * (1 + chunks), wsz))
     total = sum(a + b + c for a, b, c in sizes)
     scratch = ws.buf("leaf_scratch", max(total, 1) * 4)
     base = scratch.data_ptr()
@@ -609,7 +678,9 @@ def _leaf_table(leaves, items: list[PItem], ws: Workspace):
         off += st + sd + sw
         e["m"], e["n"], e["k"] = leaf.m, leaf.n, k
         vec = _leaf_vec(it, leaf, r0, c0) and _aligned16(int(e["T"]))
-        e["flags"] = L.LF_VEC4 if vec else 0
+        parts, _, chunks = _leaf_split(leaf, plan)
+        e["flags"] = ((L.LF_VEC4 if vec else 0) | (parts << L.LF_NSPLIT_SHIFT)
+                      | (chunks << L.LF_DCHUNK_SHIFT))
     return tab
 
 
@@ -618,6 +689,7 @@ def _leaf_table(leaves, items: list[PItem], ws: Workspace):
 # --------------------------------------------------------------------------
 
 _MOMENTS = ("exp_avg", "exp_avg_sq", "exp_avg_diff", "prev_grad")
+_HALF = {torch.bfloat16: 1, torch.float16: 2}   # PItem.half
 
 
 def _group_scalars(g: dict, t: int, phase2: bool, scao_step: int, lars: bool,
@@ -822,16 +894,17 @@ def run_step(items: list[PItem], ws: Workspace, update_norm_ema: bool,
     f32 = torch.float32
     for it in items:
         it.fp32 = it.p.dtype == f32 and it.graw.dtype == f32
+        it.half = _HALF.get(it.p.dtype, 0) if it.graw.dtype == it.p.dtype else 0
         it.ptrs = _item_ptrs(it)
         it.aligned = _aligned16(*it.ptrs)
     # the full structure key (with every block's rank) is only rebuilt when
     # the cheap one or the global factor epoch says something may have changed
     ckey = (tuple((id(it.p), it.phase2, it.diag, it.lars, it.mgrad, it.p.numel(),
-                   it.fp32, it.aligned, len(it.leaves)) for it in items), leaf_epoch())
+                   it.fp32, it.half, it.aligned, len(it.leaves)) for it in items), leaf_epoch())
     skey = ws.struct_key
     if ckey != ws.cheap_key:
         skey = tuple((id(it.p), it.phase2, it.diag, it.lars, it.mgrad, it.p.numel(),
-                      it.fp32, it.aligned,
+                      it.fp32, it.half, it.aligned,
                       tuple((id(lf), r0, c0, _leaf_k(lf)) for lf, r0, c0 in it.leaves))
                      for it in items)
         ws.cheap_key = ckey
@@ -909,9 +982,11 @@ def _launch_step(ws: Workspace, raw: np.ndarray, n: int, update_norm_ema: bool) 
 
     if N["adam"]:
         _call("scao_adam_step", tp("adam"), N["adam"], P, SL, s)
-    for var in range(12):
+    for var in _PROJ_VARIANTS:
         if N[f"proj{var}"]:
             _call("scao_kron_project", tp(f"proj{var}"), N[f"proj{var}"], LF, P, SL, var, s)
+    if N["dpart"]:
+        _call("scao_kron_delta", tp("dpart"), N["dpart"], LF, 0, 0, s)
     if N["delta"]:
         _call("scao_kron_delta", tp("delta"), N["delta"], LF, P, SL, s)
         _call("scao_kron_lift", tp("lift"), N["lift"], LF, s)
