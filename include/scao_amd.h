@@ -52,7 +52,6 @@ enum scao_dtype { SCAO_F32 = 0, SCAO_BF16 = 1, SCAO_F16 = 2 };
 #define SCAO_PF_NORM  32 /* accumulate ||g||^2 for the global grad-norm EMA         */
 #define SCAO_PF_GF32  64 /* the moments see another gradient than `graw`: the fp32
                             buffer `g`, or with FMASK/FNOISE one formed in-kernel   */
-#define SCAO_PF_ALIGNED 128 /* every pointer of the param is 16-byte aligned       */
 #define SCAO_PF_FMASK 256   /* moment grad = fp32(graw) * (fema >= *fthr): the sparse
                                filter's mask (scao_sparse_filter with out == NULL)  */
 #define SCAO_PF_FNOISE 512  /* moment grad += fp32(fnoise * z), z ~ N(0,1) drawn as
@@ -69,7 +68,7 @@ typedef struct scao_param_desc {
   float* exp_avg_sq;
   float* exp_avg_diff;
   float* prev_grad;
-  float* upd;               /* LARS staging of the update (numel) or NULL        */
+  float* upd;               /* LARS staging of the update (numel, dtype) or NULL */
   const float* diag_ema;    /* diagonal-mode curvature (numel) or NULL           */
   const float* fema;        /* SCAO_PF_FMASK: the filter's magnitude EMA (numel) */
   const float* fthr;        /* SCAO_PF_FMASK: device threshold of this step      */
@@ -117,7 +116,6 @@ typedef struct scao_leaf_desc {
 } scao_leaf_desc;
 
 #define SCAO_LF_SINV4 1     /* Sl/Sr already hold clamp(S,1e-8)^-1/4             */
-#define SCAO_LF_VEC4  2     /* off, ld, n multiples of 4 and 16-byte aligned     */
 #define SCAO_LF_DIAG  4     /* a diagonal sub-block (1 x n or m x 1 remainder of a
                                block-diagonal split): Sl is its m*n diag EMA, no
                                U/S/T/Delta/W, k = 0; it takes delta tasks (its
@@ -250,13 +248,13 @@ int scao_step_finalize(const scao_param_desc* params, int nparams, const double*
  *     update to upd (LARS params, ||u||^2 into slots) or the parameter.
  *     variant = (SCAO_PF_GF32 set ? 1 : 0) | (SCAO_PF_LARS set ? 2 : 0) |
  *     (fast ? 4 : 0); every task of a launch must belong to a parameter of
- *     that variant.  "fast" tasks promise fp32 data, SCAO_LF_VEC4,
- *     SCAO_PF_ALIGNED, k % 16 == 0 and a whole 16x256 tile at (a, b)
+ *     that variant.  "fast" tasks promise fp32 data (with variant | 64, bf16
+ *     or fp16), k % 16 == 0 and a whole 16x256 tile at (a, b)
  *     (SCAO_APPLY_WIDE_ROWS x SCAO_APPLY_WIDE_COLS); other tasks are masked
  *     64x64 tiles (SCAO_APPLY_TILE) at (a, b), clipped to the block.
  *     variant | 8 (with 4): the same fast tasks through a two-role pipeline,
  *     SCAO_APPLY_GROUP consecutive tasks per block (the engine's choice for
- *     k >= 128 other than 128 and 256).
+ *     k >= 128 other than 128 and 256; fp32 only).
  *     variant | 16 (with 4): strip runs for k = 256 (| 32: k = 128): a task
  *     (leaf, a, b, slot) covers min(SCAO_APPLY_GROUP, (mw - a) / TR) tiles
  *     of TR rows x SW columns going down from row a in the column strip at

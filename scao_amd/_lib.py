@@ -36,11 +36,10 @@ EIG_BAND = 16
 EIG_BANDW = 2 * EIG_BAND + 1
 
 F32, BF16, F16 = 0, 1, 2
-PF_DECAY, PF_LARS, PF_CLIP, PF_GSNR, PF_DIAG, PF_NORM, PF_GF32, PF_ALIGNED = (
-    1, 2, 4, 8, 16, 32, 64, 128)
+PF_DECAY, PF_LARS, PF_CLIP, PF_GSNR, PF_DIAG, PF_NORM, PF_GF32 = 1, 2, 4, 8, 16, 32, 64
 PF_FMASK, PF_FNOISE = 256, 512
 FILTER_THR_WORD = 2 * 2048 + 7
-LF_SINV4, LF_VEC4, LF_DIAG = 1, 2, 4
+LF_SINV4, LF_DIAG = 1, 4
 
 DTYPE_CODE = {torch.float32: F32, torch.bfloat16: BF16, torch.float16: F16}
 

@@ -40,29 +40,46 @@ __device__ __forceinline__ void write_slot(double* slots, int slot, double a, do
   slots[(int64_t)slot * SCAO_SLOT_WIDTH + 2] = c;
 }
 
+__device__ __forceinline__ v2u ld_halves_nt(const void* base, int64_t e) {
+  return __builtin_nontemporal_load((const gv2u*)((const uint16_t*)base + e));
+}
+__device__ __forceinline__ void st_halves_nt(void* base, int dt, int64_t e, const v4f& x) {
+  __builtin_nontemporal_store(v4f_to_halves(dt, x), (gv2u*)((uint16_t*)base + e));
+}
+
 // --------------------------------------------------------------- adam ---
-// FAST: fp32 data, 16-byte aligned, a full 4096-element chunk -- straight-line
-// non-temporal float4 traffic with every load of the thread issued first.
-template <bool FAST>
+// FAST: fp32 data (HALF: bf16 or fp16), a full 4096-element chunk --
+// straight-line non-temporal vector traffic with every load of the thread
+// issued first (323 M bf16 parameters: 1764 us through the masked form, 1490
+// here, 5.6 TB/s).
+template <bool FAST, bool HALF>
 __device__ __forceinline__ void adam_chunk(const scao_task& tk, const scao_param_desc& P,
                                            double* slots) {
   __shared__ double red[16];
-  const int dt = FAST ? SCAO_F32 : P.dtype;
+  const int dt = FAST && !HALF ? SCAO_F32 : P.dtype;
   const Chunk ch(tk, P.numel);
   const bool gf32 = P.flags & SCAO_PF_GF32;
   const bool fused = fused_mgrad(P);
   const bool fmask = P.flags & SCAO_PF_FMASK;
-  const bool aligned = FAST || (al_dt(P.p, dt) && al16(P.g) && al_dt(P.graw, dt) &&
-                                al16(P.exp_avg) && al16(P.exp_avg_sq) && al16(P.prev_grad) &&
-                                (!fmask || al16(P.fema)));
   const bool decay = P.flags & SCAO_PF_DECAY;
   const float alpha = round_to(dt, P.adam_alpha);
   v4f g[4], gr[4], p[4], m[4], v[4];
+  v2u hg[4], hp[4];   // HALF: gradient and parameter as loaded
   int mk[4];
 #pragma unroll
   for (int grp = 0; grp < 4; ++grp) {
     const int64_t e = ch.elem(grp);
-    if (FAST) {
+    if (FAST && HALF) {
+      mk[grp] = 15;
+      hg[grp] = ld_halves_nt(P.graw, e);
+      if (fmask)
+        g[grp] = gld4_nt(P.fema + e);
+      else if (gf32 && !fused)
+        g[grp] = gld4_nt((const float*)P.g + e);
+      hp[grp] = ld_halves_nt(P.p, e);
+      m[grp] = gld4_nt(P.exp_avg + e);
+      v[grp] = gld4_nt(P.exp_avg_sq + e);
+    } else if (FAST) {
       mk[grp] = 15;
       if (fused) {   // g holds the filter's EMA until finish_mgrad below
         gr[grp] = gld4_nt((const float*)P.graw + e);
@@ -76,7 +93,7 @@ __device__ __forceinline__ void adam_chunk(const scao_task& tk, const scao_param
       v[grp] = gld4_nt(P.exp_avg_sq + e);
     } else {
       mk[grp] = ch.mask(e);
-      const bool vec = aligned && mk[grp] == 15;
+      const bool vec = mk[grp] == 15;
       const v4f z = {0.f, 0.f, 0.f, 0.f};
       if (fused) {
         gr[grp] = mk[grp] ? ld4(P.graw, dt, e, vec, mk[grp]) : z;
@@ -88,6 +105,14 @@ __device__ __forceinline__ void adam_chunk(const scao_task& tk, const scao_param
       p[grp] = mk[grp] ? ld4(P.p, dt, e, vec, mk[grp]) : z;
       m[grp] = mk[grp] ? ldf4(P.exp_avg, e, vec, mk[grp]) : z;
       v[grp] = mk[grp] ? ldf4(P.exp_avg_sq, e, vec, mk[grp]) : z;
+    }
+  }
+  if (FAST && HALF) {
+#pragma unroll
+    for (int grp = 0; grp < 4; ++grp) {
+      gr[grp] = halves_to_v4f(dt, hg[grp]);
+      p[grp] = halves_to_v4f(dt, hp[grp]);
+      if (!fmask && (fused || !gf32)) g[grp] = gr[grp];
     }
   }
   if (fused) {
@@ -113,9 +138,12 @@ __device__ __forceinline__ void adam_chunk(const scao_task& tk, const scao_param
       gst4_nt(P.exp_avg + e, m[grp]);
       gst4_nt(P.exp_avg_sq + e, v[grp]);
       gst4_nt(P.prev_grad + e, g[grp]);
-      gst4_nt((float*)P.p + e, p[grp]);
+      if (HALF)
+        st_halves_nt(P.p, dt, e, p[grp]);
+      else
+        gst4_nt((float*)P.p + e, p[grp]);
     } else if (mk[grp]) {
-      const bool vec = aligned && mk[grp] == 15;
+      const bool vec = mk[grp] == 15;
       stf4(P.exp_avg, e, m[grp], vec, mk[grp]);
       stf4(P.exp_avg_sq, e, v[grp], vec, mk[grp]);
       stf4(P.prev_grad, e, g[grp], vec, mk[grp]);
@@ -127,9 +155,8 @@ __device__ __forceinline__ void adam_chunk(const scao_task& tk, const scao_param
   if (threadIdx.x == 0) write_slot(slots, tk.slot, x[0], 0.0, 0.0);
 }
 
-__device__ __forceinline__ bool flat_fast(const scao_task& tk, const scao_param_desc& P) {
-  return P.dtype == SCAO_F32 && (P.flags & SCAO_PF_ALIGNED) &&
-         (int64_t)(tk.a + 1) * SCAO_FLAT_CHUNK <= P.numel;
+__device__ __forceinline__ bool whole_chunk(const scao_task& tk, const scao_param_desc& P) {
+  return (int64_t)(tk.a + 1) * SCAO_FLAT_CHUNK <= P.numel;
 }
 
 __global__ __launch_bounds__(256) void k_adam(const scao_task* __restrict__ tasks,
@@ -137,10 +164,12 @@ __global__ __launch_bounds__(256) void k_adam(const scao_task* __restrict__ task
                                               double* slots) {
   const scao_task tk = tasks[blockIdx.x];
   const scao_param_desc& P = params[tk.idx];
-  if (flat_fast(tk, P))
-    adam_chunk<true>(tk, P, slots);
+  if (!whole_chunk(tk, P))
+    adam_chunk<false, false>(tk, P, slots);
+  else if (P.dtype == SCAO_F32)
+    adam_chunk<true, false>(tk, P, slots);
   else
-    adam_chunk<false>(tk, P, slots);
+    adam_chunk<true, true>(tk, P, slots);
 }
 
 // ------------------------------------------------------- diag reduce ---
@@ -152,7 +181,6 @@ __global__ __launch_bounds__(256) void k_diag_reduce(const scao_task* __restrict
   const scao_param_desc& P = params[tk.idx];
   const int dt = P.dtype;
   const Chunk ch(tk, P.numel);
-  const bool aligned = al_dt(P.p, dt) && al_dt(P.graw, dt) && al16(P.diag_ema);
   const bool decay = P.flags & SCAO_PF_DECAY;
   const bool lars = P.flags & SCAO_PF_LARS;
   double acc[3] = {0.0, 0.0, 0.0};
@@ -161,7 +189,7 @@ __global__ __launch_bounds__(256) void k_diag_reduce(const scao_task* __restrict
     const int64_t e = ch.elem(grp);
     const int mk = ch.mask(e);
     if (!mk) continue;
-    const bool vec = aligned && mk == 15;
+    const bool vec = mk == 15;
     const v4f g = ld4(P.graw, dt, e, vec, mk);
     const v4f dg = ldf4(P.diag_ema, e, vec, mk);
     v4f p = {0.f, 0.f, 0.f, 0.f};
@@ -194,17 +222,13 @@ __global__ __launch_bounds__(256) void k_diag_apply(const scao_task* __restrict_
   const scao_param_stat S = stat[tk.idx];
   const int dt = P.dtype;
   const Chunk ch(tk, P.numel);
-  const bool aligned = al_dt(P.p, dt) && al16(P.g) && al_dt(P.graw, dt) && al16(P.diag_ema) &&
-                       al16(P.exp_avg) && al16(P.exp_avg_sq) && al16(P.exp_avg_diff) &&
-                       al16(P.prev_grad) && (P.upd == nullptr || al16(P.upd)) &&
-                       (!(P.flags & SCAO_PF_FMASK) || al16(P.fema));
   double u2 = 0.0;
 #pragma unroll
   for (int grp = 0; grp < 4; ++grp) {
     const int64_t e = ch.elem(grp);
     const int mk = ch.mask(e);
     if (!mk) continue;
-    const bool vec = aligned && mk == 15;
+    const bool vec = mk == 15;
     const v4f graw = ld4(P.graw, dt, e, vec, mk);
     const v4f g = fused_mgrad(P)
                       ? finish_mgrad(P, e, graw,
@@ -227,43 +251,54 @@ __global__ __launch_bounds__(256) void k_diag_apply(const scao_task* __restrict_
 }
 
 // -------------------------------------------------------- lars write ---
-template <bool FAST>
+// The staged update is in the parameter's type: it enters the sum rounded to
+// that type anyway (reference optimizer.py:645, upd.to(p.dtype)).
+template <bool FAST, bool HALF>
 __device__ __forceinline__ void lars_chunk(const scao_task& tk, const scao_param_desc& P,
                                            float alpha) {
-  const int dt = FAST ? SCAO_F32 : P.dtype;
+  const int dt = FAST && !HALF ? SCAO_F32 : P.dtype;
   const Chunk ch(tk, P.numel);
-  const bool aligned = FAST || (al_dt(P.p, dt) && al16(P.upd));
   const bool decay = P.flags & SCAO_PF_DECAY;
   v4f u[4], p[4];
+  v2u hu[4], hp[4];   // HALF: as loaded
   int mk[4];
 #pragma unroll
   for (int grp = 0; grp < 4; ++grp) {
     const int64_t e = ch.elem(grp);
-    if (FAST) {
+    if (FAST && HALF) {
+      mk[grp] = 15;
+      hu[grp] = gld2w((const uint16_t*)P.upd + e);
+      hp[grp] = ld_halves_nt(P.p, e);
+    } else if (FAST) {
       mk[grp] = 15;
       u[grp] = gld4(P.upd + e);
       p[grp] = gld4_nt((const float*)P.p + e);
     } else {
       mk[grp] = ch.mask(e);
-      const bool vec = aligned && mk[grp] == 15;
+      const bool vec = mk[grp] == 15;
       const v4f z = {0.f, 0.f, 0.f, 0.f};
-      u[grp] = mk[grp] ? ldf4(P.upd, e, vec, mk[grp]) : z;
+      u[grp] = mk[grp] ? ld4(P.upd, dt, e, vec, mk[grp]) : z;
       p[grp] = mk[grp] ? ld4(P.p, dt, e, vec, mk[grp]) : z;
     }
   }
 #pragma unroll
   for (int grp = 0; grp < 4; ++grp) {
+    if (FAST && HALF) {
+      u[grp] = halves_to_v4f(dt, hu[grp]);
+      p[grp] = halves_to_v4f(dt, hp[grp]);
+    }
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
       const float pd = decay ? round_to(dt, p[grp][t] * P.decay) : p[grp][t];
-      p[grp][t] = round_to(dt, fmaf(round_to(dt, u[grp][t]), alpha, pd));
+      p[grp][t] = round_to(dt, fmaf(u[grp][t], alpha, pd));
     }
     const int64_t e = ch.elem(grp);
-    if (FAST) {
+    if (FAST && HALF)
+      st_halves_nt(P.p, dt, e, p[grp]);
+    else if (FAST)
       gst4_nt((float*)P.p + e, p[grp]);
-    } else if (mk[grp]) {
-      st4(P.p, dt, e, p[grp], aligned && mk[grp] == 15, mk[grp]);
-    }
+    else if (mk[grp])
+      st4(P.p, dt, e, p[grp], mk[grp] == 15, mk[grp]);
   }
 }
 
@@ -273,10 +308,12 @@ __global__ __launch_bounds__(256) void k_lars_write(const scao_task* __restrict_
   const scao_task tk = tasks[blockIdx.x];
   const scao_param_desc& P = params[tk.idx];
   const float alpha = stat[tk.idx].alpha;
-  if (flat_fast(tk, P))
-    lars_chunk<true>(tk, P, alpha);
+  if (!whole_chunk(tk, P))
+    lars_chunk<false, false>(tk, P, alpha);
+  else if (P.dtype == SCAO_F32)
+    lars_chunk<true, false>(tk, P, alpha);
   else
-    lars_chunk<false>(tk, P, alpha);
+    lars_chunk<true, true>(tk, P, alpha);
 }
 
 // ---------------------------------------------------------- diag ema ---
@@ -289,13 +326,12 @@ __global__ __launch_bounds__(256) void k_diag_ema(const scao_task* __restrict__ 
   const int dt = P.dtype;
   float* dg = const_cast<float*>(P.diag_ema);
   const Chunk ch(tk, P.numel);
-  const bool aligned = al_dt(P.graw, dt) && al16(dg);
 #pragma unroll
   for (int grp = 0; grp < 4; ++grp) {
     const int64_t e = ch.elem(grp);
     const int mk = ch.mask(e);
     if (!mk) continue;
-    const bool vec = aligned && mk == 15;
+    const bool vec = mk == 15;
     const v4f g = ld4(P.graw, dt, e, vec, mk);
     v4f d = ldf4(dg, e, vec, mk);
 #pragma unroll
@@ -314,14 +350,13 @@ __global__ __launch_bounds__(256) void k_lookahead(const scao_task* __restrict__
   const scao_lookahead_desc& D = descs[tk.idx];
   const int dt = D.dtype;
   const Chunk ch(tk, D.numel);
-  const bool aligned = al_dt(D.p, dt) && al_dt(D.slow, dt);
   v4f p[4], w[4];
   int mk[4];
 #pragma unroll
   for (int grp = 0; grp < 4; ++grp) {
     const int64_t e = ch.elem(grp);
     mk[grp] = ch.mask(e);
-    const bool vec = aligned && mk[grp] == 15;
+    const bool vec = mk[grp] == 15;
     const v4f z = {0.f, 0.f, 0.f, 0.f};
     p[grp] = mk[grp] ? ld4(D.p, dt, e, vec, mk[grp]) : z;
     w[grp] = mk[grp] ? ld4(D.slow, dt, e, vec, mk[grp]) : z;
@@ -330,7 +365,7 @@ __global__ __launch_bounds__(256) void k_lookahead(const scao_task* __restrict__
   for (int grp = 0; grp < 4; ++grp) {
     if (!mk[grp]) continue;
     const int64_t e = ch.elem(grp);
-    const bool vec = aligned && mk[grp] == 15;
+    const bool vec = mk[grp] == 15;
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
       const float d = round_to(dt, p[grp][t] - w[grp][t]);

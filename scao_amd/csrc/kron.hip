@@ -894,12 +894,11 @@ __device__ __forceinline__ void lift_tile(const scao_leaf_desc& L, int i0, int d
     return;
   }
   const int irow = i0 + 16 * w + (l % 16);
-  const bool kvec = (k % 4) == 0;
   for (int cb = 0; cb < k; cb += 16) {
     const int c = cb + 4 * kk;
     int cm = 0;
     for (int s = 0; s < 4; ++s) cm |= (c + s < k) ? (1 << s) : 0;
-    v4f a = (irow < m && cm) ? ldf4(L.Ul, (int64_t)irow * k + c, kvec && cm == 15, cm)
+    v4f a = (irow < m && cm) ? ldf4(L.Ul, (int64_t)irow * k + c, cm == 15, cm)
                              : v4f{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int s = 0; s < 4; ++s)
@@ -977,7 +976,6 @@ __device__ __forceinline__ void corr_tile(const scao_leaf_desc& L, int i0, int j
   const int m = L.m, n = L.n, k = L.k;
   const int kk = l / 16;
   const int irow = i0 + 16 * w + (l % 16);
-  const bool kvec = (k % 4) == 0;
 #pragma unroll
   for (int t = 0; t < 4; ++t) acc[t] = v4f{0.f, 0.f, 0.f, 0.f};
   if (k % 16 == 0) {
@@ -987,16 +985,22 @@ __device__ __forceinline__ void corr_tile(const scao_leaf_desc& L, int i0, int j
     const float* urow[4];
 #pragma unroll
     for (int t = 0; t < 4; ++t) urow[t] = L.Ur + (int64_t)min(jl + t, n - 1) * k + 4 * kk;
-#pragma unroll 4
-    for (int cb = 0; cb < k; cb += 16) {
-      const v4f a = gld4(wrow + cb);
-      v4f b[4];
+    v4f a = gld4(wrow), b[4];
 #pragma unroll
-      for (int t = 0; t < 4; ++t) b[t] = gld4(urow[t] + cb);
+    for (int t = 0; t < 4; ++t) b[t] = gld4(urow[t]);
+    for (int cb = 0; cb < k; cb += 16) {
+      const int cn = cb + 16 < k ? cb + 16 : cb;   // the last chunk repeats itself, unused
+      const v4f an = gld4(wrow + cn);
+      v4f bn[4];
+#pragma unroll
+      for (int t = 0; t < 4; ++t) bn[t] = gld4(urow[t] + cn);
 #pragma unroll
       for (int s = 0; s < 4; ++s)
 #pragma unroll
         for (int t = 0; t < 4; ++t) acc[t] = mfma16(a[s], b[t][s], acc[t]);
+      a = an;
+#pragma unroll
+      for (int t = 0; t < 4; ++t) b[t] = bn[t];
     }
     return;
   }
@@ -1004,13 +1008,13 @@ __device__ __forceinline__ void corr_tile(const scao_leaf_desc& L, int i0, int j
     const int c = cb + 4 * kk;
     int cm = 0;
     for (int s = 0; s < 4; ++s) cm |= (c + s < k) ? (1 << s) : 0;
-    const v4f a = (irow < m && cm) ? ldf4(L.W, (int64_t)irow * k + c, kvec && cm == 15, cm)
+    const v4f a = (irow < m && cm) ? ldf4(L.W, (int64_t)irow * k + c, cm == 15, cm)
                                    : v4f{0.f, 0.f, 0.f, 0.f};
     v4f b[4];
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
       const int j = jl + t;
-      b[t] = (j < n && cm) ? ldf4(L.Ur, (int64_t)j * k + c, kvec && cm == 15, cm)
+      b[t] = (j < n && cm) ? ldf4(L.Ur, (int64_t)j * k + c, cm == 15, cm)
                            : v4f{0.f, 0.f, 0.f, 0.f};
     }
 #pragma unroll
@@ -1023,6 +1027,33 @@ __device__ __forceinline__ void corr_tile(const scao_leaf_desc& L, int i0, int j
 }  // namespace
 
 namespace {
+
+// Four consecutive gradient (or parameter) values as loaded by a streaming
+// tile: fp32, or (HALF) two words of a 16-bit type, kept raw until the tail
+// converts them so that no wait sits between the loads.
+template <bool HALF> struct raw4 { typedef v4f type; };
+template <> struct raw4<true> { typedef v2u type; };
+template <bool HALF>
+__device__ __forceinline__ typename raw4<HALF>::type ld_raw4_nt(const void* base, int64_t e) {
+  if constexpr (HALF)
+    return __builtin_nontemporal_load((const gv2u*)((const uint16_t*)base + e));
+  else
+    return gld4_nt((const float*)base + e);
+}
+template <bool HALF>
+__device__ __forceinline__ v4f from_raw4(int dt, const typename raw4<HALF>::type& x) {
+  if constexpr (HALF)
+    return halves_to_v4f(dt, x);
+  else
+    return x;
+}
+template <bool HALF>
+__device__ __forceinline__ void st_raw4_nt(void* base, int dt, int64_t e, const v4f& x) {
+  if constexpr (HALF)
+    __builtin_nontemporal_store(v4f_to_halves(dt, x), (gv2u*)((uint16_t*)base + e));
+  else
+    gst4_nt((float*)base + e, x);
+}
 
 // The Phase-2 elementwise tail for one row of four columns (t = 0..3):
 // gp = G + corr -> clip -> blend -> Adan moments -> update.  With LARS the
@@ -1100,7 +1131,7 @@ __device__ __forceinline__ void apply_tile(const scao_leaf_desc& L, const scao_p
   const int jl = j0 + 4 * (l % 16);
   int cmask = 15;
   for (int t = 0; t < 4; ++t) cmask = (jl + t < n) ? cmask : (cmask & ~(1 << t));
-  const bool vec = (L.flags & SCAO_LF_VEC4) && cmask == 15;
+  const bool vec = cmask == 15;
 
   // 1) prefetch
   v4f gr[4], gm[4], mm[4], vv[4], dd[4], pp[4], par[4];
@@ -1147,7 +1178,6 @@ __device__ __forceinline__ void apply_tile(const scao_leaf_desc& L, const scao_p
     }
   }
   const int irow = i0 + 16 * w + (l % 16);
-  const bool kvec = (k % 4) == 0;
   for (int cb0 = 0; cb0 < (dleaf ? 0 : k); cb0 += 64) {
     if (cb0) __syncthreads();
 #pragma unroll
@@ -1157,7 +1187,7 @@ __device__ __forceinline__ void apply_tile(const scao_leaf_desc& L, const scao_p
       const int j = j0 + row, c = cb0 + c4;
       int mk = 0;
       for (int t = 0; t < 4; ++t) mk |= (j < n && c + t < k) ? (1 << t) : 0;
-      const v4f x = mk ? ldf4(L.Ur, (int64_t)j * k + c, kvec && mk == 15, mk)
+      const v4f x = mk ? ldf4(L.Ur, (int64_t)j * k + c, mk == 15, mk)
                        : v4f{0.f, 0.f, 0.f, 0.f};
       *(v4f*)&Us[row][c4] = x;
     }
@@ -1167,7 +1197,7 @@ __device__ __forceinline__ void apply_tile(const scao_leaf_desc& L, const scao_p
       const int c = cb0 + cb + 4 * kk;
       int cm = 15;
       for (int s = 0; s < 4; ++s) cm = (c + s < k) ? cm : (cm & ~(1 << s));
-      const v4f a = (irow < m && cm) ? ldf4(L.W, (int64_t)irow * k + c, kvec && cm == 15, cm)
+      const v4f a = (irow < m && cm) ? ldf4(L.W, (int64_t)irow * k + c, cm == 15, cm)
                                      : v4f{0.f, 0.f, 0.f, 0.f};
       v4f b[4];
 #pragma unroll
@@ -1193,28 +1223,27 @@ __device__ __forceinline__ void apply_tile(const scao_leaf_desc& L, const scao_p
     stf4(P.exp_avg_sq, e[r], vv[r], vec, cmask);
     stf4(P.exp_avg_diff, e[r], dd[r], vec, cmask);
     stf4(P.prev_grad, e[r], GF32 ? gm[r] : gr[r], vec, cmask);
-    if (LARS)
-      stf4(P.upd, e[r], out, vec, cmask);
-    else
-      st4(P.p, dt, e[r], out, vec, cmask);
+    st4(LARS ? (void*)P.upd : P.p, dt, e[r], out, vec, cmask);
   }
   write_u2_slot(slots, slot, u2, red);
 }
 
-// One 16x256 tile, wholly inside an fp32 block whose rows are 16-byte
-// aligned, k % 16 == 0.  A 16-row x 1 KB footprint per block streams
+// One 16x256 tile, wholly inside a block of fp32 or (HALF) 16-bit data whose
+// rows may start at any element, k % 16 == 0.  (One Llama-1B layer in bf16: 628
+// us on masked 64x64 tiles, 423 here; HBM bounds it, 36 B per element.)  A 16-row x 1 KB footprint per block streams
 // measurably faster than 64 rows x 256 B.  Wave w owns columns
 // j0+64w .. j0+64w+63 of all 16 rows; lane l holds rows i0+4*(l/16)+r and
 // columns jl..jl+3, jl = j0+64w+4*(l%16).  The correction for those columns
 // needs U_r rows private to the wave, so they are read straight from L2 in
 // the MFMA B layout; the 16 rows of W are common to the four waves.
-template <bool GF32, bool LARS>
+template <bool GF32, bool LARS, bool HALF>
 __device__ __forceinline__ void apply_wide(const scao_leaf_desc& L, const scao_param_desc& P,
                                            const scao_param_stat& S, int i0, int j0, int slot,
                                            double* slots) {
   __shared__ double red[16];
   const int w = threadIdx.x / 64, l = threadIdx.x % 64;
   const int k = L.k;
+  const int dt = HALF ? P.dtype : SCAO_F32;
   const int kk = l / 16;
   const int jl = j0 + 64 * w + 4 * (l % 16);
 
@@ -1222,7 +1251,8 @@ __device__ __forceinline__ void apply_wide(const scao_leaf_desc& L, const scao_p
   // operands when k = 64, before them otherwise).  A fused filter's EMA goes
   // first: its keep bits are taken as soon as the back-projection allows,
   // which frees its registers for the rest of the tile.
-  v4f gr[4], gm[4], mm[4], vv[4], dd[4], pp[4], par[4];
+  typename raw4<HALF>::type gr[4], par[4];
+  v4f gm[4], mm[4], vv[4], dd[4], pp[4];
   int64_t e[4];
   const bool fmask = GF32 && (P.flags & SCAO_PF_FMASK);
   auto load_elem = [&]() {
@@ -1230,13 +1260,13 @@ __device__ __forceinline__ void apply_wide(const scao_leaf_desc& L, const scao_p
     for (int r = 0; r < 4; ++r) {
       e[r] = L.off + (int64_t)(i0 + 4 * kk + r) * L.ld + jl;
       if (fmask) gm[r] = gld4_nt(P.fema + e[r]);
-      gr[r] = gld4_nt((const float*)P.graw + e[r]);
+      gr[r] = ld_raw4_nt<HALF>(P.graw, e[r]);
       if (GF32 && !fused_mgrad(P)) gm[r] = gld4_nt((const float*)P.g + e[r]);
       mm[r] = gld4_nt(P.exp_avg + e[r]);
       vv[r] = gld4_nt(P.exp_avg_sq + e[r]);
       dd[r] = gld4_nt(P.exp_avg_diff + e[r]);
       pp[r] = gld4_nt(P.prev_grad + e[r]);
-      if (!LARS) par[r] = gld4_nt((const float*)P.p + e[r]);
+      if (!LARS) par[r] = ld_raw4_nt<HALF>(P.p, e[r]);
     }
   };
 
@@ -1310,22 +1340,21 @@ __device__ __forceinline__ void apply_wide(const scao_leaf_desc& L, const scao_p
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
     const v4f corr = {acc[0][r], acc[1][r], acc[2][r], acc[3][r]};
-    if (GF32 && fused_mgrad(P)) gm[r] = finish_mgrad_bits(P, e[r], gr[r], (keep >> (4 * r)) & 15u, 15);
+    const v4f graw = from_raw4<HALF>(dt, gr[r]);
+    const v4f parv = LARS ? v4f{0.f, 0.f, 0.f, 0.f} : from_raw4<HALF>(dt, par[r]);
+    if (GF32 && fused_mgrad(P)) gm[r] = finish_mgrad_bits(P, e[r], graw, (keep >> (4 * r)) & 15u, 15);
     v4f out;
-    adan4<GF32, LARS>(P, S, SCAO_F32, gr[r], gm[r], corr, mm[r], vv[r], dd[r], pp[r], par[r], out,
+    adan4<GF32, LARS>(P, S, dt, graw, gm[r], corr, mm[r], vv[r], dd[r], pp[r], parv, out,
                       u2, 15);
     gst4_nt(P.exp_avg + e[r], mm[r]);
     gst4_nt(P.exp_avg_sq + e[r], vv[r]);
     gst4_nt(P.exp_avg_diff + e[r], dd[r]);
-    gst4_nt(P.prev_grad + e[r], GF32 ? gm[r] : gr[r]);
+    gst4_nt(P.prev_grad + e[r], GF32 ? gm[r] : graw);
     // the staged update streams past the caches too: it is read back only by
     // k_lars_write, after gigabytes of other traffic, and a caching store
     // evicts the U_r rows the tiles read from L2 (C3 step 12.17 -> 11.98 ms in
     // alternating runs; the strip apply at k = 256 measured slower with it)
-    if (LARS)
-      gst4_nt(P.upd + e[r], out);
-    else
-      gst4_nt((float*)P.p + e[r], out);
+    st_raw4_nt<HALF>(LARS ? (void*)P.upd : P.p, dt, e[r], out);
   }
   write_u2_slot(slots, slot, u2, red);
 }
@@ -1768,7 +1797,7 @@ __device__ __forceinline__ void strip_corr_bf(strip_a (&A)[PD], const uint16_t* 
   }
 }
 
-template <bool GF32, bool LARS, int K>
+template <bool GF32, bool LARS, int K, bool HALF>
 __global__ __launch_bounds__(strip_shape<K>::NT) void k_apply_strip(const scao_task* __restrict__ tasks,
                                                      const scao_leaf_desc* __restrict__ leaves,
                                                      const scao_param_desc* __restrict__ params,
@@ -1896,25 +1925,27 @@ __global__ __launch_bounds__(strip_shape<K>::NT) void k_apply_strip(const scao_t
   const int w = wv, rg = w % RG, cg = w / RG;
   const scao_param_desc& P = params[L.param];
   const scao_param_stat& S = stat[L.param];
-  v4f gr[4], gm[4], mm[4], vv[4], dd[4], pp[4], par[4];
+  const int dt = HALF ? P.dtype : SCAO_F32;
+  typename raw4<HALF>::type gr[4], par[4];
+  v4f gm[4], mm[4], vv[4], dd[4], pp[4];
   int64_t e[4];
   const int jc = tk.b + 64 * cg + 4 * (l % 16);
   auto prefetch = [&](int s) {
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       e[r] = L.off + (int64_t)(tk.a + s * TR + 16 * rg + 4 * kk + r) * L.ld + jc;
-      gr[r] = gld4_nt((const float*)P.graw + e[r]);
+      gr[r] = ld_raw4_nt<HALF>(P.graw, e[r]);
       if (GF32) {
         if (!fused_mgrad(P))
           gm[r] = gld4_nt((const float*)P.g + e[r]);
-        else
-          gm[r] = (P.flags & SCAO_PF_FMASK) ? gld4_nt(P.fema + e[r]) : gr[r];
+        else if (P.flags & SCAO_PF_FMASK)
+          gm[r] = gld4_nt(P.fema + e[r]);
       }
       mm[r] = gld4_nt(P.exp_avg + e[r]);
       vv[r] = gld4_nt(P.exp_avg_sq + e[r]);
       dd[r] = gld4_nt(P.exp_avg_diff + e[r]);
       pp[r] = gld4_nt(P.prev_grad + e[r]);
-      if (!LARS) par[r] = gld4_nt((const float*)P.p + e[r]);
+      if (!LARS) par[r] = ld_raw4_nt<HALF>(P.p, e[r]);
     }
   };
   auto put_slot = [&](int s) {
@@ -1945,18 +1976,20 @@ __global__ __launch_bounds__(strip_shape<K>::NT) void k_apply_strip(const scao_t
     for (int r = 0; r < 4; ++r) {
       const v4f corr =
           BF ? cr[r] : *(const v4f*)&cbuf[s & 1][16 * rg + 4 * kk + r][64 * cg + 4 * (l % 16)];
-      if (GF32 && fused_mgrad(P)) gm[r] = finish_mgrad(P, e[r], gr[r], gm[r], 15);
+      const v4f graw = from_raw4<HALF>(dt, gr[r]);
+      const v4f parv = LARS ? v4f{0.f, 0.f, 0.f, 0.f} : from_raw4<HALF>(dt, par[r]);
+      if (GF32 && fused_mgrad(P)) gm[r] = finish_mgrad(P, e[r], graw, gm[r], 15);
       v4f out;
-      adan4<GF32, LARS>(P, S, SCAO_F32, gr[r], gm[r], corr, mm[r], vv[r], dd[r], pp[r], par[r],
+      adan4<GF32, LARS>(P, S, dt, graw, gm[r], corr, mm[r], vv[r], dd[r], pp[r], parv,
                         out, u2, 15);
       gst4_nt(P.exp_avg + e[r], mm[r]);
       gst4_nt(P.exp_avg_sq + e[r], vv[r]);
       gst4_nt(P.exp_avg_diff + e[r], dd[r]);
-      gst4_nt(P.prev_grad + e[r], GF32 ? gm[r] : gr[r]);
-      if (LARS)
+      gst4_nt(P.prev_grad + e[r], GF32 ? gm[r] : graw);
+      if (LARS && !HALF)
         gst4(P.upd + e[r], out);
       else
-        gst4_nt((float*)P.p + e[r], out);
+        st_raw4_nt<HALF>(LARS ? (void*)P.upd : P.p, dt, e[r], out);
     }
     const double wsum = wave_sum((double)u2);
     if (l == 0) part[s & 1][w] = wsum;
@@ -1976,17 +2009,15 @@ __device__ __forceinline__ void apply_out_tile(const scao_leaf_desc& L, const fl
   corr_tile(L, i0, jl, acc);
   int cmask = 0;
   for (int t = 0; t < 4; ++t) cmask |= (jl + t < n) ? (1 << t) : 0;
-  const bool gvec = (L.flags & SCAO_LF_VEC4) && cmask == 15;
-  const bool ovec = (n % 4 == 0) && cmask == 15;
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
     const int i = i0 + 16 * w + 4 * (l / 16) + r;
     if (i >= m || !cmask) continue;
-    const v4f g = ldf4(G, (int64_t)i * L.ld + jl, gvec, cmask);
+    const v4f g = ldf4(G, (int64_t)i * L.ld + jl, cmask == 15, cmask);
     v4f o;
 #pragma unroll
     for (int t = 0; t < 4; ++t) o[t] = g[t] + acc[t][r];
-    stf4(out, (int64_t)i * n + jl, o, ovec, cmask);
+    stf4(out, (int64_t)i * n + jl, o, cmask == 15, cmask);
   }
 }
 
@@ -2045,7 +2076,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   else
     lift_tile(L, tk.a, tk.b);
 }
-template <bool GF32, bool LARS, bool FAST>
+template <bool GF32, bool LARS, bool FAST, bool HALF = false>
 __global__ __launch_bounds__(256) void k_apply(const scao_task* __restrict__ tasks,
                                                const scao_leaf_desc* __restrict__ leaves,
                                                const scao_param_desc* __restrict__ params,
@@ -2054,7 +2085,7 @@ __global__ __launch_bounds__(256) void k_apply(const scao_task* __restrict__ tas
   const scao_task tk = tasks[blockIdx.x];
   const scao_leaf_desc L = leaves[tk.idx];
   if (FAST)
-    apply_wide<GF32, LARS>(L, params[L.param], stat[L.param], tk.a, tk.b, tk.slot, slots);
+    apply_wide<GF32, LARS, HALF>(L, params[L.param], stat[L.param], tk.a, tk.b, tk.slot, slots);
   else
     apply_tile<GF32, LARS>(L, params[L.param], stat[L.param], tk.a, tk.b, tk.slot, slots);
 }
@@ -2197,14 +2228,20 @@ extern "C" int scao_kron_apply(const scao_task* tasks, int ntasks, const scao_le
   SCAO_CHECK_ARG(ntasks >= 0, "scao_kron_apply: ntasks < 0");
   if (ntasks == 0) return SCAO_OK;
   SCAO_CHECK_ARG(tasks && leaves && params && stat && slots, "scao_kron_apply: null pointer");
-  SCAO_CHECK_ARG(variant >= 0 && variant < 64 && (variant < 8 || (variant & 4)),
+  const bool half = variant & 64;
+  SCAO_CHECK_ARG(variant >= 0 && variant < 128 && ((variant & ~3) == 0 || (variant & 4)) &&
+                     !(half && (variant & 8)),
                  "scao_kron_apply: bad variant %d", variant);
   hipStream_t s = (hipStream_t)stream;
   if (variant & 16) {
     const dim3 gs(ntasks);
-#define SCAO_APPLY_STRIP(GF, LA, KR)                                                          \
-  hipLaunchKernelGGL((k_apply_strip<GF, LA, KR>), gs, dim3(strip_shape<KR>::NT), 0, s, tasks, \
-                     leaves, params, stat, slots)
+#define SCAO_APPLY_STRIP(GF, LA, KR)                                                            \
+  if (half)                                                                                     \
+    hipLaunchKernelGGL((k_apply_strip<GF, LA, KR, true>), gs, dim3(strip_shape<KR>::NT), 0, s,  \
+                       tasks, leaves, params, stat, slots);                                     \
+  else                                                                                          \
+    hipLaunchKernelGGL((k_apply_strip<GF, LA, KR, false>), gs, dim3(strip_shape<KR>::NT), 0, s, \
+                       tasks, leaves, params, stat, slots)
     if (variant & 32) {
       switch (variant & 3) {
         case 0: SCAO_APPLY_STRIP(false, false, 128); break;
@@ -2239,8 +2276,8 @@ extern "C" int scao_kron_apply(const scao_task* tasks, int ntasks, const scao_le
     return SCAO_OK;
   }
   dim3 g(ntasks), b(256);
-#define SCAO_APPLY(GF, LA, FA) \
-  hipLaunchKernelGGL((k_apply<GF, LA, FA>), g, b, 0, s, tasks, leaves, params, stat, slots)
+#define SCAO_APPLY(...) \
+  hipLaunchKernelGGL((k_apply<__VA_ARGS__>), g, b, 0, s, tasks, leaves, params, stat, slots)
   switch (variant) {
     case 0: SCAO_APPLY(false, false, false); break;
     case 1: SCAO_APPLY(true, false, false); break;
@@ -2249,7 +2286,11 @@ extern "C" int scao_kron_apply(const scao_task* tasks, int ntasks, const scao_le
     case 4: SCAO_APPLY(false, false, true); break;
     case 5: SCAO_APPLY(true, false, true); break;
     case 6: SCAO_APPLY(false, true, true); break;
-    default: SCAO_APPLY(true, true, true); break;
+    case 7: SCAO_APPLY(true, true, true); break;
+    case 68: SCAO_APPLY(false, false, true, true); break;
+    case 69: SCAO_APPLY(true, false, true, true); break;
+    case 70: SCAO_APPLY(false, true, true, true); break;
+    default: SCAO_APPLY(true, true, true, true); break;
   }
 #undef SCAO_APPLY
   SCAO_LAUNCH_CHECK("scao_kron_apply");
@@ -2283,7 +2324,6 @@ int launch_fused_kronecker(const float* U_l, const float* s_l_inv4, const float*
   L.n = (int)n;
   L.k = (int)k;
   L.flags = SCAO_LF_SINV4;
-  L.flags |= SCAO_LF_VEC4;
   scao_param_desc P = {};
   P.g = G;
   P.graw = G;

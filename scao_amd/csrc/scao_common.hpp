@@ -166,20 +166,35 @@ __device__ __forceinline__ void st1(void* base, int dt, int64_t i, float x) {
   }
 }
 
-// Four consecutive elements starting at element i.  `vec` promises 16-byte
-// (fp32) / 8-byte (16-bit) alignment and that all four are in bounds; else
-// element t is loaded only when mask bit t is set (zero otherwise).
+// four packed 16-bit values (bf16 or fp16) <-> float
+__device__ __forceinline__ v4f halves_to_v4f(int dt, const v2u& x) {
+  v4f r;
+  if (dt == SCAO_BF16) {
+    r = v4f{__uint_as_float(x[0] << 16), __uint_as_float(x[0] & 0xffff0000u),
+            __uint_as_float(x[1] << 16), __uint_as_float(x[1] & 0xffff0000u)};
+  } else {
+#pragma unroll
+    for (int t = 0; t < 4; ++t) r[t] = f16_to_f((uint16_t)(x[t / 2] >> (16 * (t & 1))));
+  }
+  return r;
+}
+__device__ __forceinline__ v2u v4f_to_halves(int dt, const v4f& x) {
+  uint16_t h[4];
+#pragma unroll
+  for (int t = 0; t < 4; ++t) h[t] = dt == SCAO_BF16 ? f_to_bf16(x[t]) : f_to_f16(x[t]);
+  return v2u{(uint32_t)h[0] | ((uint32_t)h[1] << 16), (uint32_t)h[2] | ((uint32_t)h[3] << 16)};
+}
+
+// Four consecutive elements starting at element i.  `vec` promises that all
+// four are in bounds; else element t is loaded only when mask bit t is set
+// (zero otherwise).
 __device__ __forceinline__ v4f ld4(const void* base, int dt, int64_t i, bool vec, int mask) {
   v4f r = {0.f, 0.f, 0.f, 0.f};
   if (vec) {
-    if (dt == SCAO_F32) {
+    if (dt == SCAO_F32)
       r = gld4((const float*)base + i);
-    } else {
-      const v2u x = *(const gv2u*)((const uint16_t*)base + i);
-      uint16_t h[4] = {(uint16_t)(x[0] & 0xffff), (uint16_t)(x[0] >> 16), (uint16_t)(x[1] & 0xffff),
-                       (uint16_t)(x[1] >> 16)};
-      for (int t = 0; t < 4; ++t) r[t] = dt == SCAO_BF16 ? bf16_to_f(h[t]) : f16_to_f(h[t]);
-    }
+    else
+      r = halves_to_v4f(dt, gld2w((const uint16_t*)base + i));
   } else {
     for (int t = 0; t < 4; ++t)
       if (mask & (1 << t)) r[t] = ld1(base, dt, i + t);
@@ -188,14 +203,10 @@ __device__ __forceinline__ v4f ld4(const void* base, int dt, int64_t i, bool vec
 }
 __device__ __forceinline__ void st4(void* base, int dt, int64_t i, v4f x, bool vec, int mask) {
   if (vec) {
-    if (dt == SCAO_F32) {
+    if (dt == SCAO_F32)
       gst4((float*)base + i, x);
-    } else {
-      uint16_t h[4];
-      for (int t = 0; t < 4; ++t) h[t] = dt == SCAO_BF16 ? f_to_bf16(x[t]) : f_to_f16(x[t]);
-      const v2u y = {(uint32_t)h[0] | ((uint32_t)h[1] << 16), (uint32_t)h[2] | ((uint32_t)h[3] << 16)};
-      *(gv2u*)((uint16_t*)base + i) = y;
-    }
+    else
+      *(gv2u*)((uint16_t*)base + i) = v4f_to_halves(dt, x);
   } else {
     for (int t = 0; t < 4; ++t)
       if (mask & (1 << t)) st1(base, dt, i + t, x[t]);
@@ -421,7 +432,7 @@ __device__ __forceinline__ float write_update(const scao_param_desc& P, int64_t 
   const int dt = P.dtype;
   float u2 = 0.f;
   if (P.flags & SCAO_PF_LARS) {
-    stf4(P.upd, e, u, vec, mask);
+    st4(P.upd, dt, e, u, vec, mask);   // in the parameter's type, as it will be added
 #pragma unroll
     for (int t = 0; t < 4; ++t)
       if (mask & (1 << t)) u2 = fmaf(u[t], u[t], u2);

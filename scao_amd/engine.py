@@ -51,13 +51,6 @@ def _align4(n: int) -> int:
     return (n + 3) & ~3
 
 
-def _aligned16(*ptrs) -> bool:
-    x = 0
-    for p in ptrs:
-        x |= p
-    return x & 15 == 0
-
-
 def _item_ptrs(it: "PItem") -> tuple:
     """PItem.ptrs: the device addresses a step reads, once per step."""
     st, ms = it.st, it.msrc
@@ -96,7 +89,6 @@ class PItem:
     leaves: list = field(default_factory=list)  # [(leaf, r0, c0)]
     fp32: bool = True            # param and gradient are float32
     half: int = 0                # param and gradient are both bf16 (1) or fp16 (2)
-    aligned: bool = True         # every pointer of the param is 16-byte aligned
     msrc: "MomentSource | None" = None   # filter/noise formed inside the step kernels
     # device addresses, read once per step: p, graw, gmom, filter EMA (0 when
     # absent) and the four moments in _MOMENTS order
@@ -241,8 +233,11 @@ def _flat_chunks(numel: int) -> int:
 
 _LEAF_TASKS = ("dpart", "delta", "lift")   # with proj* and apply*: idx is a block index
 _PROJ_VARIANTS = [0, 2] + [1 | p | w | t for t in (0, 16, 32) for w in (0, 4, 8) for p in (0, 2)]
+# masked tiles, wide, pipelined, strip (k = 256, 128); | 64: 16-bit data
+_APPLY_VARIANTS = [t | v for t in (0, 4, 12, 20, 52, 68, 84, 116) for v in range(4)]
 _TASK_TYPES = (["adam", "dpart", "delta", "lift", "dred", "dapply", "lars"] +
-               [f"proj{v}" for v in sorted({*range(12), *_PROJ_VARIANTS})] + [f"apply{v}" for v in range(64)])
+               [f"proj{v}" for v in sorted({*range(12), *_PROJ_VARIANTS})] +
+               [f"apply{v}" for v in sorted({*range(64), *_APPLY_VARIANTS})])
 
 
 STEP_WIDTHS = (64, 128, 256)   # eigenfactor widths the step kernels are built for
@@ -399,8 +394,10 @@ def _param_tasks(it: PItem, plan: SplitPlan):
                 for d0 in range(0, k, 64):
                     add("lift", (li, i0, d0, -1))
             var = (1 if it.mgrad else 0) | (2 if it.lars else 0)
-            ok = (leaf.use_kronecker and _leaf_vec(it, leaf, r0, c0l) and it.fp32 and it.aligned
-                  and k % 16 == 0)
+            # 16-bit data has wide and strip tiles, but no pipelined ones
+            pipe = k >= PIPE_MIN_RANK and k not in STRIP_RANKS
+            ok = leaf.use_kronecker and (it.fp32 or (it.half and not pipe))
+            typed = 64 if it.half else 0
             m, n, T = leaf.m, leaf.n, L.APPLY_TILE
             if ok and k in STRIP_RANKS:
                 # runs of strip tiles over the interior they tile exactly
@@ -408,7 +405,7 @@ def _param_tasks(it: PItem, plan: SplitPlan):
                 mw, nw = m - m % tr, n - n % sw
                 if not (mw and nw):
                     mw = nw = 0
-                wide = var | 4 | 16 | (32 if k == 128 else 0)
+                wide = var | 4 | 16 | (32 if k == 128 else 0) | typed
                 for i0, j0 in _strip_runs(mw, nw, tr, sw):
                     add(f"apply{wide}", (li, i0, j0, slot))
                     slot += min(L.APPLY_GROUP, (mw - i0) // tr)
@@ -420,8 +417,8 @@ def _param_tasks(it: PItem, plan: SplitPlan):
                 nw = n - n % L.APPLY_WIDE_COLS if ok else 0
                 if not (mw and nw):
                     mw = nw = 0
-                wide = var | 4 | (8 if k >= PIPE_MIN_RANK else 0)
-                for i0, j0 in _wide_tiles(mw, nw, k, k >= PIPE_MIN_RANK):
+                wide = var | 4 | (8 if pipe else typed)
+                for i0, j0 in _wide_tiles(mw, nw, k, pipe):
                     add(f"apply{wide}", (li, i0, j0, slot))
                     slot += 1
             for i0 in range(0, m, T):
@@ -442,7 +439,7 @@ def _param_tasks(it: PItem, plan: SplitPlan):
 
 def _item_key(it: PItem) -> tuple:
     """Everything _param_tasks reads from an item."""
-    return (id(it.p), it.phase2, it.diag, it.lars, it.mgrad, it.p.numel(), it.fp32, it.aligned,
+    return (id(it.p), it.phase2, it.diag, it.lars, it.mgrad, it.p.numel(), it.fp32,
             _cols(it.p), it.half, tuple((id(lf), r0, c0, _leaf_k(lf)) for lf, r0, c0 in it.leaves)
             if it.phase2 and not it.diag else ())
 
@@ -587,13 +584,6 @@ def _cols(t: Tensor) -> int:
     return math.prod(shape[1:])
 
 
-def _leaf_vec(it: PItem, leaf, r0: int, c0: int) -> bool:
-    """float4 access is legal for the block: 4-aligned origin, row stride and width."""
-    cols = _cols(it.p)
-    return ((r0 * cols + c0) % 4 == 0 and cols % 4 == 0 and leaf.n % 4 == 0
-            and it.aligned)
-
-
 def _padded_factors(leaves, ws: Workspace) -> dict:
     """{leaf index: (U_l, U_r, S_l, S_r)} padded to _leaf_k columns for the
     leaves whose rank is below it: U's extra columns zero, S's extra entries
@@ -677,10 +667,8 @@ def _leaf_table(leaves, items: list[PItem], ws: Workspace):
         e["Wb"] = base + 4 * (off + st + sd + _align4(leaf.m * k)) if k in STRIP_RANKS else 0
         off += st + sd + sw
         e["m"], e["n"], e["k"] = leaf.m, leaf.n, k
-        vec = _leaf_vec(it, leaf, r0, c0) and _aligned16(int(e["T"]))
         parts, _, chunks = _leaf_split(leaf, plan)
-        e["flags"] = ((L.LF_VEC4 if vec else 0) | (parts << L.LF_NSPLIT_SHIFT)
-                      | (chunks << L.LF_DCHUNK_SHIFT))
+        e["flags"] = (parts << L.LF_NSPLIT_SHIFT) | (chunks << L.LF_DCHUNK_SHIFT)
     return tab
 
 
@@ -810,8 +798,6 @@ def _param_table(items: list[PItem], ranges, ws: Workspace, gsnr: float | None):
             flags |= L.PF_DIAG
             diag = it.pre.diag_ema.data_ptr()
             dbias.append((i, getattr(it.pre, "_diag_bias_factor", 1.0)))
-        if it.aligned:
-            flags |= L.PF_ALIGNED
         u8rows.append((pp, gmom or graw, graw, m0, m1, m2, m3, upd, diag, fema, fthr, fseed,
                        seen[5], seen[6]))
         r = ranges[i]
@@ -851,7 +837,7 @@ class StepClass:
     scao_step: int
     lars: bool
     rows: np.ndarray
-    extra_flags: np.ndarray   # per-row flags beyond the group's (alignment, diagonal mode)
+    extra_flags: np.ndarray   # per-row flags beyond the group's (diagonal mode)
 
 
 @dataclass(slots=True)
@@ -896,15 +882,14 @@ def run_step(items: list[PItem], ws: Workspace, update_norm_ema: bool,
         it.fp32 = it.p.dtype == f32 and it.graw.dtype == f32
         it.half = _HALF.get(it.p.dtype, 0) if it.graw.dtype == it.p.dtype else 0
         it.ptrs = _item_ptrs(it)
-        it.aligned = _aligned16(*it.ptrs)
     # the full structure key (with every block's rank) is only rebuilt when
     # the cheap one or the global factor epoch says something may have changed
     ckey = (tuple((id(it.p), it.phase2, it.diag, it.lars, it.mgrad, it.p.numel(),
-                   it.fp32, it.half, it.aligned, len(it.leaves)) for it in items), leaf_epoch())
+                   it.fp32, it.half, len(it.leaves)) for it in items), leaf_epoch())
     skey = ws.struct_key
     if ckey != ws.cheap_key:
         skey = tuple((id(it.p), it.phase2, it.diag, it.lars, it.mgrad, it.p.numel(),
-                      it.fp32, it.half, it.aligned,
+                      it.fp32, it.half,
                       tuple((id(lf), r0, c0, _leaf_k(lf)) for lf, r0, c0 in it.leaves))
                      for it in items)
         ws.cheap_key = ckey
@@ -934,7 +919,7 @@ def run_step(items: list[PItem], ws: Workspace, update_norm_ema: bool,
     if ws.upd_total:
         ws.buf("upd", ws.upd_total * 4)
     # the block table holds no gradient pointer: a gradient that moves keeps
-    # it valid (its alignment is part of the structure key)
+    # it valid
     if ws.leaf_epoch != leaf_epoch() or ws.leaf_dev is None:
         tab = _leaf_table(ws.leaves, items, ws)
         ws.leaf_dev = L.upload(tab, dev) if len(tab) else None
@@ -994,7 +979,7 @@ def _launch_step(ws: Workspace, raw: np.ndarray, n: int, update_norm_ema: bool) 
         _call("scao_diag_reduce", tp("dred"), N["dred"], P, SL, s)
     _call("scao_step_finalize", P, n, SL, S, ws.runtime.data_ptr(), 0,
            1 if update_norm_ema else 0, n, s)
-    for var in range(64):
+    for var in _APPLY_VARIANTS:
         if N[f"apply{var}"]:
             _call("scao_kron_apply", tp(f"apply{var}"), N[f"apply{var}"], LF, P, S, SL, var, s)
     if N["dapply"]:

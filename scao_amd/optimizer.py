@@ -361,7 +361,7 @@ class SCAO(Optimizer):
     def _planned_step(self, ws, host_norms: bool, gsnr) -> bool:
         """The next step of the last plain step's parameters, when nothing
         but the step counters changes: the same parameters (same groups, same
-        order) have gradients, contiguous and with the planned alignment; the
+        order) have contiguous gradients of the planned type; the
         moment tensors and the parameters' storage are the planned ones; no
         refresh is due and no phase changes (a Phase-1 class stays inside its
         warm-up, a Phase-2 class keeps its LARS setting); no filter, noise or
@@ -390,7 +390,7 @@ class SCAO(Optimizer):
                 if it.p is not p or it.group is not g or gr.is_sparse or not gr.is_contiguous():
                     return False
                 ptr = gr.data_ptr()
-                if (it.aligned and ptr & 15) or it.ptrs[0] != p.data_ptr():
+                if it.ptrs[0] != p.data_ptr():
                     return False
                 ptrs.append(ptr)
                 grads.append(gr)
