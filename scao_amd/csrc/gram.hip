@@ -655,6 +655,13 @@ __global__ __launch_bounds__(256) void k_flags_clear(int* flags, int n) {
   if (i < n) flags[i] = 0;
 }
 
+// LDS traffic of one wavefront is ordered; this keeps the compiler from moving
+// its accesses across the point.
+__device__ __forceinline__ void wave_lds_order() {
+  __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
 // Eigenpairs of an exactly diagonal eigh input, one block per factor: the
 // diagonal of X = deq / fp32(bias) + shift as k_eig_prep forms it (the shift
 // from k_eig_trace), ordered by the selection sort above, then flipped to
@@ -662,114 +669,161 @@ __global__ __launch_bounds__(256) void k_flags_clear(int* flags, int n) {
 // Writes w[j] (double) and column j of U (n x kq, row-major) = e_{r_j} for the
 // kq largest, and total = sum of max(d, 0) in double.
 //
-// Each thread owns the positions p = tid (mod 256).  A step scans the owned
-// positions >= i for the first minimum (increasing p, strict <), reduces
-// (value, position) over the block (smaller value, then smaller position: the
-// first position of the minimum), and the owner of the winning position k
-// records it and moves position i's value and index into k.  Position i is
-// never read or written again after step i, and position k is only touched
-// by its owner, so one barrier per step suffices (the reduction slots
-// alternate between two buffers).
-__global__ __launch_bounds__(256) void k_eig_diag(const scao_prep_desc* __restrict__ descs, int dim,
-                                                  int kq, double* __restrict__ w, float* __restrict__ U,
-                                                  int64_t ustride, double* __restrict__ total) {
-  __shared__ float val[DIAG_MAX];
-  __shared__ int idx[DIAG_MAX];
-  __shared__ int top[DIAG_MAX];   // top[j]: row of the unit vector in column j
-  __shared__ float rv[2][4];
-  __shared__ int rp[2][4];
-  __shared__ double red[4];
+// The sort is replayed a group of equal values at a time, not a position at a
+// time.  Once everything smaller is in place, the group's s elements stand at
+// some positions q_0 < q_1 < ... of the rest [a, n), and the sort's steps a, a
+// + 1, ... take them in that order (the first position of the minimum each
+// time; only larger elements move meanwhile).  Step a + j puts the element of
+// q_j at a + j and what stood there, unless it was a member, at q_j; if q_j <
+// a + s, a later step of the group moves that one on, to q_(q_j - a), which is
+// further right.  So each displaced element follows its chain by itself.
+//   * the values are ranked by counting (all 1024 threads), which gives the
+//     groups and the sorted values;
+//   * the first wave goes through the groups: member positions are marked in
+//     a bit mask, whose prefix counts rank them; chains are followed a lane
+//     each.  A group of one takes one exchange.
+// The time is the groups' LDS round trips: a few dozen groups for int8 EMAs
+// (the codes of their diagonals), up to one per row for fp32 EMAs.  2048 rows
+// with some 20 distinct codes (13 factors): 1596 us a step at a time -> 287 us.
+constexpr int ED_T = 1024;
+constexpr int ED_WORDS = (DIAG_MAX + 31) / 32;   // mask words
+
+__global__ __launch_bounds__(ED_T) void k_eig_diag(const scao_prep_desc* __restrict__ descs,
+                                                   int dim, int kq, double* __restrict__ w,
+                                                   float* __restrict__ U, int64_t ustride,
+                                                   double* __restrict__ total) {
+  __shared__ __attribute__((aligned(16))) float val[DIAG_MAX + 4];
+  __shared__ float sv[DIAG_MAX];          // values in ascending order
+  __shared__ uint16_t ord[DIAG_MAX];      // elements by (value, row)
+  __shared__ uint16_t arr[DIAG_MAX];      // element at a position
+  __shared__ uint16_t at[DIAG_MAX];       // position of an element
+  __shared__ uint16_t qs[DIAG_MAX], el[DIAG_MAX];   // a group's positions, its elements there
+  __shared__ uint32_t mask[ED_WORDS];
+  __shared__ int pref[ED_WORDS];
+  __shared__ double red[ED_T / 64];
   const int f = blockIdx.x;
   const scao_prep_desc D = descs[f];
   const int n = D.dim;
   if (n != dim || n < 1 || n > DIAG_MAX || kq > n) return;   // outside the call's contract
-  const int tid = threadIdx.x, lane = tid % 64, wv = tid / 64;
+  const int tid = threadIdx.x, lane = tid % 64;
   const float sf = D.q ? (float)(*D.scale) : 0.f;
   const float eps = *D.shift;
-  double pos = 0.0;
-  for (int i = tid; i < n; i += 256) {
+  double acc[1] = {0.0};
+  bool nan = false;
+  for (int i = tid; i < n; i += ED_T) {
     const float y = prep_val(D, sf, (int64_t)i * n + i) + eps;
     val[i] = y;
-    idx[i] = i;
-    pos += y > 0.f ? (double)y : 0.0;
+    arr[i] = at[i] = (uint16_t)i;
+    nan |= y != y;
+    acc[0] += y > 0.f ? (double)y : 0.0;
   }
-  double acc[1] = {pos};
-  block_sum<1>(acc, red);   // ends with a barrier: val/idx are complete
+  if (tid < 4) val[n + tid] = INFINITY;
+  if (tid < ED_WORDS) mask[tid] = 0u;
+  block_sum_n<1, ED_T>(acc, red);
   if (tid == 0) total[f] = acc[0];
-  double* wf = w + (int64_t)f * kq;
-  for (int i = 0; i + 1 < n; ++i) {
-    // first owned position >= i
-    const int r = i % 256;
-    int p = i - r + tid + (tid < r ? 256 : 0);
-    float bv = INFINITY;
-    int bp = n;
-    if (p < n) {
-      bv = val[p];
-      bp = p;
-      for (p += 256; p < n; p += 256) {
-        const float v = val[p];
-        if (v < bv) {
-          bv = v;
-          bp = p;
-        }
-      }
-    }
+  if (!__syncthreads_or(nan)) {   // a NaN has no order: the rows stay in place
+    // rank of each value: smaller ones, and equal ones of earlier rows
+    for (int i = tid; i < n; i += ED_T) {
+      const float y = val[i];
+      int r = 0;
+      for (int j = 0; j < n; j += 4) {
+        const v4f x = *(const v4f*)&val[j];
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-      const float ov = __shfl_xor(bv, o, 64);
-      const int op = __shfl_xor(bp, o, 64);
-      if (ov < bv || (ov == bv && op < bp)) {
-        bv = ov;
-        bp = op;
+        for (int t = 0; t < 4; ++t) r += x[t] < y || (x[t] == y && j + t < i);
       }
-    }
-    const int b = i & 1;
-    if (lane == 0) {
-      rv[b][wv] = bv;
-      rp[b][wv] = bp;
+      ord[r] = (uint16_t)i;
+      sv[r] = y;
     }
     __syncthreads();
-    float kv = rv[b][0];
-    int k = rp[b][0];
-#pragma unroll
-    for (int q = 1; q < 4; ++q)
-      if (rv[b][q] < kv || (rv[b][q] == kv && rp[b][q] < k)) {
-        kv = rv[b][q];
-        k = rp[b][q];
-      }
-    if (k < i || k >= n) k = i;   // only reachable with NaN values
-    if (k % 256 == tid) {
-      const int j = n - 1 - i;    // column after the flip
-      if (j < kq) {
-        top[j] = idx[k];
-        wf[j] = (double)val[k];
-      }
-      if (k != i) {
-        val[k] = val[i];
-        idx[k] = idx[i];
+    if (tid < 64) {
+      int a = 0;
+      while (a < n) {
+        // 64 sorted values from a: bit t is set when one ends its group
+        const int i = a + lane;
+        const bool end = i >= n - 1 || sv[i] != sv[i + 1];
+        uint64_t ends = __ballot(end);
+        const int mine = i < n ? ord[i] : 0;
+        // the single-element groups up to the first larger one
+        int t = 0;
+        while (t < 64 && a + t < n && ((ends >> t) & 1)) {
+          const int e = __builtin_amdgcn_readlane(mine, t);
+          const int q = at[e], x = arr[a + t];
+          if (q != a + t) {
+            if (lane == 0) {
+              arr[q] = (uint16_t)x;
+              at[x] = (uint16_t)q;
+              arr[a + t] = (uint16_t)e;
+            }
+            wave_lds_order();
+          }
+          ++t;
+        }
+        a += t;
+        if (t == 64 || a >= n) continue;
+        // a group of several: its end, a wave of values at a time
+        int b = a;
+        for (;;) {
+          const int c = b + lane;
+          const uint64_t m = __ballot(c >= n - 1 || sv[c] != sv[c + 1]);
+          if (m) {
+            b += __ffsll((long long)m);
+            break;
+          }
+          b += 64;
+        }
+        for (int c = a + lane; c < b; c += 64) {
+          const int p = at[ord[c]];
+          atomicOr(&mask[p >> 5], 1u << (p & 31));
+        }
+        wave_lds_order();
+        int base = 0;
+        for (int w0 = 0; w0 < ED_WORDS; w0 += 64) {
+          const int wd = w0 + lane;
+          const int cnt = wd < ED_WORDS ? __popc(mask[wd]) : 0;
+          int inc = cnt;
+          for (int o = 1; o < 64; o <<= 1) {
+            const int up = __shfl_up(inc, o);
+            if (lane >= o) inc += up;
+          }
+          if (wd < ED_WORDS) pref[wd] = base + inc - cnt;
+          base += __builtin_amdgcn_readlane(inc, 63);
+        }
+        wave_lds_order();
+        for (int c = a + lane; c < b; c += 64) {
+          const int e = ord[c], p = at[e];
+          const int r = pref[p >> 5] + __popc(mask[p >> 5] & ((1u << (p & 31)) - 1u));
+          qs[r] = (uint16_t)p;
+          el[r] = (uint16_t)e;
+        }
+        wave_lds_order();
+        // displaced elements to the ends of their chains (all at or past b)
+        for (int r = a + lane; r < b; r += 64) {
+          if ((mask[r >> 5] >> (r & 31)) & 1u) continue;
+          const int x = arr[r];
+          int q = qs[r - a];
+          while (q < b) q = qs[q - a];
+          arr[q] = (uint16_t)x;
+          at[x] = (uint16_t)q;
+        }
+        wave_lds_order();
+        for (int r = a + lane; r < b; r += 64) arr[r] = el[r - a];
+        for (int wd = lane; wd < ED_WORDS; wd += 64) mask[wd] = 0u;
+        wave_lds_order();
+        a = b;
       }
     }
-  }
-  if ((n - 1) % 256 == tid) {   // the last position holds the largest value
-    top[0] = idx[n - 1];
-    wf[0] = (double)val[n - 1];
   }
   __syncthreads();
+  double* wf = w + (int64_t)f * kq;
   float* Uf = U + (int64_t)f * ustride;
   const int total_e = n * kq;   // <= DIAG_MAX^2
-  if (kq % 4 == 0 && ((uintptr_t)Uf & 15) == 0) {
-    for (int e = 4 * tid; e < total_e; e += 4 * 256) {
-      const int row = e / kq, j = e - row * kq;
-      v4f x;
-#pragma unroll
-      for (int t = 0; t < 4; ++t) x[t] = top[j + t] == row ? 1.f : 0.f;
-      gst4(Uf + e, x);
-    }
-  } else {
-    for (int e = tid; e < total_e; e += 256) {
-      const int row = e / kq, j = e - row * kq;
-      Uf[e] = top[j] == row ? 1.f : 0.f;
-    }
+  for (int e = 4 * tid; e + 4 <= total_e; e += 4 * ED_T) gst4(Uf + e, v4f{0.f, 0.f, 0.f, 0.f});
+  if (tid < total_e % 4) Uf[total_e - 1 - tid] = 0.f;
+  __syncthreads();   // the zeros are in place before the ones
+  for (int j = tid; j < kq; j += ED_T) {
+    const int r = arr[n - 1 - j];   // column j after the flip
+    wf[j] = (double)val[r];
+    Uf[(int64_t)r * kq + j] = 1.f;
   }
 }
 
@@ -861,7 +915,7 @@ extern "C" int scao_eig_diag(const scao_prep_desc* descs, int ndescs, int n, int
                  "scao_eig_diag: bad arguments n=%d kq=%d", n, kq);
   hipStream_t s = (hipStream_t)stream;
   hipLaunchKernelGGL(k_eig_trace, dim3(ndescs), dim3(256), 0, s, descs);
-  hipLaunchKernelGGL(k_eig_diag, dim3(ndescs), dim3(256), 0, s, descs, n, kq, w, U, ustride, total);
+  hipLaunchKernelGGL(k_eig_diag, dim3(ndescs), dim3(ED_T), 0, s, descs, n, kq, w, U, ustride, total);
   SCAO_LAUNCH_CHECK("scao_eig_diag");
   return SCAO_OK;
 }
