@@ -1213,143 +1213,49 @@ __global__ __launch_bounds__(SB_W * 64) void k_sb2st(double* band, int n, double
 }
 
 // ------------------------------------------------------------- bisection ---
-// Sturm count of T - x: the number of eigenvalues below x (float64, with
-// LAPACK's pivmin guard against a zero pivot).
-// Number of eigenvalues of T below x (float64 Sturm count with dstebz's
-// pivmin guard); e2[i] = e[i]^2.  The coefficients stream in groups of SG,
-// the next group's loads issued before the current group's steps, so their
-// latency hides under the division chain (the addresses are uniform: scalar
-// loads).
+// Sturm counts: the number of eigenvalues of the tridiagonal T below x, as
+// sign changes of the leading minors' recurrence
+//   p_i = (d_i - x) p_{i-1} - e_{i-1}^2 p_{i-2}
+// (Givens; Barth, Martin and Wilkinson 1967), in float64, rescaled by a power
+// of two every four steps: two dependent operations a step, where the ratio
+// form q_i = p_i / p_{i-1} has a division.  The computed minors are those of a
+// matrix within a few ulps of T elementwise, as the ratios are.  A minor that
+// comes out zero takes the sign opposite to its predecessor and a size far
+// below it (2^-200), so a decoupled block (e = 0) goes on counting from it;
+// four steps of that stay far above underflow.  e2[i] = e[i]^2.  The
+// coefficients stream in groups of SG, the next group's loads issued before
+// the current group's steps (the addresses are uniform: scalar loads).
 constexpr int SG = 8;
-__device__ __forceinline__ int sturm(const double* __restrict__ d, const double* __restrict__ e2,
-                                     int n, double x, double pivmin) {
-  int c = 0;
-  double qv = d[0] - x;
-  if (fabs(qv) < pivmin) qv = -pivmin;
-  c += qv < 0.0;
-  int i = 1;
-  if (n - 1 >= SG) {
-    double dn[SG], en[SG];
-#pragma unroll
-    for (int t = 0; t < SG; ++t) {
-      dn[t] = d[1 + t];
-      en[t] = e2[t];
-    }
-    for (; i + SG <= n; i += SG) {
-      double dc[SG], ec[SG];
-#pragma unroll
-      for (int t = 0; t < SG; ++t) {
-        dc[t] = dn[t];
-        ec[t] = en[t];
-      }
-      if (i + 2 * SG <= n) {
-#pragma unroll
-        for (int t = 0; t < SG; ++t) {
-          dn[t] = d[i + SG + t];
-          en[t] = e2[i + SG - 1 + t];
-        }
-      }
-#pragma unroll
-      for (int t = 0; t < SG; ++t) {
-        qv = (dc[t] - x) - ec[t] / qv;
-        if (fabs(qv) < pivmin) qv = -pivmin;
-        c += qv < 0.0;
-      }
-    }
-  }
-  for (; i < n; ++i) {
-    qv = (d[i] - x) - e2[i - 1] / qv;
-    if (fabs(qv) < pivmin) qv = -pivmin;
-    c += qv < 0.0;
-  }
-  return c;
-}
+constexpr double STURM_TINY = 0x1p-200;
 
-// Per matrix: Gershgorin bounds, pivmin, the trace (float64), the number of
-// negative eigenvalues.  info = {lo, hi, pivmin, trace}, nneg.
-__global__ __launch_bounds__(256) void k_tri_info(const double* d, const double* e, int n,
-                                                  double* info, int* nneg, double* e2) {
-  __shared__ double red[16];
-  const int mat = blockIdx.x;
-  const double* dm = d + (int64_t)mat * n;
-  const double* em = e + (int64_t)mat * n;
-  double* e2m = e2 + (int64_t)mat * n;
-  double lo = 1e300, hi = -1e300, tr = 0.0, e2max = 0.0;
-  for (int i = threadIdx.x; i < n; i += 256) {
-    const double r = (i > 0 ? fabs(em[i - 1]) : 0.0) + (i + 1 < n ? fabs(em[i]) : 0.0);
-    lo = fmin(lo, dm[i] - r);
-    hi = fmax(hi, dm[i] + r);
-    tr += dm[i];
-    if (i + 1 < n) {
-      e2m[i] = em[i] * em[i];
-      e2max = fmax(e2max, e2m[i]);
-    }
-  }
-  double x[2] = {tr, 0.0};
-  block_sum<2>(x, red);
-  // min / max / max through the same LDS, one at a time
-  __shared__ double mm[3][256];
-  mm[0][threadIdx.x] = lo;
-  mm[1][threadIdx.x] = hi;
-  mm[2][threadIdx.x] = e2max;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    for (int t = 1; t < 256; ++t) {
-      lo = fmin(lo, mm[0][t]);
-      hi = fmax(hi, mm[1][t]);
-      e2max = fmax(e2max, mm[2][t]);
-    }
-    const double tnorm = fmax(fabs(lo), fabs(hi));
-    const double pivmin = 2.2250738585072014e-308 * fmax(1.0, e2max);
-    // widen the interval so bisection brackets every eigenvalue
-    const double pad = 2.0 * 2.220446049250313e-16 * tnorm * n + 2.0 * pivmin;
-    info[4 * mat + 0] = lo - pad;
-    info[4 * mat + 1] = hi + pad;
-    info[4 * mat + 2] = pivmin;
-    info[4 * mat + 3] = x[0];
-    nneg[mat] = sturm(dm, e2m, n, 0.0, pivmin);
-  }
-}
-
-// Multisection.  BL lanes share one eigenvalue index and each runs BS Sturm
-// counts at once, so an iteration evaluates BP = BL * BS points and shrinks
-// the bracket (BP + 1) times (about 13 iterations to fp64 resolution against
-// 53 halvings).  The counts' divisions are reciprocals (v_rcp_f64 and two
-// Newton steps, no condition-register chain as in IEEE division), so a lane's
-// BS counts interleave.  A quotient with a few ulps of error is a relative
-// perturbation of the matrix of that size, as the rounding of the divisions
-// already is (dstebz's analysis), so counts and brackets stay those of a
-// matrix within a few ulps of T.
-constexpr int BL = 4;
-constexpr int BS = 4;
-constexpr int BP = BL * BS;
-
-__device__ __forceinline__ double recip(double q) {
-  double r = __builtin_amdgcn_rcp(q);
-  double t = fma(-q, r, 1.0);
-  r = fma(r, t, r);
-  t = fma(-q, r, 1.0);
-  return fma(r, t, r);
-}
-
-// Sturm counts of T - x[t] for S points at once (as sturm above).
 template <int S>
 __device__ __forceinline__ void sturm_ms(const double* __restrict__ d,
                                          const double* __restrict__ e2, int n,
-                                         const double (&x)[S], double pivmin, int (&c)[S]) {
-  double q[S];
+                                         const double (&x)[S], int (&c)[S]) {
+  double p[S], pm[S];
 #pragma unroll
   for (int t = 0; t < S; ++t) {
-    q[t] = d[0] - x[t];
-    if (fabs(q[t]) < pivmin) q[t] = -pivmin;
-    c[t] = q[t] < 0.0;
+    pm[t] = 1.0;
+    p[t] = d[0] - x[t];
+    if (p[t] == 0.0) p[t] = -STURM_TINY;
+    c[t] = p[t] < 0.0;
   }
   auto step = [&](double dv, double ev) {
 #pragma unroll
     for (int t = 0; t < S; ++t) {
-      q[t] = fma(-ev, recip(q[t]), dv - x[t]);
-      if (fabs(q[t]) < pivmin) q[t] = -pivmin;
-      c[t] += q[t] < 0.0;
+      double q = fma(dv - x[t], p[t], -(ev * pm[t]));
+      if (__builtin_expect(q == 0.0, 0)) q = -STURM_TINY * p[t];
+      c[t] += (int)((uint32_t)(__double2hiint(q) ^ __double2hiint(p[t])) >> 31);
+      pm[t] = p[t];
+      p[t] = q;
+    }
+  };
+  auto rescale = [&]() {
+#pragma unroll
+    for (int t = 0; t < S; ++t) {
+      const int ex = max(__builtin_amdgcn_frexp_exp(p[t]), __builtin_amdgcn_frexp_exp(pm[t]));
+      p[t] = ldexp(p[t], -ex);
+      pm[t] = ldexp(pm[t], -ex);
     }
   };
   int i = 1;
@@ -1375,24 +1281,134 @@ __device__ __forceinline__ void sturm_ms(const double* __restrict__ d,
         }
       }
 #pragma unroll
-      for (int t = 0; t < SG; ++t) step(dc[t], ec[t]);
+      for (int t = 0; t < SG; ++t) {
+        step(dc[t], ec[t]);
+        if (t % 4 == 3) rescale();
+      }
     }
   }
-  for (; i < n; ++i) step(d[i], e2[i - 1]);
+  for (; i < n; ++i) {
+    step(d[i], e2[i - 1]);
+    rescale();
+  }
 }
 
-// The eigenvalues wanted per matrix: the kq largest (indices n-1 .. n-kq),
-// and the negative ones not among them (indices 0 .. nneg-1), which only
-// enter the sum of the clamped spectrum.  Waves 0 .. WT-1 of a matrix serve
-// the largest, 64 / BL per wave by multisection; the rest the negative ones,
-// NB2 per lane by bisection (interleaved counts, one point each: with many
-// eigenvalues to find, the halving that needs the fewest counts is
-// cheapest), bracketed by [lo, 0] and stopped at an absolute width of
-// 1e-12 |T| (at most 1e-12 |T| n off in the sum; the largest are resolved
-// to a few ulps of themselves).  The matrix is blockIdx.x: workgroups go to
-// the XCDs round-robin by linear index, and with the matrix index slowest
-// every block with work would land on one XCD.
-constexpr int NB2 = 2;
+// Per matrix: Gershgorin bounds, pivmin, the trace (float64), the number of
+// negative eigenvalues.  info = {lo, hi, pivmin, trace}, nneg.
+__global__ __launch_bounds__(256) void k_tri_info(const double* d, const double* e, int n,
+                                                  double* info, int* nneg, double* e2) {
+  __shared__ double red[16];
+  const int mat = blockIdx.x;
+  const double* dm = d + (int64_t)mat * n;
+  const double* em = e + (int64_t)mat * n;
+  double* e2m = e2 + (int64_t)mat * n;
+  double lo = 1e300, hi = -1e300, tr = 0.0, e2max = 0.0;
+  for (int i = threadIdx.x; i < n; i += 256) {
+    const double r = (i > 0 ? fabs(em[i - 1]) : 0.0) + (i + 1 < n ? fabs(em[i]) : 0.0);
+    lo = fmin(lo, dm[i] - r);
+    hi = fmax(hi, dm[i] + r);
+    tr += dm[i];
+    if (i + 1 < n) {
+      e2m[i] = em[i] * em[i];
+      e2max = fmax(e2max, e2m[i]);
+    }
+  }
+  double x[2] = {tr, 0.0};
+  block_sum<2>(x, red);
+  // min / max / max: within each wave, then the four waves' through LDS
+  __shared__ double mm[3][4];
+  for (int o = 32; o > 0; o >>= 1) {
+    lo = fmin(lo, __shfl_xor(lo, o));
+    hi = fmax(hi, __shfl_xor(hi, o));
+    e2max = fmax(e2max, __shfl_xor(e2max, o));
+  }
+  if (threadIdx.x % 64 == 0) {
+    mm[0][threadIdx.x / 64] = lo;
+    mm[1][threadIdx.x / 64] = hi;
+    mm[2][threadIdx.x / 64] = e2max;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int t = 1; t < 4; ++t) {
+      lo = fmin(lo, mm[0][t]);
+      hi = fmax(hi, mm[1][t]);
+      e2max = fmax(e2max, mm[2][t]);
+    }
+    const double tnorm = fmax(fabs(lo), fabs(hi));
+    const double pivmin = 2.2250738585072014e-308 * fmax(1.0, e2max);
+    // widen the interval so bisection brackets every eigenvalue
+    const double pad = 2.0 * 2.220446049250313e-16 * tnorm * n + 2.0 * pivmin;
+    info[4 * mat + 0] = lo - pad;
+    info[4 * mat + 1] = hi + pad;
+    info[4 * mat + 2] = pivmin;
+    info[4 * mat + 3] = x[0];
+    const double zero[1] = {0.0};
+    int c[1];
+    sturm_ms<1>(dm, e2m, n, zero, c);
+    nneg[mat] = c[0];
+  }
+}
+
+// Multisection.  The eigenvalues wanted per matrix: the kq largest (indices
+// n-1 .. n-kq), resolved to a few ulps of themselves, and the negative ones
+// not among them (indices 0 .. nneg-1), which only enter the sum of the
+// clamped spectrum, bracketed by [lo, 0] and stopped at an absolute width of
+// 1e-12 |T| (at most 1e-12 |T| n off in the sum).  A group of lanes shares one
+// eigenvalue; each lane runs some Sturm counts at once, and with P points in
+// all an iteration shrinks the bracket P + 1 times.
+//
+// A count is a chain of n steps, and with a point per lane the chain's
+// latency, not its issue, is the time.  So few matrices take many lanes per
+// eigenvalue, a point each (TL = 16: 13 iterations for the largest, NL = 8:
+// 13 for the negative ones).  A batch that fills the chip is bound by issue
+// and takes the fewest counts: four lanes of four points (the largest are few)
+// and plain halving, two eigenvalues to a lane, for the negative ones.
+// 13 matrices of 2048 rows, with negative eigenvalues from int8 EMAs: 6.6 -> 1.5
+// ms.  The matrix is blockIdx.x: workgroups go to the XCDs round-robin by
+// linear index, and with the matrix index slowest every block with work would
+// land on one XCD.
+constexpr int NB2 = 2;   // halving: eigenvalues per lane
+
+// waves for `count` eigenvalues at L lanes each (L = 1: NB2 per lane)
+__host__ __device__ constexpr int bisect_waves(int count, int lanes) {
+  return lanes == 1 ? (count + 64 * NB2 - 1) / (64 * NB2) : (count * lanes + 63) / 64;
+}
+
+// One eigenvalue (index j) per group of LN lanes, PT points per lane, from
+// [lo, hi] until the width is at most rel * max(|lo|, |hi|) + tol.
+template <int LN, int PT>
+__device__ __forceinline__ double multisect(const double* dm, const double* em, int n, int j,
+                                            double lo, double hi, double rel, double tol,
+                                            bool done) {
+  constexpr int PTS = LN * PT;
+  const int sub = (int)threadIdx.x % LN;
+  for (int it = 0; it < 64; ++it) {
+    if (hi - lo <= rel * fmax(fabs(lo), fabs(hi)) + tol) done = true;
+    if (__all(done)) break;
+    // points lo + h * (p + 1), p = 0 .. PTS-1; this lane's are p = sub * PT + t
+    const double h = (hi - lo) / (PTS + 1);
+    double x[PT];
+#pragma unroll
+    for (int t = 0; t < PT; ++t) x[t] = lo + h * (double)(sub * PT + t + 1);
+    int c[PT];
+    sturm_ms<PT>(dm, em, n, x, c);
+    // r = number of points whose count is <= j (a prefix: counts grow with x)
+    int r = 0;
+#pragma unroll
+    for (int t = 0; t < PT; ++t) r += c[t] <= j;
+#pragma unroll
+    for (int o = 1; o < LN; o <<= 1) r += __shfl_xor(r, o);
+    if (!done) {
+      const double nlo = r > 0 ? lo + h * (double)r : lo;
+      const double nhi = r < PTS ? lo + h * (double)(r + 1) : hi;
+      lo = nlo;
+      hi = nhi;
+    }
+  }
+  return 0.5 * (lo + hi);
+}
+
+template <int TL, int TS, int NL>
 __global__ __launch_bounds__(256) void k_bisect(const double* d, const double* e2, int n, int kq,
                                                 const double* info, const int* nneg,
                                                 double* wall) {
@@ -1401,98 +1417,82 @@ __global__ __launch_bounds__(256) void k_bisect(const double* d, const double* e
   const int l = threadIdx.x % 64;
   const int neg = nneg[mat];
   const int nn = neg < n - kq ? neg : n - kq;   // negative ones to find
-  const int wt = (kq + 64 / BL - 1) / (64 / BL);
+  const int wt = bisect_waves(kq, TL);
   const double* dm = d + (int64_t)mat * n;
   const double* em = e2 + (int64_t)mat * n;
+  double* wm = wall + (int64_t)mat * n;
   const double lo0 = info[4 * mat + 0], hi0 = info[4 * mat + 1];
   const double pivmin = info[4 * mat + 2];
   if (wv < wt) {
-    const int sub = l % BL;
-    const int slot = wv * (64 / BL) + l / BL;
+    const int slot = wv * (64 / TL) + l / TL;
     const bool act = slot < kq;
     const int j = n - 1 - (act ? slot : 0);
-    double lo = lo0, hi = hi0;
-    bool done = !act;
-    for (int it = 0; it < 40; ++it) {
-      if (hi - lo <= 2.0 * 2.220446049250313e-16 * fmax(fabs(lo), fabs(hi)) + pivmin) done = true;
-      if (__all(done)) break;
-      // points lo + h * (p + 1), p = 0 .. BP-1; this lane's are p = sub * BS + t
-      const double h = (hi - lo) / (BP + 1);
-      double x[BS];
-#pragma unroll
-      for (int t = 0; t < BS; ++t) x[t] = lo + h * (double)(sub * BS + t + 1);
-      int c[BS];
-      sturm_ms<BS>(dm, em, n, x, pivmin, c);
-      // r = number of points whose count is <= j (a prefix: counts grow with x)
-      int r = 0;
-#pragma unroll
-      for (int t = 0; t < BS; ++t) r += c[t] <= j;
-      r += __shfl_xor(r, 1);
-      r += __shfl_xor(r, 2);
-      if (!done) {
-        const double nlo = r > 0 ? lo + h * (double)r : lo;
-        const double nhi = r < BP ? lo + h * (double)(r + 1) : hi;
-        lo = nlo;
-        hi = nhi;
-      }
-    }
-    if (act && sub == 0) wall[(int64_t)mat * n + j] = 0.5 * (lo + hi);
+    const double x = multisect<TL, TS>(dm, em, n, j, lo0, hi0, 2.0 * 2.220446049250313e-16,
+                                       pivmin, !act);
+    if (act && l % TL == 0) wm[j] = x;
     return;
   }
-  const int base = (wv - wt) * 64 * NB2;
-  if (base >= nn) return;                 // the whole wavefront
   const double tol = 1e-12 * fmax(fabs(lo0), fabs(hi0)) + pivmin;
-  int j[NB2];
-  bool done[NB2];
-  double lo[NB2], hi[NB2];
-#pragma unroll
-  for (int t = 0; t < NB2; ++t) {
-    j[t] = base + l + 64 * t;
-    done[t] = j[t] >= nn;
-    lo[t] = lo0;
-    hi[t] = 0.0;
-  }
-  for (int it = 0; it < 64; ++it) {
-    bool all = true;
+  if constexpr (NL > 1) {
+    const int base = (wv - wt) * (64 / NL);
+    if (base >= nn) return;                 // the whole wavefront
+    const int j = base + l / NL;
+    const double x = multisect<NL, 1>(dm, em, n, j, lo0, 0.0, 0.0, tol, j >= nn);
+    if (j < nn && l % NL == 0) wm[j] = x;
+  } else {
+    const int base = (wv - wt) * 64 * NB2;
+    if (base >= nn) return;                 // the whole wavefront
+    int j[NB2];
+    bool done[NB2];
+    double lo[NB2], hi[NB2];
 #pragma unroll
     for (int t = 0; t < NB2; ++t) {
-      if (hi[t] - lo[t] <= tol) done[t] = true;
-      all = all && done[t];
+      j[t] = base + l + 64 * t;
+      done[t] = j[t] >= nn;
+      lo[t] = lo0;
+      hi[t] = 0.0;
     }
-    if (__all(all)) break;
-    double x[NB2];
+    for (int it = 0; it < 64; ++it) {
+      bool all = true;
 #pragma unroll
-    for (int t = 0; t < NB2; ++t) x[t] = 0.5 * (lo[t] + hi[t]);
-    int c[NB2];
-    sturm_ms<NB2>(dm, em, n, x, pivmin, c);
+      for (int t = 0; t < NB2; ++t) {
+        if (hi[t] - lo[t] <= tol) done[t] = true;
+        all = all && done[t];
+      }
+      if (__all(all)) break;
+      double x[NB2];
+#pragma unroll
+      for (int t = 0; t < NB2; ++t) x[t] = 0.5 * (lo[t] + hi[t]);
+      int c[NB2];
+      sturm_ms<NB2>(dm, em, n, x, c);
+#pragma unroll
+      for (int t = 0; t < NB2; ++t)
+        if (!done[t]) {
+          if (c[t] > j[t])
+            hi[t] = x[t];
+          else
+            lo[t] = x[t];
+        }
+    }
 #pragma unroll
     for (int t = 0; t < NB2; ++t)
-      if (!done[t]) {
-        if (c[t] > j[t])
-          hi[t] = x[t];
-        else
-          lo[t] = x[t];
-      }
+      if (j[t] < nn) wm[j[t]] = 0.5 * (lo[t] + hi[t]);
   }
-#pragma unroll
-  for (int t = 0; t < NB2; ++t)
-    if (j[t] < nn) wall[(int64_t)mat * n + j[t]] = 0.5 * (lo[t] + hi[t]);
 }
 
 // The kq largest, descending, and total = trace - sum of the negative ones
-// (summed in ascending order, fixed), i.e. the sum of the clamped spectrum.
+// (summed in a fixed order), i.e. the sum of the clamped spectrum.
 __global__ __launch_bounds__(64) void k_bisect_finish(const double* wall, int n, int kq,
                                                       const double* info, const int* nneg,
                                                       double* w, double* total) {
   const int mat = blockIdx.x;
   const double* wm = wall + (int64_t)mat * n;
   for (int i = threadIdx.x; i < kq; i += 64) w[(int64_t)mat * kq + i] = wm[n - 1 - i];
-  if (threadIdx.x == 0) {
-    double s = 0.0;
-    const int neg = nneg[mat];
-    for (int j = 0; j < neg; ++j) s += wm[j];
-    total[mat] = info[4 * mat + 3] - s;
-  }
+  double s = 0.0;
+  const int neg = nneg[mat];
+  for (int j = threadIdx.x; j < neg; j += 64) s += wm[j];
+  s = wave_sum(s);
+  if (threadIdx.x == 0) total[mat] = info[4 * mat + 3] - s;
 }
 
 // ------------------------------------------------------ inverse iteration ---
@@ -2353,11 +2353,18 @@ extern "C" int scao_eig_bisect(const double* d, const double* e, int n, int batc
   double* e2 = info + 5 * (int64_t)batch;     // after nneg's batch 8-byte slots
   hipLaunchKernelGGL(k_tri_info, dim3(batch), dim3(256), 0, s, d, e, n, info, nneg, e2);
   SCAO_LAUNCH_CHECK("scao_eig_bisect/info");
-  // wavefronts for the kq largest (64 / BL each) and for up to n - kq
-  // negative ones (64 * NB2 each)
-  const int nwave = (kq + 64 / BL - 1) / (64 / BL) + (n - kq + 64 * NB2 - 1) / (64 * NB2);
-  hipLaunchKernelGGL(k_bisect, dim3(batch, (nwave + 3) / 4), dim3(256), 0, s, d, e2, n, kq, info,
-                     nneg, wall);
+  // few matrices: many lanes per eigenvalue (k_bisect); 8 n / 64 waves for the
+  // negative ones and kq / 4 for the largest leave a SIMD about one wave each
+  // up to some 16 matrices of 2048 rows
+  if ((int64_t)batch * n <= 64 * 1024) {
+    const int nwave = bisect_waves(kq, 16) + bisect_waves(n - kq, 8);
+    hipLaunchKernelGGL((k_bisect<16, 1, 8>), dim3(batch, (nwave + 3) / 4), dim3(256), 0, s, d, e2,
+                       n, kq, info, nneg, wall);
+  } else {
+    const int nwave = bisect_waves(kq, 4) + bisect_waves(n - kq, 1);
+    hipLaunchKernelGGL((k_bisect<4, 4, 1>), dim3(batch, (nwave + 3) / 4), dim3(256), 0, s, d, e2,
+                       n, kq, info, nneg, wall);
+  }
   SCAO_LAUNCH_CHECK("scao_eig_bisect/bisect");
   hipLaunchKernelGGL(k_bisect_finish, dim3(batch), dim3(64), 0, s, wall, n, kq, info, nneg, w,
                      total);
