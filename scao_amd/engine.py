@@ -1331,7 +1331,8 @@ def _refresh_kron(kron, dev, s, eigen_only=False, ema_only=False):
     for leaf, *_ in kron:
         jobs.setdefault(leaf.m, []).append((leaf, 0))
         jobs.setdefault(leaf.n, []).append((leaf, 1))
-    spectra = {}   # (id(leaf), side) -> (S_desc, U_desc, total)
+    spectra = {}   # (id(leaf), side) -> (S_desc, U_desc)
+    parts = []     # (factors, dim, kq, eigenvalues in float64, total) per batch
     LAST_REFRESH_ROUTES.clear()
     eig_timer = _mark("refresh:eigh+rank")
     eig_timer.__enter__()
@@ -1341,12 +1342,7 @@ def _refresh_kron(kron, dev, s, eigen_only=False, ema_only=False):
     # few small factors leaves most of the GPU idle, and its latency-bound
     # kernels fit beside the large batch's.
     main = torch.cuda.current_stream(dev)
-    # a batch's transient buffers (the stacked inputs, the band copies, the
-    # eigenvector workspace) come to about twice its inputs: keep the inputs
-    # to a quarter of what is free (the caching allocator's idle blocks count)
-    free = torch.cuda.mem_get_info(dev)[0] + (torch.cuda.memory_reserved(dev) -
-                                               torch.cuda.memory_allocated(dev))
-    hip_budget = min(EIGEN_BATCH_BYTES, free // EIGEN_BATCH_FREE_FRACTION)
+    hip_budget = None
     order = sorted(jobs.items(), key=lambda kv: len(kv[1]) * kv[0] ** 2)
     side = _side_stream(dev) if len(order) > 1 else None
     if side is not None:
@@ -1363,6 +1359,14 @@ def _refresh_kron(kron, dev, s, eigen_only=False, ema_only=False):
                 routes.setdefault(r, []).append(key)
             if "hip" in routes and batch_route("hip", dim, len(routes["hip"])) == "library":
                 routes.setdefault("library", []).extend(routes.pop("hip"))
+            if "hip" in routes and hip_budget is None:
+                # a batch's transient buffers (the stacked inputs, the band
+                # copies, the eigenvector workspace) come to about twice its
+                # inputs: keep the inputs to a quarter of what is free (the
+                # caching allocator's idle blocks count)
+                free = torch.cuda.mem_get_info(dev)[0] + (torch.cuda.memory_reserved(dev) -
+                                                           torch.cuda.memory_allocated(dev))
+                hip_budget = min(EIGEN_BATCH_BYTES, free // EIGEN_BATCH_FREE_FRACTION)
             for r, keys in routes.items():
                 LAST_REFRESH_ROUTES[r] = LAST_REFRESH_ROUTES.get(r, 0) + len(keys)
             for route, keys in routes.items():
@@ -1385,35 +1389,32 @@ def _refresh_kron(kron, dev, s, eigen_only=False, ema_only=False):
                         S_desc = w.flip(-1).clamp(min=0.0)[:, :kq].contiguous()
                         U_desc = V.flip(-1)[:, :, :kq].contiguous()
                         total = w.clamp(min=0.0).sum(dim=1).double()
+                        w = S_desc.double()
                         del X, V
                     if strm is not main:   # used on the current stream from here on
-                        for t in (S_desc, U_desc, total):
+                        for t in (w, S_desc, U_desc, total):
                             t.record_stream(main)
-                    for (leaf, side_), Sd, Ud, tot in zip(part, S_desc, U_desc, total):
-                        spectra[(id(leaf), side_)] = (Sd, Ud, tot)
+                    parts.append((part, dim, kq, w, total))
+                    for (leaf, side_), Sd, Ud in zip(part, S_desc, U_desc):
+                        spectra[(id(leaf), side_)] = (Sd, Ud)
     if side is not None:
         main.wait_stream(side)
-    # 3) adaptive rank for every (leaf, side) in one device pass + one read
-    keys = [(leaf, side) for leaf, *_ in kron for side in (0, 1)]
+    # 3) adaptive rank: one read of every spectrum, the choice on the host (a
+    # few dozen small device operations per dimension took 0.6 ms of launches)
     ranks = {}
-    by_dim = {}
-    for leaf, side in keys:
-        dim = leaf.m if side == 0 else leaf.n
-        by_dim.setdefault(dim, []).append((leaf, side))
-    dev_ranks = []
-    for dim, lst in by_dim.items():
-        S = torch.stack([spectra[(id(lf), sd)][0] for lf, sd in lst])
-        eps = torch.tensor([lf.epsilon_sparse for lf, _ in lst], device=dev, dtype=torch.float64)
-        kmin = torch.tensor([lf.k_min for lf, _ in lst], device=dev, dtype=torch.int64)
-        kmax = torch.tensor([lf.k_max for lf, _ in lst], device=dev, dtype=torch.int64)
-        tot = torch.stack([spectra[(id(lf), sd)][2] for lf, sd in lst])
-        dev_ranks.append((lst, batched_adaptive_rank_topk(S, tot, dim, eps, kmin, kmax)))
-    host = torch.cat([r for _, r in dev_ranks]).cpu().tolist() if dev_ranks else []
-    i = 0
-    for lst, _ in dev_ranks:
-        for key in lst:
-            ranks[(id(key[0]), key[1])] = int(host[i])
-            i += 1
+    if parts:
+        host = torch.cat([x.reshape(-1) for *_, w, tot in parts for x in (w, tot)]).cpu()
+    off = 0
+    for part, dim, kq, _, _ in parts:
+        n = len(part)
+        w, tot = host[off:off + n * kq].reshape(n, kq), host[off + n * kq:off + n * (kq + 1)]
+        off += n * (kq + 1)
+        ks = batched_adaptive_rank_topk(
+            w.clamp(min=0.0).float(), tot, dim,
+            torch.tensor([lf.epsilon_sparse for lf, _ in part], dtype=torch.float64),
+            torch.tensor([lf.k_min for lf, _ in part]), torch.tensor([lf.k_max for lf, _ in part]))
+        for (leaf, side_), k in zip(part, ks.tolist()):
+            ranks[(id(leaf), side_)] = k
     eig_timer.__exit__(None, None, None)
     # 4) rank momentum and truncation (reference :437-451)
     for leaf, *_ in kron:
@@ -1422,8 +1423,8 @@ def _refresh_kron(kron, dev, s, eigen_only=False, ema_only=False):
         k = min(k, leaf._k + 4)
         k = int(min(leaf.k_max, max(leaf.k_min, k)))
         leaf._k = k
-        Sl, Ul, _ = spectra[(id(leaf), 0)]
-        Sr, Ur, _ = spectra[(id(leaf), 1)]
+        Sl, Ul = spectra[(id(leaf), 0)]
+        Sr, Ur = spectra[(id(leaf), 1)]
         leaf.U_l = Ul[:, :k].contiguous()
         leaf.S_l = Sl[:k].contiguous()
         leaf.U_r = Ur[:, :k].contiguous()
