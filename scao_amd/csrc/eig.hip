@@ -111,27 +111,37 @@ __device__ __forceinline__ double wave_sum_d(double y) {
 }
 
 // ------------------------------------------------------------ panel QR ---
-// Block reduction of NV floats over a workgroup of up to 1024 threads: every thread
-// receives the NV sums in out[] (LDS).  (A reduce-scatter across the wave's
-// lanes, 28 shuffles for 16 values instead of 96, measured slower: its
-// lane-dependent selects cost more than the shuffles they save.)
-template <int NV>
-__device__ __forceinline__ void block_sum_f(float (&x)[NV], float (*red)[NV + 1], float* out) {
-  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+// Sums of 16 values over the wavefront, spread over its four 16-lane rows: on
+// return x[q] (q < 4) holds, in every lane of row (hi, lo), the sum of value
+// q + 4 lo + 8 hi.  A permlane swap of two different registers puts one
+// value's halves in the lower half of the lanes and the other's in the upper,
+// so each level halves the registers: 8 + 4 swaps and adds, then four levels
+// within the rows on the four that remain (28 adds for 16 values; 96 when
+// every lane takes every sum).
+__device__ __forceinline__ void wave_sum16(float (&x)[16]) {
 #pragma unroll
-  for (int v = 0; v < NV; ++v) {
-    x[v] = wave_sum_f(x[v]);
+  for (int q = 0; q < 8; ++q) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x[q]),
+                                                    __float_as_uint(x[q + 8]), false, false);
+    x[q] = __uint_as_float(r[0]) + __uint_as_float(r[1]);
   }
-  if (lane == 0)
 #pragma unroll
-    for (int v = 0; v < NV; ++v) red[wid][v] = x[v];
-  __syncthreads();
-  if (threadIdx.x < NV) {
-    float s = 0.f;
-    for (int w = 0; w < (int)(blockDim.x >> 6); ++w) s += red[w][threadIdx.x];
-    out[threadIdx.x] = s;
+  for (int q = 0; q < 4; ++q) {
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x[q]),
+                                                    __float_as_uint(x[q + 4]), false, false);
+    x[q] = __uint_as_float(r[0]) + __uint_as_float(r[1]);
   }
-  __syncthreads();
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    x[q] += dpp_f<DPP_ROR8>(x[q]);
+    x[q] += dpp_f<DPP_ROR4>(x[q]);
+    x[q] += dpp_f<DPP_XOR2>(x[q]);
+    x[q] += dpp_f<DPP_XOR1>(x[q]);
+  }
+}
+// lane c's float in every lane (c the same in all of them)
+__device__ __forceinline__ float lane_f(float x, int c) {
+  return __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(x), c));
 }
 
 // f(integral_constant<int, J>) for J = 0, 1, .., in order
@@ -148,11 +158,16 @@ __device__ __forceinline__ void static_for(F& f, std::integer_sequence<int, J...
 // each: few waves keep the per-column block reductions cheap and let two
 // workgroups share a CU (480 panels of 2032 rows: 19.7 -> 11.3 ms for a
 // sweep with 256-512 threads of 4 rows instead of 512-1024 of 2).
+// A column is a chain of a block reduction, a square root and two divisions,
+// and 16 of them are the panel's time: the reduction spreads its values over
+// the lanes (wave_sum16), its partial sums wait in LDS for one barrier per
+// column, and every wave adds them and keeps the sums as scalars.  13 panels of
+// up to 2032 rows: 47 -> 32 us.
 template <int RPT, int NT>
 __global__ __launch_bounds__(NT) void k_panel_qr(float* A, int64_t stride, int n, int c0,
                                                    float* Tout, float* band, int64_t bstride) {
-  __shared__ float red[16][NB + 1];
-  __shared__ float bc[NB + 2];
+  constexpr int NW = NT / 64;
+  __shared__ float red[2][NW][NB];   // partial sums, by column parity
   __shared__ float rowj[2][NB];
   __shared__ float Ts[NB][NB];
   __shared__ float betas[NB], taus[NB];
@@ -213,17 +228,30 @@ __global__ __launch_bounds__(NT) void k_panel_qr(float* A, int64_t stride, int n
         for (int c = 0; c < NB; ++c) acc[c] = fmaf(pj, P[h][c], acc[c]);
       }
     }
-    block_sum_f<NB>(acc, red, bc);
-    const float alpha = rj[j], sig2 = bc[j];
+    wave_sum16(acc);
+    const int lane = tid & 63;
+    if ((lane & 15) == 0) {
+      const int c0q = 4 * ((lane >> 4) & 1) + 8 * (lane >> 5);
+#pragma unroll
+      for (int q = 0; q < 4; ++q) red[j & 1][tid >> 6][c0q + q] = acc[q];
+    }
+    __syncthreads();   // the buffers of column j - 1 are not written again before column j + 1
+    // lane c (and c + 16, ..) holds G[c] and row j's entry
+    float gl = 0.f;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) gl += red[j & 1][w][lane & 15];
+    const float rl = rj[lane & 15];
+    const float alpha = lane_f(rl, j), sig2 = lane_f(gl, j);
     float tau = 0.f, beta = alpha, scale = 0.f;
     if (sig2 > 0.f) {
       beta = -copysignf(sqrtf(alpha * alpha + sig2), alpha);
       tau = (beta - alpha) / beta;
       scale = 1.f / (alpha - beta);
     }
+    const float dl = fmaf(scale, gl, rl);
     float dot[NB];
 #pragma unroll
-    for (int c = 0; c < NB; ++c) dot[c] = fmaf(scale, bc[c], rj[c]);
+    for (int c = 0; c < NB; ++c) dot[c] = lane_f(dl, c);
     // v (rows > j) replaces column j; P[:, c] -= tau v w_c for c > j
 #pragma unroll
     for (int h = 0; h < RPT; ++h) {
