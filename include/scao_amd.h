@@ -204,8 +204,8 @@ int scao_fused_kronecker_precond_noalloc(const float* U_l, const float* s_l_inv4
                                          int64_t n, int64_t k, void* stream);
 /* x = fp32(q)*fp32(scale) * fp32(rho) + new_val; scale' = max|x|/127 (double)
  * or 1.0; q' = clamp(rint(x * fp32(1/scale')), +-127).  Updates q in place,
- * writes scale' to *scale_out (device double).  scratch: n floats +
- * scao_reduce_scratch_bytes(n). */
+ * writes scale' to *scale_out (device double).  scratch:
+ * scao_int8_ema_scratch_bytes(n) bytes. */
 int64_t scao_int8_ema_scratch_bytes(int64_t n);
 int scao_int8_ema_update(int8_t* q, double scale_in, const float* new_val, double rho,
                          int64_t n, double* scale_out, void* scratch, void* stream);

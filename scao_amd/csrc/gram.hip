@@ -436,8 +436,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   }
 }
 
-// Requantise x[0:n) given the per-tile maxima; divide (utils.quantize_sym_int8)
-// or multiply by the fp32 reciprocal (the int8_ema_update operator).
 // Code for one value: rint(y) clamped to +-127 (rintf rounds half to even,
 // as torch.round does).
 __device__ __forceinline__ uint32_t code_of(float y) {
@@ -445,14 +443,13 @@ __device__ __forceinline__ uint32_t code_of(float y) {
 }
 
 // Requantise one SCAO_FLAT_CHUNK-element chunk of x into q.  The scale is
-// max|x| / 127 in double from the per-tile maxima amax[0..nparts); `recip`
-// selects the reference operator's reciprocal multiply
-// (scao/cuda/__init__.py:122-142) instead of quantize_sym_int8's division
-// (scao/utils.py:170-189).  Whole, aligned chunks stream 4 values per load
-// and store 4 codes per 32-bit write, each wave covering 1 KB of x per
-// instruction; other chunks go element by element.
+// max|x| / 127 in double from the per-tile maxima amax[0..nparts), and x is
+// divided by it (utils.quantize_sym_int8, scao/utils.py:170-189).  Whole,
+// aligned chunks stream 4 values per load and store 4 codes per 32-bit write,
+// each wave covering 1 KB of x per instruction; other chunks go element by
+// element.
 __device__ __forceinline__ void requant_chunk(const float* x, int64_t n, const float* amax, int nparts,
-                              int8_t* q, double* scale_out, int chunk, bool recip) {
+                              int8_t* q, double* scale_out, int chunk) {
   __shared__ float red[4];
   const int64_t base = (int64_t)chunk * SCAO_FLAT_CHUNK;
   const bool vec = base + SCAO_FLAT_CHUNK <= n && (((uintptr_t)x | (uintptr_t)q) & 15) == 0;
@@ -465,19 +462,9 @@ __device__ __forceinline__ void requant_chunk(const float* x, int64_t n, const f
   for (int i = threadIdx.x; i < nparts; i += 256) mx = fmaxf(mx, amax[i]);
   mx = block_max(mx, red);
   const double amax_d = (double)mx;
-  double scale;
-  float mul = 0.f, div = 1.f;
-  bool zero;
-  if (recip) {
-    scale = amax_d > 1e-30 ? amax_d / 127.0 : 1.0;
-    const double inv = scale > 1e-30 ? 1.0 / scale : 0.0;
-    mul = (float)inv;
-    zero = false;
-  } else {
-    zero = amax_d < 1e-30;
-    scale = zero ? 1.0 : amax_d / 127.0;
-    div = (float)scale;
-  }
+  const bool zero = amax_d < 1e-30;
+  const double scale = zero ? 1.0 : amax_d / 127.0;
+  const float div = (float)scale;
   if (chunk == 0 && threadIdx.x == 0) *scale_out = scale;
   if (vec) {
 #pragma unroll
@@ -486,7 +473,7 @@ __device__ __forceinline__ void requant_chunk(const float* x, int64_t n, const f
       if (!zero) {
 #pragma unroll
         for (int t = 0; t < 4; ++t)
-          w |= code_of(recip ? v[j][t] * mul : v[j][t] / div) << (8 * t);
+          w |= code_of(v[j][t] / div) << (8 * t);
       }
       gst1((uint32_t*)(q + base) + threadIdx.x + 256 * j, w);
     }
@@ -495,7 +482,7 @@ __device__ __forceinline__ void requant_chunk(const float* x, int64_t n, const f
   for (int t = threadIdx.x; t < SCAO_FLAT_CHUNK; t += 256) {
     const int64_t e = base + t;
     if (e >= n) break;
-    q[e] = zero ? (int8_t)0 : (int8_t)code_of(recip ? x[e] * mul : x[e] / div);
+    q[e] = zero ? (int8_t)0 : (int8_t)code_of(x[e] / div);
   }
 }
 
@@ -505,7 +492,7 @@ __global__ __launch_bounds__(256) void k_requant(const scao_task* __restrict__ t
   const scao_task tk = tasks[blockIdx.x];
   const scao_gram_desc D = descs[tk.idx];
   const int dim = D.side == 0 ? D.rows : D.cols;
-  requant_chunk(D.ema, (int64_t)dim * dim, D.amax, D.ntiles, D.q, scale_out[tk.idx], tk.a, false);
+  requant_chunk(D.ema, (int64_t)dim * dim, D.amax, D.ntiles, D.q, scale_out[tk.idx], tk.a);
 }
 
 // eigh input, pass 1 (one block per factor): shift = fp32(max(1e-8,
@@ -827,29 +814,98 @@ __global__ __launch_bounds__(ED_T) void k_eig_diag(const scao_prep_desc* __restr
   }
 }
 
-// int8_ema_update pass 1: x = fp32(fp32(q*s)*rho) + v, per-block |x| max
+// int8_ema_update: x = fp32(fp32(q*s)*rho) + v, requantised at max|x| / 127.
+// Pass 1 takes max|x| per block, pass 2 forms x again (the same operations)
+// and writes the codes, x times the fp32 reciprocal of the scale (the reference
+// operator's arithmetic, scao/cuda/__init__.py:122-142): 5 + 6 B per element,
+// where keeping x between the passes takes 14.  Blocks take chunks blockIdx.x, + gridDim.x, .. of at most
+// EMA_BLOCKS blocks: pass 2 reads every block's maximum, and with a block per
+// chunk those reads grow with the square of n (at 4096 x 4096, 64 MB of them).
+// 4096 x 4096: 46 -> 32 us for the two passes.
+constexpr int EMA_BLOCKS = 1024;
+typedef uint32_t u32_a1 __attribute__((aligned(1)));   // four codes at any address
+typedef __attribute__((address_space(1))) u32_a1 gu32_a1;
+
+// thread's elements of a chunk: 4 * threadIdx.x + 1024 * j + t, j and t < 4
+struct ema_chunk {
+  v4f v[4];
+  uint32_t q[4];
+  __device__ __forceinline__ void load(const int8_t* qs, const float* vs, int64_t base,
+                                       int64_t n) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int64_t e = base + 4 * threadIdx.x + 1024 * j;
+      if (e + 4 <= n) {
+        v[j] = gld4(vs + e);
+        q[j] = *(const gu32_a1*)(qs + e);
+      } else {   // past the end: zeros
+        v[j] = v4f{0.f, 0.f, 0.f, 0.f};
+        q[j] = 0u;
+        for (int t = 0; t < 4; ++t)
+          if (e + t < n) {
+            v[j][t] = vs[e + t];
+            q[j] |= (uint32_t)(uint8_t)qs[e + t] << (8 * t);
+          }
+      }
+    }
+  }
+  __device__ __forceinline__ float x(int j, int t, float sf, float rho) const {
+    return ((float)(int8_t)(q[j] >> (8 * t)) * sf) * rho + v[j][t];
+  }
+};
+
 __global__ __launch_bounds__(256) void k_ema_pass1(const int8_t* __restrict__ q, float sf,
                                                    float rho, const float* __restrict__ v,
-                                                   int64_t n, float* __restrict__ x,
-                                                   float* __restrict__ amax) {
+                                                   int64_t n, float* __restrict__ amax) {
   __shared__ float red[4];
-  const int64_t base = (int64_t)blockIdx.x * SCAO_FLAT_CHUNK;
   float mx = 0.f;
-  for (int t = threadIdx.x; t < SCAO_FLAT_CHUNK; t += 256) {
-    const int64_t e = base + t;
-    if (e >= n) break;
-    const float y = ((float)q[e] * sf) * rho + v[e];
-    x[e] = y;
-    mx = fmaxf(mx, fabsf(y));
+  for (int64_t base = (int64_t)blockIdx.x * SCAO_FLAT_CHUNK; base < n;
+       base += (int64_t)gridDim.x * SCAO_FLAT_CHUNK) {
+    ema_chunk c;
+    c.load(q, v, base, n);
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int t = 0; t < 4; ++t) mx = fmaxf(mx, fabsf(c.x(j, t, sf, rho)));
   }
   mx = block_max(mx, red);
   if (threadIdx.x == 0) amax[blockIdx.x] = mx;
 }
 
-__global__ __launch_bounds__(256) void k_ema_pass2(const float* __restrict__ x, int64_t n,
+__global__ __launch_bounds__(256) void k_ema_pass2(int8_t* __restrict__ q, float sf, float rho,
+                                                   const float* __restrict__ v, int64_t n,
                                                    const float* __restrict__ amax, int nparts,
-                                                   int8_t* __restrict__ q, double* scale_out) {
-  requant_chunk(x, n, amax, nparts, q, scale_out, blockIdx.x, true);
+                                                   double* scale_out) {
+  __shared__ float red[4];
+  const int64_t step = (int64_t)gridDim.x * SCAO_FLAT_CHUNK;
+  int64_t base = (int64_t)blockIdx.x * SCAO_FLAT_CHUNK;
+  ema_chunk c;
+  c.load(q, v, base, n);   // the first chunk's loads go out before the scale is known
+  float mx = 0.f;
+  for (int i = threadIdx.x; i < nparts; i += 256) mx = fmaxf(mx, amax[i]);
+  mx = block_max(mx, red);
+  const double amax_d = (double)mx;
+  const double scale = amax_d > 1e-30 ? amax_d / 127.0 : 1.0;
+  const float mul = (float)(scale > 1e-30 ? 1.0 / scale : 0.0);
+  if (blockIdx.x == 0 && threadIdx.x == 0) *scale_out = scale;
+  for (;;) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      uint32_t w = 0;
+#pragma unroll
+      for (int t = 0; t < 4; ++t) w |= code_of(c.x(j, t, sf, rho) * mul) << (8 * t);
+      const int64_t e = base + 4 * threadIdx.x + 1024 * j;
+      if (e + 4 <= n) {
+        *(gu32_a1*)(q + e) = w;
+      } else {
+        for (int t = 0; t < 4; ++t)
+          if (e + t < n) q[e + t] = (int8_t)(w >> (8 * t));
+      }
+    }
+    base += step;
+    if (base >= n) break;
+    c.load(q, v, base, n);
+  }
 }
 
 }  // namespace
@@ -932,14 +988,15 @@ extern "C" int scao_int8_ema_update(int8_t* q, double scale_in, const float* new
   SCAO_CHECK_ARG(n < (int64_t)SCAO_FLAT_CHUNK * 0x7fffffffLL, "scao_int8_ema_update: n too large");
   if (n == 0) return SCAO_OK;
   SCAO_CHECK_ARG(q && new_val && scale_out && scratch, "scao_int8_ema_update: null pointer");
-  const int parts = (int)((n + SCAO_FLAT_CHUNK - 1) / SCAO_FLAT_CHUNK);
-  float* x = (float*)scratch;
-  float* amax = x + n;
+  const int64_t chunks = (n + SCAO_FLAT_CHUNK - 1) / SCAO_FLAT_CHUNK;
+  const int parts = (int)(chunks < EMA_BLOCKS ? chunks : EMA_BLOCKS);
+  float* amax = (float*)scratch;
   hipStream_t s = (hipStream_t)stream;
   hipLaunchKernelGGL(k_ema_pass1, dim3(parts), dim3(256), 0, s, q, (float)scale_in, (float)rho,
-                     new_val, n, x, amax);
+                     new_val, n, amax);
   SCAO_LAUNCH_CHECK("scao_int8_ema_update/pass1");
-  hipLaunchKernelGGL(k_ema_pass2, dim3(parts), dim3(256), 0, s, x, n, amax, parts, q, scale_out);
+  hipLaunchKernelGGL(k_ema_pass2, dim3(parts), dim3(256), 0, s, q, (float)scale_in, (float)rho,
+                     new_val, n, amax, parts, scale_out);
   SCAO_LAUNCH_CHECK("scao_int8_ema_update/pass2");
   return SCAO_OK;
 }
