@@ -973,6 +973,18 @@ __device__ __forceinline__ double sum16(double x) {
   x += dpp_d<DPP_ROW_MIRROR>(x);
   return x;
 }
+// 1 / sqrt(x) and 1 / x for normal x: the hardware estimates and two Newton steps
+__device__ __forceinline__ double rsqrt_d(double x) {
+  double r = __builtin_amdgcn_rsq(x);
+  const double xh = 0.5 * x;
+  r = fma(r, fma(-xh * r, r, 0.5), r);
+  return fma(r, fma(-xh * r, r, 0.5), r);
+}
+__device__ __forceinline__ double recip_d(double x) {
+  double r = __builtin_amdgcn_rcp(x);
+  r = fma(r, fma(-x, r, 1.0), r);
+  return fma(r, fma(-x, r, 1.0), r);
+}
 // LDS traffic of one wavefront is ordered; this keeps the compiler from
 // moving its accesses across the point.
 __device__ __forceinline__ void wave_sync() {
@@ -1095,11 +1107,18 @@ __global__ __launch_bounds__(SB_W * 64) void k_sb2st(double* band, int n, double
         const double x0 = rr < LM ? S.E[rr][0] : 0.0;
         const double alpha = S.E[0][0];
         const double s2 = sum16(rr >= 1 ? x0 * x0 : 0.0);
+        // beta = -sign(alpha) |x|, tau = (beta - alpha) / beta = 1 + |alpha| / |x|,
+        // scale = 1 / (alpha - beta), from Newton-refined reciprocal roots (a few
+        // ulps; a square root and two divisions are twice the instructions: 13
+        // matrices of 2048 rows 27.2 -> 26.5 ms).
+        // Below 1e-300 (entries under 1e-150 of an fp32 matrix's) nothing is
+        // left to annihilate.
         double tau = 0.0, beta = alpha, scale = 0.0;
-        if (s2 > 0.0) {
-          beta = -copysign(sqrt(alpha * alpha + s2), alpha);
-          tau = (beta - alpha) / beta;
-          scale = 1.0 / (alpha - beta);
+        if (s2 > 1e-300) {
+          const double h = fma(alpha, alpha, s2), r = rsqrt_d(h), nx = h * r;
+          beta = -copysign(nx, alpha);
+          tau = fma(fabs(alpha), r, 1.0);
+          scale = copysign(recip_d(fabs(alpha) + nx), alpha);
         }
         wave_sync();
         if (l < NB) {
