@@ -239,7 +239,7 @@ __global__ __launch_bounds__(256) void k_diag_apply(const scao_task* __restrict_
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
       const float x = dg[t] / P.diag_bias;
-      const float den = (float)pow((double)x, 0.25) + 1e-8f;
+      const float den = root4(x) + 1e-8f;
       gp[t] = round_to(dt, graw[t] / den);
     }
     const v4f u = adan_tail(P, S, e, g, gp, vec, mk);
@@ -378,81 +378,16 @@ __global__ __launch_bounds__(256) void k_lookahead(const scao_task* __restrict__
 }
 
 // ---------------------------------------------------------- finalize ---
-__global__ __launch_bounds__(256) void k_finalize_params(const scao_param_desc* __restrict__ params,
-                                                         const double* __restrict__ slots,
-                                                         scao_param_stat* stat, int phase) {
-  __shared__ double red[16];
-  const scao_param_desc& P = params[blockIdx.x];
-  scao_param_stat& S = stat[blockIdx.x];
-  const int l = threadIdx.x;
-  const int dt = P.dtype;
-  const double* __restrict__ sl = slots;
-  if (phase == 0) {
-    // four independent partial sums per thread keep four slot loads in
-    // flight (an Adam-path embedding has tens of thousands of slots); they
-    // are combined in a fixed order
-    double a4[3][4] = {};
-    int s = P.pre_begin + l;
-    for (; s + 768 < P.pre_end; s += 1024)
-#pragma unroll
-      for (int u = 0; u < 4; ++u)
-#pragma unroll
-        for (int q = 0; q < 3; ++q) a4[q][u] += sl[(int64_t)(s + 256 * u) * SCAO_SLOT_WIDTH + q];
-    for (; s < P.pre_end; s += 256)
-#pragma unroll
-      for (int q = 0; q < 3; ++q) a4[q][0] += sl[(int64_t)s * SCAO_SLOT_WIDTH + q];
-    double a[3];
-#pragma unroll
-    for (int q = 0; q < 3; ++q) a[q] = (a4[q][0] + a4[q][1]) + (a4[q][2] + a4[q][3]);
-    block_sum<3>(a, red);
-    if (l == 0) {
-      S.g2 = a[0];
-      S.p2 = a[1];
-      S.nu2 = a[2];
-      S.gnorm = round_to(dt, (float)sqrt(a[0]));
-      S.pnorm = round_to(dt, (float)sqrt(a[1]));
-      const float nu = (float)sqrt(a[2]);
-      S.nu = nu;
-      float clip = 1.0f;
-      if ((P.flags & SCAO_PF_CLIP) && nu > P.tau) clip = (1.0f / fmaxf(nu, P.eps)) * P.tau;
-      S.clip = clip;
-      S.u2 = 0.0;
-      S.unorm = 0.f;
-      S.trust = 1.0f;
-      S.alpha = round_to(dt, (float)(-P.lr));
-    }
-  } else {
-    double a4[4] = {0.0, 0.0, 0.0, 0.0};
-    int s = P.post_begin + l;
-    for (; s + 768 < P.post_end; s += 1024)
-#pragma unroll
-      for (int u = 0; u < 4; ++u) a4[u] += sl[(int64_t)(s + 256 * u) * SCAO_SLOT_WIDTH + 2];
-    for (; s < P.post_end; s += 256) a4[0] += sl[(int64_t)s * SCAO_SLOT_WIDTH + 2];
-    double ax[1] = {(a4[0] + a4[1]) + (a4[2] + a4[3])};
-    block_sum<1>(ax, red);
-    const double a = ax[0];
-    if (l == 0) {
-      S.u2 = a;
-      const float un = (float)sqrt(a);
-      S.unorm = un;
-      float trust = 1.0f;
-      if ((P.flags & SCAO_PF_LARS) && !(S.pnorm == 0.f || un == 0.f)) {
-        const float num = round_to(dt, P.lars * S.pnorm);
-        const float wdp = round_to(dt, P.wd * S.pnorm);
-        trust = num / ((un + wdp) + 1e-8f);
-      }
-      S.trust = trust;
-      S.alpha = round_to(dt, (float)(-(P.lr * (double)trust)));
-    }
-  }
-}
+// threads of a block: one block adds all of a parameter's slots (64 K of them
+// for a Llama-1B embedding's Phase 1: 41 us with 256 threads, 21 with 1024)
+constexpr int FIN_T = 1024;
 
 // The average of the per-parameter gradient norms, summed in parameter order
-// as the reference's Python sum does; 256 threads stage each batch of norms in
+// as the reference's Python sum does; the block stages each batch of norms in
 // LDS so that the ordered sum does not wait on one global load per term.
-__global__ __launch_bounds__(256) void k_finalize_global(const scao_param_desc* __restrict__ params,
-                                                         int nparams, const scao_param_stat* stat,
-                                                         double* runtime, int norm_count) {
+__device__ __forceinline__ void finalize_global(const scao_param_desc* __restrict__ params,
+                                                int nparams, const scao_param_stat* stat,
+                                                double* runtime, int norm_count) {
   constexpr int B = 1024;
   __shared__ double v[B];
   __shared__ int use[B];
@@ -460,7 +395,7 @@ __global__ __launch_bounds__(256) void k_finalize_global(const scao_param_desc* 
   int cnt = 0;
   for (int b0 = 0; b0 < nparams; b0 += B) {
     const int nb = nparams - b0 < B ? nparams - b0 : B;
-    for (int i = threadIdx.x; i < nb; i += 256) {
+    for (int i = threadIdx.x; i < nb; i += FIN_T) {
       use[i] = params[b0 + i].norm_index >= 0;
       v[i] = (double)stat[b0 + i].gnorm;
     }
@@ -481,6 +416,88 @@ __global__ __launch_bounds__(256) void k_finalize_global(const scao_param_desc* 
   const double avg = sum / (double)cnt;
   runtime[1] = avg;
   runtime[0] = 0.95 * runtime[0] + 0.05 * avg;
+}
+
+__global__ __launch_bounds__(FIN_T) void k_finalize_global(
+    const scao_param_desc* __restrict__ params, int nparams, const scao_param_stat* stat,
+    double* runtime, int norm_count) {
+  finalize_global(params, nparams, stat, runtime, norm_count);
+}
+
+// One block per parameter; a last block, when `runtime` is given, takes the
+// global average (its inputs are the first phase's, so it shares the second
+// phase's launch).
+__global__ __launch_bounds__(FIN_T) void k_finalize_params(
+    const scao_param_desc* __restrict__ params, int nparams, const double* __restrict__ slots,
+    scao_param_stat* stat, int phase, double* runtime, int norm_count) {
+  __shared__ double red[3 * FIN_T / 64];
+  if ((int)blockIdx.x == nparams) {
+    finalize_global(params, nparams, stat, runtime, norm_count);
+    return;
+  }
+  const scao_param_desc& P = params[blockIdx.x];
+  scao_param_stat& S = stat[blockIdx.x];
+  const int l = threadIdx.x;
+  const int dt = P.dtype;
+  const double* __restrict__ sl = slots;
+  if (phase == 0) {
+    // four independent partial sums per thread keep four slot loads in
+    // flight (an Adam-path embedding has tens of thousands of slots); they
+    // are combined in a fixed order
+    double a4[3][4] = {};
+    int s = P.pre_begin + l;
+    for (; s + 3 * FIN_T < P.pre_end; s += 4 * FIN_T)
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+#pragma unroll
+        for (int q = 0; q < 3; ++q) a4[q][u] += sl[(int64_t)(s + FIN_T * u) * SCAO_SLOT_WIDTH + q];
+    for (; s < P.pre_end; s += FIN_T)
+#pragma unroll
+      for (int q = 0; q < 3; ++q) a4[q][0] += sl[(int64_t)s * SCAO_SLOT_WIDTH + q];
+    double a[3];
+#pragma unroll
+    for (int q = 0; q < 3; ++q) a[q] = (a4[q][0] + a4[q][1]) + (a4[q][2] + a4[q][3]);
+    block_sum_n<3, FIN_T>(a, red);
+    if (l == 0) {
+      S.g2 = a[0];
+      S.p2 = a[1];
+      S.nu2 = a[2];
+      S.gnorm = round_to(dt, (float)sqrt(a[0]));
+      S.pnorm = round_to(dt, (float)sqrt(a[1]));
+      const float nu = (float)sqrt(a[2]);
+      S.nu = nu;
+      float clip = 1.0f;
+      if ((P.flags & SCAO_PF_CLIP) && nu > P.tau) clip = (1.0f / fmaxf(nu, P.eps)) * P.tau;
+      S.clip = clip;
+      S.u2 = 0.0;
+      S.unorm = 0.f;
+      S.trust = 1.0f;
+      S.alpha = round_to(dt, (float)(-P.lr));
+    }
+  } else {
+    double a4[4] = {0.0, 0.0, 0.0, 0.0};
+    int s = P.post_begin + l;
+    for (; s + 3 * FIN_T < P.post_end; s += 4 * FIN_T)
+#pragma unroll
+      for (int u = 0; u < 4; ++u) a4[u] += sl[(int64_t)(s + FIN_T * u) * SCAO_SLOT_WIDTH + 2];
+    for (; s < P.post_end; s += FIN_T) a4[0] += sl[(int64_t)s * SCAO_SLOT_WIDTH + 2];
+    double ax[1] = {(a4[0] + a4[1]) + (a4[2] + a4[3])};
+    block_sum_n<1, FIN_T>(ax, red);
+    const double a = ax[0];
+    if (l == 0) {
+      S.u2 = a;
+      const float un = (float)sqrt(a);
+      S.unorm = un;
+      float trust = 1.0f;
+      if ((P.flags & SCAO_PF_LARS) && !(S.pnorm == 0.f || un == 0.f)) {
+        const float num = round_to(dt, P.lars * S.pnorm);
+        const float wdp = round_to(dt, P.wd * S.pnorm);
+        trust = num / ((un + wdp) + 1e-8f);
+      }
+      S.trust = trust;
+      S.alpha = round_to(dt, (float)(-(P.lr * (double)trust)));
+    }
+  }
 }
 
 }  // namespace
@@ -544,12 +561,14 @@ extern "C" int scao_step_finalize(const scao_param_desc* params, int nparams, co
   if (nparams == 0) return SCAO_OK;
   SCAO_CHECK_ARG(params && slots && stat, "scao_step_finalize: null pointer");
   hipStream_t s = (hipStream_t)stream;
-  hipLaunchKernelGGL(k_finalize_params, dim3(nparams), dim3(256), 0, s, params, slots, stat, phase);
+  SCAO_CHECK_ARG(!update_norm_ema || runtime != nullptr, "scao_step_finalize: null runtime");
+  const int with_global = phase == 1 && update_norm_ema ? 1 : 0;
+  hipLaunchKernelGGL(k_finalize_params, dim3(nparams + with_global), dim3(FIN_T), 0, s, params,
+                     nparams, slots, stat, phase, runtime, norm_count);
   SCAO_LAUNCH_CHECK("scao_step_finalize");
   if (phase == 0 && update_norm_ema) {
-    SCAO_CHECK_ARG(runtime != nullptr, "scao_step_finalize: null runtime");
-    hipLaunchKernelGGL(k_finalize_global, dim3(1), dim3(256), 0, s, params, nparams, stat, runtime,
-                       norm_count);
+    hipLaunchKernelGGL(k_finalize_global, dim3(1), dim3(FIN_T), 0, s, params, nparams, stat,
+                       runtime, norm_count);
     SCAO_LAUNCH_CHECK("scao_step_finalize/global");
   }
   return SCAO_OK;

@@ -177,11 +177,24 @@ __device__ __forceinline__ void project_tile(project_lds<CR>& lds, const scao_le
         int64_t col[NJ];
 #pragma unroll
         for (int t = 0; t < NJ; ++t) col[t] = L.off + min(gcol + t, n - 1);
+        if (dt == SCAO_F32) {
 #pragma unroll
-        for (int e = 0; e < 8; ++e)
+          for (int e = 0; e < 8; ++e)
 #pragma unroll
-          for (int t = 0; t < NJ; ++t)
-            r.x[e][t] = __float_as_uint(ld1(base, dt, col[t] + row(e)));
+            for (int t = 0; t < NJ; ++t) r.x[e][t] = gld1((const uint32_t*)base + col[t] + row(e));
+        } else {
+#pragma unroll
+          for (int e = 0; e < 8; ++e)
+#pragma unroll
+            for (int t = 0; t < NJ; ++t) r.x[e][t] = ((const gu16*)base)[col[t] + row(e)];
+#pragma unroll
+          for (int e = 0; e < 8; ++e)
+#pragma unroll
+            for (int t = 0; t < NJ; ++t) {
+              const uint16_t x = (uint16_t)r.x[e][t];
+              r.x[e][t] = __float_as_uint(dt == SCAO_BF16 ? bf16_to_f(x) : f16_to_f(x));
+            }
+        }
       }
 #pragma unroll
       for (int e = 0; e < 8; ++e)
@@ -601,6 +614,21 @@ __device__ __forceinline__ void delta_part(const scao_leaf_desc& L, int a0, int 
 #pragma unroll
   for (int t = 0; t < 4; ++t) acc[t] = v4f{0.f, 0.f, 0.f, 0.f};
   for (int jb = jbeg; jb < jend; jb += 64) {
+    // rows of U_r past n repeat row n - 1 and meet zeros of T
+    v4f cb[2][8];
+    if (dm == 15) {
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+          cb[h][e] = gld4(L.Ur + (int64_t)min(jb + 32 * h + 8 * g + e, n - 1) * k + dl);
+    } else {
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+          cb[h][e] = ldf4(L.Ur, (int64_t)min(jb + 32 * h + 8 * g + e, n - 1) * k + dl, false, dm);
+    }
     // 64 columns of T, summed over the row parts: thread -> rows tid / 16 + 16q
     const int col = jb + 4 * (tid % 16);
     int cm = 0;
@@ -626,21 +654,6 @@ __device__ __forceinline__ void delta_part(const scao_leaf_desc& L, int a0, int 
       for (int s = 1; s < parts; ++s)
 #pragma unroll
         for (int q = 0; q < 4; ++q) x[q] += ldf4(first + s * tp, at[q], false, cm);
-    }
-    // rows of U_r past n repeat row n - 1 and meet zeros of T
-    v4f cb[2][8];
-    if (dm == 15) {
-#pragma unroll
-      for (int h = 0; h < 2; ++h)
-#pragma unroll
-        for (int e = 0; e < 8; ++e)
-          cb[h][e] = gld4(L.Ur + (int64_t)min(jb + 32 * h + 8 * g + e, n - 1) * k + dl);
-    } else {
-#pragma unroll
-      for (int h = 0; h < 2; ++h)
-#pragma unroll
-        for (int e = 0; e < 8; ++e)
-          cb[h][e] = ldf4(L.Ur, (int64_t)min(jb + 32 * h + 8 * g + e, n - 1) * k + dl, false, dm);
     }
     if (jb > jbeg) __syncthreads();   // the previous columns' reads
 #pragma unroll
@@ -746,9 +759,10 @@ __device__ __forceinline__ void diag_leaf_reduce(const scao_leaf_desc& L,
   const bool decay = P.flags & SCAO_PF_DECAY;
   const bool lars = P.flags & SCAO_PF_LARS;
   double acc[3] = {0.0, 0.0, 0.0};
-  for (int q = threadIdx.x; q < 64 * 64; q += 256) {
-    const int i = i0 + q / 64, j = j0 + q % 64;
-    if (i >= L.m || j >= L.n) continue;
+  // only the elements that are there: the sub-block is one wide, so at most 64
+  const int rows = min(64, L.m - i0), cols = min(64, L.n - j0);
+  for (int q = threadIdx.x; q < rows * cols; q += 256) {
+    const int i = i0 + q / cols, j = j0 + q % cols;
     const int64_t e = L.off + (int64_t)i * L.ld + j;
     const float g = ld1(P.graw, dt, e);
     const float dg = gld1(L.Sl + (int64_t)i * L.n + j);
@@ -770,7 +784,7 @@ __device__ __forceinline__ void diag_leaf_reduce(const scao_leaf_desc& L,
 
 // -------------------------------------------------------------- lift ---
 // W[i0:i0+64, d0:d0+64] = U_l Delta.  Wave w computes rows i0+16w .. +15.
-// On whole tiles (k % 16 == 0, 16-byte aligned factors) lane column jj holds
+// On whole columns (k % 16 == 0, d0 + 64 <= k) lane column jj holds
 // W columns d0 + 4*jj + t of MFMA tile t, so one float4 of a Delta row feeds
 // all four tiles and each row of the result leaves as one float4; the
 // reduction runs with NH chunks of operands in flight (fully unrolled for
@@ -868,11 +882,9 @@ __device__ __forceinline__ void lift_tile(const scao_leaf_desc& L, int i0, int d
   v4f acc[4];
 #pragma unroll
   for (int t = 0; t < 4; ++t) acc[t] = v4f{0.f, 0.f, 0.f, 0.f};
-  const bool whole = k % 16 == 0 && i0 + 64 <= m && d0 + 64 <= k &&
-                     (((uintptr_t)L.Ul | (uintptr_t)L.Delta | (uintptr_t)L.W) & 15) == 0 &&
-                     ((uintptr_t)L.Wb & 7) == 0;
-  if (whole) {
-    const int irow = i0 + 16 * w + (l % 16);
+  if (k % 16 == 0 && d0 + 64 <= k) {
+    // rows past the block repeat its last one and are not stored
+    const int irow = min(i0 + 16 * w + (l % 16), m - 1);
     const int dl = d0 + 4 * (l % 16);
     const float* __restrict__ urow = L.Ul + (int64_t)irow * k + 4 * kk;
     const float* __restrict__ drow = L.Delta + (int64_t)(4 * kk) * k + dl;
@@ -886,7 +898,9 @@ __device__ __forceinline__ void lift_tile(const scao_leaf_desc& L, int i0, int d
       lift_chunks<0>(urow, drow, k, acc);
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      const int64_t o = (int64_t)(i0 + 16 * w + 4 * kk + r) * k + dl;
+      const int i = i0 + 16 * w + 4 * kk + r;
+      if (i >= m) continue;
+      const int64_t o = (int64_t)i * k + dl;
       const v4f x = v4f{acc[0][r], acc[1][r], acc[2][r], acc[3][r]};
       gst4(L.W + o, x);
       if (L.Wb) store_split4(L.Wb, (int64_t)m * k, o, x);
@@ -930,9 +944,7 @@ __device__ __forceinline__ void lift_tile(const scao_leaf_desc& L, int i0, int d
 // and wave w adds rows 16w .. 16w + 15 of them in order (((w0 + w1) + w2) + w3)
 // and writes those rows of W (and Wb).
 __device__ __forceinline__ bool lift_x6_ok(const scao_leaf_desc& L, int i0, int d0) {
-  return L.k % 128 == 0 && i0 + 64 <= L.m && d0 + 64 <= L.k &&
-         (((uintptr_t)L.Ul | (uintptr_t)L.Delta | (uintptr_t)L.W) & 15) == 0 &&
-         ((uintptr_t)L.Wb & 7) == 0;
+  return L.k % 128 == 0 && i0 + 64 <= L.m && d0 + 64 <= L.k;
 }
 __device__ __forceinline__ void lift_tile_x6(const scao_leaf_desc& L, int i0, int d0,
                                              float (*Ps)[64][DP]) {
@@ -1133,27 +1145,65 @@ __device__ __forceinline__ void apply_tile(const scao_leaf_desc& L, const scao_p
   for (int t = 0; t < 4; ++t) cmask = (jl + t < n) ? cmask : (cmask & ~(1 << t));
   const bool vec = cmask == 15;
 
-  // 1) prefetch
+  // 1) prefetch.  A lane whose four columns all lie in the block loads every
+  // row unconditionally, rows past the block from its last one (they are not
+  // stored): a branch per load would wait for each.
   v4f gr[4], gm[4], mm[4], vv[4], dd[4], pp[4], par[4];
   int64_t e[4];
   bool rok[4];
+  const v4f z = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
     const int i = i0 + 16 * w + 4 * kk + r;
-    e[r] = L.off + (int64_t)i * L.ld + jl;
+    e[r] = L.off + (int64_t)min(i, m - 1) * L.ld + jl;
     rok[r] = i < m && cmask;
-    const v4f z = {0.f, 0.f, 0.f, 0.f};
-    gr[r] = rok[r] ? ld4(P.graw, dt, e[r], vec, cmask) : z;
+  }
+  const bool fused = GF32 && fused_mgrad(P), fmask = GF32 && (P.flags & SCAO_PF_FMASK);
+  if (vec) {
+    if (dt == SCAO_F32) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        gr[r] = gld4((const float*)P.graw + e[r]);
+        if (!LARS) par[r] = gld4((const float*)P.p + e[r]);
+      }
+    } else {
+      v2u hg[4], hp[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        hg[r] = gld2w((const uint16_t*)P.graw + e[r]);
+        if (!LARS) hp[r] = gld2w((const uint16_t*)P.p + e[r]);
+      }
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        gr[r] = halves_to_v4f(dt, hg[r]);
+        if (!LARS) par[r] = halves_to_v4f(dt, hp[r]);
+      }
+    }
     // GF32: the fp32 moment buffer, or (fused) the filter's EMA until finish_mgrad
-    gm[r] = (GF32 && rok[r])
-                ? (fused_mgrad(P) ? ((P.flags & SCAO_PF_FMASK) ? ldf4(P.fema, e[r], vec, cmask) : gr[r])
-                                  : ldf4((const float*)P.g, e[r], vec, cmask))
-                : z;
-    mm[r] = rok[r] ? ldf4(P.exp_avg, e[r], vec, cmask) : z;
-    vv[r] = rok[r] ? ldf4(P.exp_avg_sq, e[r], vec, cmask) : z;
-    dd[r] = rok[r] ? ldf4(P.exp_avg_diff, e[r], vec, cmask) : z;
-    pp[r] = rok[r] ? ldf4(P.prev_grad, e[r], vec, cmask) : z;
-    par[r] = (!LARS && rok[r]) ? ld4(P.p, dt, e[r], vec, cmask) : z;
+    if (GF32 && (fmask || !fused)) {
+      const float* src = fused ? P.fema : (const float*)P.g;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) gm[r] = gld4(src + e[r]);
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      mm[r] = gld4(P.exp_avg + e[r]);
+      vv[r] = gld4(P.exp_avg_sq + e[r]);
+      dd[r] = gld4(P.exp_avg_diff + e[r]);
+      pp[r] = gld4(P.prev_grad + e[r]);
+    }
+  } else {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      gr[r] = ld4(P.graw, dt, e[r], false, cmask);
+      if (GF32 && (fmask || !fused))
+        gm[r] = ldf4(fused ? P.fema : (const float*)P.g, e[r], false, cmask);
+      mm[r] = ldf4(P.exp_avg, e[r], false, cmask);
+      vv[r] = ldf4(P.exp_avg_sq, e[r], false, cmask);
+      dd[r] = ldf4(P.exp_avg_diff, e[r], false, cmask);
+      pp[r] = ldf4(P.prev_grad, e[r], false, cmask);
+      if (!LARS) par[r] = ld4(P.p, dt, e[r], false, cmask);
+    }
   }
 
   // 2) corr = W U_r^T; for a diagonal sub-block the preconditioned gradient
@@ -1172,40 +1222,55 @@ __device__ __forceinline__ void apply_tile(const scao_leaf_desc& L, const scao_p
 #pragma unroll
       for (int t = 0; t < 4; ++t) {
         const float x = dg[t] / L.dbias;
-        const float den = (float)pow((double)x, 0.25) + 1e-8f;
+        const float den = root4(x) + 1e-8f;
         acc[t][r] = gr[r][t] / den;
       }
     }
   }
-  const int irow = i0 + 16 * w + (l % 16);
+  // Rows past the block repeat its last ones (their products are not used);
+  // columns of k past it (k % 64 != 0) are masked.
+  const float* wrow = L.W + (int64_t)min(i0 + 16 * w + (l % 16), m - 1) * k;
   for (int cb0 = 0; cb0 < (dleaf ? 0 : k); cb0 += 64) {
+    const int c4 = (threadIdx.x % 16) * 4;
+    const bool whole = cb0 + 64 <= k;
+    v4f x[4];
+    if (whole) {
+#pragma unroll
+      for (int h = 0; h < 4; ++h)
+        x[h] = gld4(L.Ur + (int64_t)min(j0 + (int)threadIdx.x / 16 + 16 * h, n - 1) * k + cb0 + c4);
+    } else {
+      int mk = 0;
+      for (int t = 0; t < 4; ++t) mk |= (cb0 + c4 + t < k) ? (1 << t) : 0;
+#pragma unroll
+      for (int h = 0; h < 4; ++h)
+        x[h] = ldf4(L.Ur, (int64_t)min(j0 + (int)threadIdx.x / 16 + 16 * h, n - 1) * k + cb0 + c4,
+                    false, mk);
+    }
+    v4f a[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int c = cb0 + 16 * q + 4 * kk;
+      if (whole) {
+        a[q] = gld4(wrow + c);
+      } else {
+        int cm = 0;
+        for (int s = 0; s < 4; ++s) cm |= (c + s < k) ? (1 << s) : 0;
+        a[q] = ldf4(wrow, c, false, cm);
+      }
+    }
     if (cb0) __syncthreads();
 #pragma unroll
-    for (int h = 0; h < 4; ++h) {
-      const int idx = threadIdx.x + 256 * h;
-      const int row = idx / 16, c4 = (idx % 16) * 4;
-      const int j = j0 + row, c = cb0 + c4;
-      int mk = 0;
-      for (int t = 0; t < 4; ++t) mk |= (j < n && c + t < k) ? (1 << t) : 0;
-      const v4f x = mk ? ldf4(L.Ur, (int64_t)j * k + c, mk == 15, mk)
-                       : v4f{0.f, 0.f, 0.f, 0.f};
-      *(v4f*)&Us[row][c4] = x;
-    }
+    for (int h = 0; h < 4; ++h) *(v4f*)&Us[threadIdx.x / 16 + 16 * h][c4] = x[h];
     __syncthreads();
-    const int cend = k - cb0 < 64 ? k - cb0 : 64;
-    for (int cb = 0; cb < cend; cb += 16) {
-      const int c = cb0 + cb + 4 * kk;
-      int cm = 15;
-      for (int s = 0; s < 4; ++s) cm = (c + s < k) ? cm : (cm & ~(1 << s));
-      const v4f a = (irow < m && cm) ? ldf4(L.W, (int64_t)irow * k + c, cm == 15, cm)
-                                     : v4f{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
       v4f b[4];
 #pragma unroll
-      for (int t = 0; t < 4; ++t) b[t] = *(const v4f*)&Us[jl - j0 + t][cb + 4 * kk];
+      for (int t = 0; t < 4; ++t) b[t] = *(const v4f*)&Us[jl - j0 + t][16 * q + 4 * kk];
 #pragma unroll
       for (int s = 0; s < 4; ++s)
 #pragma unroll
-        for (int t = 0; t < 4; ++t) acc[t] = mfma16(a[s], b[t][s], acc[t]);
+        for (int t = 0; t < 4; ++t) acc[t] = mfma16(a[q][s], b[t][s], acc[t]);
     }
   }
 

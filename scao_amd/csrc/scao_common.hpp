@@ -375,12 +375,16 @@ __device__ __forceinline__ float block_max(float x, float* lds) {
   return r;
 }
 
-// clamp(S, 1e-8)^(-1/4) for the eigenvalue scaling (torch: pow(-0.25)); the
-// double evaluation is correctly rounded, torch's CPU path is within 1 ulp.
+// clamp(S, 1e-8)^(-1/4) for the eigenvalue scaling (torch: pow(-0.25)), from two
+// square roots in double: within an ulp of a double, so the float is the
+// correctly rounded one but for ties; torch's CPU path is within 1 ulp.  (A
+// double pow is several times the instructions.)
 __device__ __forceinline__ float inv4(float s) {
-  float c = fmaxf(s, 1e-8f);
-  return (float)pow((double)c, -0.25);
+  const float c = fmaxf(s, 1e-8f);
+  return (float)(1.0 / sqrt(sqrt((double)c)));
 }
+// x^(1/4) likewise (x >= 0: an average of squares over its bias factor)
+__device__ __forceinline__ float root4(float x) { return (float)sqrt(sqrt((double)x)); }
 // clamp(S, eps)^(-1/2) = 1/sqrt (torch lowers pow(-0.5) to a reciprocal sqrt)
 __device__ __forceinline__ float inv2(float s, float eps) {
   float c = fmaxf(s, eps);

@@ -977,15 +977,17 @@ def _launch_step(ws: Workspace, raw: np.ndarray, n: int, update_norm_ema: bool) 
         _call("scao_kron_lift", tp("lift"), N["lift"], LF, s)
     if N["dred"]:
         _call("scao_diag_reduce", tp("dred"), N["dred"], P, SL, s)
-    _call("scao_step_finalize", P, n, SL, S, ws.runtime.data_ptr(), 0,
-           1 if update_norm_ema else 0, n, s)
+    # the global norm average joins the second finalize launch, if there is one
+    norm_ema = 1 if update_norm_ema else 0
+    R = ws.runtime.data_ptr()
+    _call("scao_step_finalize", P, n, SL, S, R, 0, 0 if N["lars"] else norm_ema, n, s)
     for var in _APPLY_VARIANTS:
         if N[f"apply{var}"]:
             _call("scao_kron_apply", tp(f"apply{var}"), N[f"apply{var}"], LF, P, S, SL, var, s)
     if N["dapply"]:
         _call("scao_diag_apply", tp("dapply"), N["dapply"], P, S, SL, s)
     if N["lars"]:
-        _call("scao_step_finalize", P, n, SL, S, 0, 1, 0, n, s)
+        _call("scao_step_finalize", P, n, SL, S, R, 1, norm_ema, n, s)
         _call("scao_lars_write", tp("lars"), N["lars"], P, S, s)
     ws.finish_params()
 
