@@ -261,7 +261,9 @@ int scao_step_finalize(const scao_param_desc* params, int nparams, const double*
  *     of TR rows x SW columns going down from row a in the column strip at
  *     b (SW = 64, TR = 128 for k = 256; SW = 128, TR = 64 for k = 128; mw =
  *     m - m % TR), with reduction slots slot, slot + 1, ...; b + SW <= n.
- *     Without SCAO_PF_GF32 the leaf needs Wb (written by scao_kron_lift).
+ *     | 128 (with 1 and 16): SCAO_PF_FMASK without SCAO_PF_FNOISE.  Without
+ *     SCAO_PF_GF32, and with | 128, the leaf needs Wb (written by
+ *     scao_kron_lift).
  *     A leaf of another k, or one lacking Wb, gets NaN in its run's slots. */
 int scao_kron_apply(const scao_task* tasks, int ntasks, const scao_leaf_desc* leaves,
                     const scao_param_desc* params, const scao_param_stat* stat,

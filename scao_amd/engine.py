@@ -99,6 +99,12 @@ class PItem:
         """The moments see another gradient than p.grad."""
         return self.gmom is not None or self.msrc is not None
 
+    @property
+    def masked(self) -> bool:
+        """... which is p.grad masked by the filter, without noise."""
+        ms = self.msrc
+        return self.gmom is None and ms is not None and ms.ema is not None and ms.noise == 0.0
+
 
 PARAM_RING = 4   # parameter-table staging slots (steps the host may run ahead)
 
@@ -233,8 +239,10 @@ def _flat_chunks(numel: int) -> int:
 
 _LEAF_TASKS = ("dpart", "delta", "lift")   # with proj* and apply*: idx is a block index
 _PROJ_VARIANTS = [0, 2] + [1 | p | w | t for t in (0, 16, 32) for w in (0, 4, 8) for p in (0, 2)]
-# masked tiles, wide, pipelined, strip (k = 256, 128); | 64: 16-bit data
-_APPLY_VARIANTS = [t | v for t in (0, 4, 12, 20, 52, 68, 84, 116) for v in range(4)]
+# masked tiles, wide, pipelined, strip (k = 256, 128); | 64: 16-bit data;
+# | 128: strip tiles whose moments see the filtered gradient without noise
+_APPLY_VARIANTS = ([t | v for t in (0, 4, 12, 20, 52, 68, 84, 116) for v in range(4)]
+                   + [128 | t | v for t in (20, 52, 84, 116) for v in (1, 3)])
 _TASK_TYPES = (["adam", "dpart", "delta", "lift", "dred", "dapply", "lars"] +
                [f"proj{v}" for v in sorted({*range(12), *_PROJ_VARIANTS})] +
                [f"apply{v}" for v in sorted({*range(64), *_APPLY_VARIANTS})])
@@ -405,7 +413,7 @@ def _param_tasks(it: PItem, plan: SplitPlan):
                 mw, nw = m - m % tr, n - n % sw
                 if not (mw and nw):
                     mw = nw = 0
-                wide = var | 4 | 16 | (32 if k == 128 else 0) | typed
+                wide = var | 4 | 16 | (32 if k == 128 else 0) | typed | (128 if it.masked else 0)
                 for i0, j0 in _strip_runs(mw, nw, tr, sw):
                     add(f"apply{wide}", (li, i0, j0, slot))
                     slot += min(L.APPLY_GROUP, (mw - i0) // tr)
@@ -439,7 +447,7 @@ def _param_tasks(it: PItem, plan: SplitPlan):
 
 def _item_key(it: PItem) -> tuple:
     """Everything _param_tasks reads from an item."""
-    return (id(it.p), it.phase2, it.diag, it.lars, it.mgrad, it.p.numel(), it.fp32,
+    return (id(it.p), it.phase2, it.diag, it.lars, it.mgrad, it.masked, it.p.numel(), it.fp32,
             _cols(it.p), it.half, tuple((id(lf), r0, c0, _leaf_k(lf)) for lf, r0, c0 in it.leaves)
             if it.phase2 and not it.diag else ())
 
@@ -884,11 +892,11 @@ def run_step(items: list[PItem], ws: Workspace, update_norm_ema: bool,
         it.ptrs = _item_ptrs(it)
     # the full structure key (with every block's rank) is only rebuilt when
     # the cheap one or the global factor epoch says something may have changed
-    ckey = (tuple((id(it.p), it.phase2, it.diag, it.lars, it.mgrad, it.p.numel(),
+    ckey = (tuple((id(it.p), it.phase2, it.diag, it.lars, it.mgrad, it.masked, it.p.numel(),
                    it.fp32, it.half, len(it.leaves)) for it in items), leaf_epoch())
     skey = ws.struct_key
     if ckey != ws.cheap_key:
-        skey = tuple((id(it.p), it.phase2, it.diag, it.lars, it.mgrad, it.p.numel(),
+        skey = tuple((id(it.p), it.phase2, it.diag, it.lars, it.mgrad, it.masked, it.p.numel(),
                       it.fp32, it.half,
                       tuple((id(lf), r0, c0, _leaf_k(lf)) for lf, r0, c0 in it.leaves))
                      for it in items)
