@@ -235,7 +235,9 @@ int scao_kron_delta(const scao_task* tasks, int ntasks, const scao_leaf_desc* le
 /* A3  W = U_l Delta per 64-row strip. */
 int scao_kron_lift(const scao_task* tasks, int ntasks, const scao_leaf_desc* leaves,
                    void* stream);
-/* Diagonal-mode params: ||g||^2, ||p*decay||^2 and sum g^2/(sqrt(diag)+eps). */
+/* Diagonal-mode params: ||g||^2, ||p*decay||^2 and sum g^2/(sqrt(diag)+eps).
+ * Here and in scao_diag_apply a task is chunk a of SCAO_FLAT_CHUNK elements, or
+ * with b = 1 .. 4 that quarter of it. */
 int scao_diag_reduce(const scao_task* tasks, int ntasks, const scao_param_desc* params,
                      double* slots, void* stream);
 /* phase 0: per param ||g||, ||p||, nu, clip; global grad-norm EMA in runtime[0]

@@ -18,12 +18,15 @@ using namespace scao;
 
 namespace {
 
-// element range of a flat task and this thread's 4 groups of 4 elements
+// element range of a flat task and this thread's 4 groups of 4 elements; with
+// b = 1 .. 4 the task is that quarter of the chunk (one group), which spreads
+// the long per-element chains of the diagonal kernels over more CUs
 struct Chunk {
   int64_t base, end;
   __device__ Chunk(const scao_task& tk, int64_t numel) {
-    base = (int64_t)tk.a * SCAO_FLAT_CHUNK;
-    end = base + SCAO_FLAT_CHUNK < numel ? base + SCAO_FLAT_CHUNK : numel;
+    base = (int64_t)tk.a * SCAO_FLAT_CHUNK + (tk.b ? (tk.b - 1) * (SCAO_FLAT_CHUNK / 4) : 0);
+    end = base + (tk.b ? SCAO_FLAT_CHUNK / 4 : SCAO_FLAT_CHUNK);
+    end = end < numel ? end : numel;
   }
   __device__ int64_t elem(int grp) const { return base + grp * 1024 + threadIdx.x * 4; }
   __device__ int mask(int64_t e) const {

@@ -248,6 +248,7 @@ _TASK_TYPES = (["adam", "dpart", "delta", "lift", "dred", "dapply", "lars"] +
                [f"apply{v}" for v in sorted({*range(64), *_APPLY_VARIANTS})])
 
 
+DIAG_SPLIT_CHUNKS = 64         # 1-D parameters up to this many chunks take quarter tasks
 STEP_WIDTHS = (64, 128, 256)   # eigenfactor widths the step kernels are built for
 
 
@@ -341,12 +342,18 @@ def _param_tasks(it: PItem, plan: SplitPlan):
             slot += 1
         rng = (0, slot, slot, slot)
     elif it.diag:
-        for c in range(_flat_chunks(it.p.numel())):
-            add("dred", (0, c, 0, slot))
+        # up to a few chunks: quarters, each a task (Chunk in elementwise.hip)
+        n, chunks = it.p.numel(), _flat_chunks(it.p.numel())
+        quarter = L.FLAT_CHUNK // 4
+        parts = ([(c, q + 1) for c in range(chunks) for q in range(4)
+                  if c * L.FLAT_CHUNK + q * quarter < n] if chunks <= DIAG_SPLIT_CHUNKS
+                 else [(c, 0) for c in range(chunks)])
+        for c, q in parts:
+            add("dred", (0, c, q, slot))
             slot += 1
         pre_end = slot
-        for c in range(_flat_chunks(it.p.numel())):
-            add("dapply", (0, c, 0, slot))
+        for c, q in parts:
+            add("dapply", (0, c, q, slot))
             slot += 1
         rng = (0, pre_end, pre_end, slot)
     else:
