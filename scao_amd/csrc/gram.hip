@@ -671,7 +671,7 @@ __device__ __forceinline__ void wave_lds_order() {
 //     each.  A group of one takes one exchange.
 // The time is the groups' LDS round trips: a few dozen groups for int8 EMAs
 // (the codes of their diagonals), up to one per row for fp32 EMAs.  2048 rows
-// with some 20 distinct codes (13 factors): 1596 us a step at a time -> 287 us.
+// with some 20 distinct codes (13 factors): 1596 us a step at a time -> 113 us.
 constexpr int ED_T = 1024;
 constexpr int ED_WORDS = (DIAG_MAX + 31) / 32;   // mask words
 
@@ -709,14 +709,28 @@ __global__ __launch_bounds__(ED_T) void k_eig_diag(const scao_prep_desc* __restr
   block_sum_n<1, ED_T>(acc, red);
   if (tid == 0) total[f] = acc[0];
   if (!__syncthreads_or(nan)) {   // a NaN has no order: the rows stay in place
-    // rank of each value: smaller ones, and equal ones of earlier rows
+    // rank of each value: smaller ones, and equal ones of earlier rows.  A
+    // wave's 64 rows start at wb; rows before them count by <=, rows after them
+    // by <, so only those 64 need the row compared too.
     for (int i = tid; i < n; i += ED_T) {
       const float y = val[i];
+      const int wb = __builtin_amdgcn_readfirstlane(i), we = min(wb + 64, (n + 3) & ~3);
       int r = 0;
-      for (int j = 0; j < n; j += 4) {
+      for (int j = 0; j < wb; j += 4) {
+        const v4f x = *(const v4f*)&val[j];
+#pragma unroll
+        for (int t = 0; t < 4; ++t) r += x[t] <= y;
+      }
+      for (int j = wb; j < we; j += 4) {
         const v4f x = *(const v4f*)&val[j];
 #pragma unroll
         for (int t = 0; t < 4; ++t) r += x[t] < y || (x[t] == y && j + t < i);
+      }
+#pragma unroll 4
+      for (int j = we; j < n; j += 4) {
+        const v4f x = *(const v4f*)&val[j];
+#pragma unroll
+        for (int t = 0; t < 4; ++t) r += x[t] < y;
       }
       ord[r] = (uint16_t)i;
       sv[r] = y;
