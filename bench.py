@@ -557,7 +557,7 @@ def mfma_summary(counter_csv: str, stats_csv: str, config: str, cmd: str) -> str
                    f"| {tf:.1f} | {tf / 157.3:.2f} |")
     out += ["", "Notes.  `k_gram_ema`'s average duration includes the run's first, cold refresh "
             "(the refresh summary gives the steady per-refresh time); it computes the lower tiles "
-            "of each symmetric Gram only.  `k_project_x6` does exactly 2mnk fp32-equivalent flops "
+            "of each symmetric Gram only.  `k_project` does exactly 2mnk fp32-equivalent flops "
             "per step (six bf16 products each) and also streams p for the LARS norm.  `k_apply` "
             "runs the back-projection's MFMAs under its streaming pass (HBM-bound).  "
             "`k_sy2sb_update_vec` is the refresh's lower-triangle band-reduction pass."]

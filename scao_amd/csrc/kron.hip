@@ -49,7 +49,7 @@ namespace {
 // from the loaded registers (every element passes through exactly one lane).
 //
 // EDGE: the strip may end past column n and the rows past i_end (those count
-// as zero); every load is masked and G may have any of the three types (dt).
+// as zero); every load is masked and G has type DT.
 // KEDGE: c0 + CR may lie past k, so U_l's loads and T's stores are masked.
 // Loads need element alignment only, in every form.
 //
