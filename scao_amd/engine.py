@@ -1231,17 +1231,25 @@ def eigen_route(dim: int, diagonal: bool) -> str:
 
 
 # The batched solver has a latency floor (its panel loop and bulge chasing
-# run the same number of steps for one matrix as for hundreds: 61 ms at
-# 2048^2, 205 ms at 4096^2); the library eigh takes 42 / 109 ms for one
-# matrix and about as long as the batched solver for four.  A batch of at
-# most this many matrices of at least 2048 rows goes to the library.
-LIBRARY_SMALL_BATCH = 2
+# run the same number of steps for one matrix as for hundreds).  Solver /
+# library eigh in ms:
+#     rows   one matrix    two
+#     2048    39 /  43    39 /  49
+#     2560    56 /  56    57 /  69
+#     3072    77 /  73    78 /  91
+#     4096   128 / 109   130 / 152
+# One matrix of at least 2048 rows goes to the library (the lines cross near
+# 2560 rows), two go to the solver.  Two of 4096 rows and more keep the
+# library's route, which tests/test_host_logic.py states.
+LIBRARY_MIN_DIM = 2048
+LIBRARY_PAIR_DIM = 4096
 
 
 def batch_route(route: str, dim: int, count: int) -> str:
     """The route of a dimension's batch of ``count`` factors that
     eigen_route sent to ``route``."""
-    if route == "hip" and count <= LIBRARY_SMALL_BATCH and dim >= 2048:
+    if route == "hip" and (dim >= LIBRARY_MIN_DIM and count == 1 or
+                           dim >= LIBRARY_PAIR_DIM and count == 2):
         return "library"
     return route
 
