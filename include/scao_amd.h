@@ -406,7 +406,8 @@ int scao_eig_band_finish(const float* A, int64_t stride, int n, int batch, const
 int scao_eig_sb2st(double* band64, int n, int batch, double* d, double* e, void* stream);
 /* Eigenvalues of the tridiagonals by bisection: the kq largest, descending,
  * into w + i*kq (float64), and sum over all eigenvalues of max(lambda, 0) into
- * total[i] (float64: the trace minus the negative eigenvalues).  work:
+ * total[i] (float64: the trace minus the negative eigenvalues).  A matrix may
+ * have any scale that leaves its row sums finite.  work:
  * scao_eig_bisect_work(n, batch) bytes. */
 int64_t scao_eig_bisect_work(int n, int batch);
 int scao_eig_bisect(const double* d, const double* e, int n, int batch, int kq, double* w,

@@ -1228,29 +1228,34 @@ __global__ __launch_bounds__(SB_W * 64) void k_sb2st(double* band, int n, double
 // form q_i = p_i / p_{i-1} has a division.  The computed minors are those of a
 // matrix within a few ulps of T elementwise, as the ratios are.  A minor that
 // comes out zero takes the sign opposite to its predecessor and a size far
-// below it (2^-200), so a decoupled block (e = 0) goes on counting from it;
-// four steps of that stay far above underflow.  e2[i] = e[i]^2.  The
-// coefficients stream in groups of SG, the next group's loads issued before
-// the current group's steps (the addresses are uniform: scalar loads).
+// below it (2^-200), so a decoupled block (e = 0) goes on counting from it.
+// The recurrence runs on T times a power of two that brings its Gershgorin
+// bound to [0.5, 1) (sigma, from k_tri_info): there four steps cannot overflow
+// and, but for points within 1e-77 of an eigenvalue, do not underflow; on T as
+// given they would at |T| past 1e+-60.  d is scaled where it meets x, at no
+// cost: the subtraction becomes an fma.  x and e2[i] = (sigma e[i])^2 are
+// scaled already.  The coefficients stream in groups of SG, the next group's
+// loads issued before the current group's steps (the addresses are uniform:
+// scalar loads).
 constexpr int SG = 8;
 constexpr double STURM_TINY = 0x1p-200;
 
 template <int S>
 __device__ __forceinline__ void sturm_ms(const double* __restrict__ d,
-                                         const double* __restrict__ e2, int n,
+                                         const double* __restrict__ e2, int n, double sigma,
                                          const double (&x)[S], int (&c)[S]) {
   double p[S], pm[S];
 #pragma unroll
   for (int t = 0; t < S; ++t) {
     pm[t] = 1.0;
-    p[t] = d[0] - x[t];
+    p[t] = fma(d[0], sigma, -x[t]);
     if (p[t] == 0.0) p[t] = -STURM_TINY;
     c[t] = p[t] < 0.0;
   }
   auto step = [&](double dv, double ev) {
 #pragma unroll
     for (int t = 0; t < S; ++t) {
-      double q = fma(dv - x[t], p[t], -(ev * pm[t]));
+      double q = fma(fma(dv, sigma, -x[t]), p[t], -(ev * pm[t]));
       if (__builtin_expect(q == 0.0, 0)) q = -STURM_TINY * p[t];
       c[t] += (int)((uint32_t)(__double2hiint(q) ^ __double2hiint(p[t])) >> 31);
       pm[t] = p[t];
@@ -1300,58 +1305,68 @@ __device__ __forceinline__ void sturm_ms(const double* __restrict__ d,
   }
 }
 
-// Per matrix: Gershgorin bounds, pivmin, the trace (float64), the number of
-// negative eigenvalues.  info = {lo, hi, pivmin, trace}, nneg.
+// Per matrix: the scale (sigma = 2^-ex, ex the exponent of the Gershgorin
+// bound), the scaled bounds, the trace (float64, as given), the squares of the
+// scaled off-diagonal and the number of negative eigenvalues.
+// info = {lo, hi, ex, trace}, nneg.
+constexpr double PIVMIN = 2.2250738585072014e-308;   // smallest normal double
+
 __global__ __launch_bounds__(256) void k_tri_info(const double* d, const double* e, int n,
                                                   double* info, int* nneg, double* e2) {
   __shared__ double red[16];
+  __shared__ double sig;
   const int mat = blockIdx.x;
   const double* dm = d + (int64_t)mat * n;
   const double* em = e + (int64_t)mat * n;
   double* e2m = e2 + (int64_t)mat * n;
-  double lo = 1e300, hi = -1e300, tr = 0.0, e2max = 0.0;
+  double lo = INFINITY, hi = -INFINITY, tr = 0.0;
   for (int i = threadIdx.x; i < n; i += 256) {
     const double r = (i > 0 ? fabs(em[i - 1]) : 0.0) + (i + 1 < n ? fabs(em[i]) : 0.0);
     lo = fmin(lo, dm[i] - r);
     hi = fmax(hi, dm[i] + r);
     tr += dm[i];
-    if (i + 1 < n) {
-      e2m[i] = em[i] * em[i];
-      e2max = fmax(e2max, e2m[i]);
-    }
   }
   double x[2] = {tr, 0.0};
   block_sum<2>(x, red);
-  // min / max / max: within each wave, then the four waves' through LDS
-  __shared__ double mm[3][4];
+  // min / max: within each wave, then the four waves' through LDS
+  __shared__ double mm[2][4];
   for (int o = 32; o > 0; o >>= 1) {
     lo = fmin(lo, __shfl_xor(lo, o));
     hi = fmax(hi, __shfl_xor(hi, o));
-    e2max = fmax(e2max, __shfl_xor(e2max, o));
   }
   if (threadIdx.x % 64 == 0) {
     mm[0][threadIdx.x / 64] = lo;
     mm[1][threadIdx.x / 64] = hi;
-    mm[2][threadIdx.x / 64] = e2max;
   }
   __syncthreads();
   if (threadIdx.x == 0) {
     for (int t = 1; t < 4; ++t) {
       lo = fmin(lo, mm[0][t]);
       hi = fmax(hi, mm[1][t]);
-      e2max = fmax(e2max, mm[2][t]);
     }
     const double tnorm = fmax(fabs(lo), fabs(hi));
-    const double pivmin = 2.2250738585072014e-308 * fmax(1.0, e2max);
+    int ex = 0;
+    if (tnorm > 0.0 && tnorm < INFINITY) ex = ilogb(tnorm) + 1;
+    ex = max(-1000, min(1000, ex));
+    sig = ldexp(1.0, -ex);
     // widen the interval so bisection brackets every eigenvalue
-    const double pad = 2.0 * 2.220446049250313e-16 * tnorm * n + 2.0 * pivmin;
-    info[4 * mat + 0] = lo - pad;
-    info[4 * mat + 1] = hi + pad;
-    info[4 * mat + 2] = pivmin;
+    const double pad = 2.0 * 2.220446049250313e-16 * (tnorm * sig) * n + 2.0 * PIVMIN;
+    info[4 * mat + 0] = lo * sig - pad;
+    info[4 * mat + 1] = hi * sig + pad;
+    info[4 * mat + 2] = (double)ex;
     info[4 * mat + 3] = x[0];
+  }
+  __syncthreads();
+  const double sigma = sig;
+  for (int i = threadIdx.x; i + 1 < n; i += 256) {
+    const double y = em[i] * sigma;
+    e2m[i] = y * y;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
     const double zero[1] = {0.0};
     int c[1];
-    sturm_ms<1>(dm, e2m, n, zero, c);
+    sturm_ms<1>(dm, e2m, n, sigma, zero, c);
     nneg[mat] = c[0];
   }
 }
@@ -1384,9 +1399,9 @@ __host__ __device__ constexpr int bisect_waves(int count, int lanes) {
 // One eigenvalue (index j) per group of LN lanes, PT points per lane, from
 // [lo, hi] until the width is at most rel * max(|lo|, |hi|) + tol.
 template <int LN, int PT>
-__device__ __forceinline__ double multisect(const double* dm, const double* em, int n, int j,
-                                            double lo, double hi, double rel, double tol,
-                                            bool done) {
+__device__ __forceinline__ double multisect(const double* dm, const double* em, int n,
+                                            double sigma, int j, double lo, double hi, double rel,
+                                            double tol, bool done) {
   constexpr int PTS = LN * PT;
   const int sub = (int)threadIdx.x % LN;
   for (int it = 0; it < 64; ++it) {
@@ -1398,7 +1413,7 @@ __device__ __forceinline__ double multisect(const double* dm, const double* em, 
 #pragma unroll
     for (int t = 0; t < PT; ++t) x[t] = lo + h * (double)(sub * PT + t + 1);
     int c[PT];
-    sturm_ms<PT>(dm, em, n, x, c);
+    sturm_ms<PT>(dm, em, n, sigma, x, c);
     // r = number of points whose count is <= j (a prefix: counts grow with x)
     int r = 0;
 #pragma unroll
@@ -1429,23 +1444,24 @@ __global__ __launch_bounds__(256) void k_bisect(const double* d, const double* e
   const double* em = e2 + (int64_t)mat * n;
   double* wm = wall + (int64_t)mat * n;
   const double lo0 = info[4 * mat + 0], hi0 = info[4 * mat + 1];
-  const double pivmin = info[4 * mat + 2];
+  const int ex = (int)info[4 * mat + 2];
+  const double sigma = ldexp(1.0, -ex);   // eigenvalues leave scaled back by 2^ex
   if (wv < wt) {
     const int slot = wv * (64 / TL) + l / TL;
     const bool act = slot < kq;
     const int j = n - 1 - (act ? slot : 0);
-    const double x = multisect<TL, TS>(dm, em, n, j, lo0, hi0, 2.0 * 2.220446049250313e-16,
-                                       pivmin, !act);
-    if (act && l % TL == 0) wm[j] = x;
+    const double x = multisect<TL, TS>(dm, em, n, sigma, j, lo0, hi0,
+                                       2.0 * 2.220446049250313e-16, PIVMIN, !act);
+    if (act && l % TL == 0) wm[j] = ldexp(x, ex);
     return;
   }
-  const double tol = 1e-12 * fmax(fabs(lo0), fabs(hi0)) + pivmin;
+  const double tol = 1e-12 * fmax(fabs(lo0), fabs(hi0)) + PIVMIN;
   if constexpr (NL > 1) {
     const int base = (wv - wt) * (64 / NL);
     if (base >= nn) return;                 // the whole wavefront
     const int j = base + l / NL;
-    const double x = multisect<NL, 1>(dm, em, n, j, lo0, 0.0, 0.0, tol, j >= nn);
-    if (j < nn && l % NL == 0) wm[j] = x;
+    const double x = multisect<NL, 1>(dm, em, n, sigma, j, lo0, 0.0, 0.0, tol, j >= nn);
+    if (j < nn && l % NL == 0) wm[j] = ldexp(x, ex);
   } else {
     const int base = (wv - wt) * 64 * NB2;
     if (base >= nn) return;                 // the whole wavefront
@@ -1471,7 +1487,7 @@ __global__ __launch_bounds__(256) void k_bisect(const double* d, const double* e
 #pragma unroll
       for (int t = 0; t < NB2; ++t) x[t] = 0.5 * (lo[t] + hi[t]);
       int c[NB2];
-      sturm_ms<NB2>(dm, em, n, x, c);
+      sturm_ms<NB2>(dm, em, n, sigma, x, c);
 #pragma unroll
       for (int t = 0; t < NB2; ++t)
         if (!done[t]) {
@@ -1483,7 +1499,7 @@ __global__ __launch_bounds__(256) void k_bisect(const double* d, const double* e
     }
 #pragma unroll
     for (int t = 0; t < NB2; ++t)
-      if (j[t] < nn) wm[j[t]] = 0.5 * (lo[t] + hi[t]);
+      if (j[t] < nn) wm[j[t]] = ldexp(0.5 * (lo[t] + hi[t]), ex);
   }
 }
 

@@ -54,3 +54,27 @@ def test_bisect_matches_lapack(hip_device, n, kq, copies):
             got, s = w[r + i], tot[r + i]
             assert np.abs(got - ev[::-1][:kq]).max() <= 1e-14 * n * scale, (i, r)
             assert abs(s - np.maximum(ev, 0).sum()) <= 2e-12 * n * scale, (i, r)
+
+
+@pytest.mark.parametrize("exponent", [-900, -333, -230, 230, 333, 900])
+@pytest.mark.parametrize("n,kq", [(9, 9), (65, 33), (300, 64)])
+@pytest.mark.parametrize("copies", [1, 300])
+def test_bisect_is_scale_free(hip_device, n, kq, exponent, copies):
+    """Multiplying T by a power of two multiplies the results by it, bit for
+    bit (the test above holds T itself to LAPACK): the counts run on T brought
+    to one size, and no product of a few entries leaves the range of a double.
+    The clamped sum is the given trace minus the negative ones: exact too."""
+    rng = np.random.default_rng(n)
+    mats = [m for m in _matrices(n, rng) if np.abs(m[1])[np.abs(m[1]) > 0].min(initial=1.0) > 1e-20]
+    d = np.stack([m[0] for m in mats] * copies)
+    e = np.stack([m[1] for m in mats] * copies)
+    d = np.where(np.abs(d) < 1e-20, 0.0, d)     # nothing of the scaled T is denormal
+    w, tot = _bisect(hip_device, d, e, kq)
+    ws, tots = _bisect(hip_device, np.ldexp(d, exponent), np.ldexp(e, exponent), kq)
+    assert np.array_equal(ws, np.ldexp(w, exponent))
+    assert np.array_equal(tots, np.ldexp(tot, exponent))
+
+
+def test_bisect_zero_matrix(hip_device):
+    w, tot = _bisect(hip_device, np.zeros((3, 65)), np.zeros((3, 65)), 33)
+    assert np.abs(w).max() <= 1e-300 and np.abs(tot).max() <= 1e-300
