@@ -1111,14 +1111,19 @@ __global__ __launch_bounds__(SB_W * 64) void k_sb2st(double* band, int n, double
         // scale = 1 / (alpha - beta), from Newton-refined reciprocal roots (a few
         // ulps; a square root and two divisions are twice the instructions: 13
         // matrices of 2048 rows 27.2 -> 26.5 ms).
-        // Below 1e-300 (entries under 1e-150 of an fp32 matrix's) nothing is
-        // left to annihilate.
+        // Where |x|^2 nears the smallest normal double the estimates' refinement
+        // has no range left: those take the plain forms (a band at 1e-150 and
+        // less; no fp32-born one).
         double tau = 0.0, beta = alpha, scale = 0.0;
         if (s2 > 1e-300) {
           const double h = fma(alpha, alpha, s2), r = rsqrt_d(h), nx = h * r;
           beta = -copysign(nx, alpha);
           tau = fma(fabs(alpha), r, 1.0);
           scale = copysign(recip_d(fabs(alpha) + nx), alpha);
+        } else if (__builtin_expect(s2 > 0.0, 0)) {
+          beta = -copysign(sqrt(fma(alpha, alpha, s2)), alpha);
+          tau = (beta - alpha) / beta;
+          scale = 1.0 / (alpha - beta);
         }
         wave_sync();
         if (l < NB) {
