@@ -2406,7 +2406,8 @@ extern "C" int scao_kron_apply(const scao_task* tasks, int ntasks, const scao_le
   SCAO_CHECK_ARG(tasks && leaves && params && stat && slots, "scao_kron_apply: null pointer");
   const bool half = variant & 64, mask = variant & 128;
   SCAO_CHECK_ARG(variant >= 0 && variant < 256 && ((variant & ~3) == 0 || (variant & 4)) &&
-                     !(half && (variant & 8)) && (!mask || (variant & 17) == 17),
+                     !(half && (variant & 8)) && (!mask || (variant & 17) == 17) &&
+                     (!(variant & 32) || (variant & 24)),
                  "scao_kron_apply: bad variant %d", variant);
   hipStream_t s = (hipStream_t)stream;
   if (variant & 16) {
@@ -2455,7 +2456,8 @@ extern "C" int scao_kron_apply(const scao_task* tasks, int ntasks, const scao_le
     case 68: SCAO_APPLY(false, false, true, true); break;
     case 69: SCAO_APPLY(true, false, true, true); break;
     case 70: SCAO_APPLY(false, true, true, true); break;
-    default: SCAO_APPLY(true, true, true, true); break;
+    case 71: SCAO_APPLY(true, true, true, true); break;
+    default: SCAO_CHECK_ARG(false, "scao_kron_apply: bad variant %d", variant);
   }
 #undef SCAO_APPLY
   SCAO_LAUNCH_CHECK("scao_kron_apply");

@@ -160,3 +160,16 @@ def test_entry_point_rejects_bad_arguments(name):
     lib = L.lib()
     assert getattr(lib, name)(*BAD_ARGS[name]) == 1
     assert lib.scao_last_error().decode().startswith(name + ":")
+
+
+@pytest.mark.parametrize("variant", [*range(36, 40), *range(100, 104), *range(8, 12), 76, 128, 132,
+                                     256])
+def test_kron_apply_rejects_variants_it_does_not_have(variant):
+    """Bit 32 (the strip's k = 128) without the strip's bit, and the forms
+    that no kernel serves: refused before any launch (one of them used to
+    reach the 16-bit kernel with an fp32 parameter)."""
+    from scao_amd import _lib as L
+    lib = L.lib()
+    p = 16   # non-null dummies: nothing is launched
+    assert lib.scao_kron_apply(p, 1, p, p, p, p, variant, None) == 1
+    assert b"bad variant" in lib.scao_last_error()
