@@ -168,9 +168,11 @@ int scao_struct_layout(int which, int64_t* out, int cap);
 
 /* ---- reference operator surface ------------------------------------- */
 /* out = G + U_l ((s_l s_r^T - 1) * (U_l^T G U_r)) U_r^T   (m x n, k <= 256).
- * G has row stride ldG; out is dense m x n.  workspace: k*n + k*k + m*k
- * floats + 4 leaf/task descriptors worth of bytes given by
- * scao_fused_kronecker_workspace(). */
+ * G has row stride ldG; out is dense m x n and also holds partial sums until
+ * the last stage writes it, unless it shares storage with G (in place: out ==
+ * G, ldG == n), U_l, s_l_inv4 or s_r_inv4, which it may; it must not overlap
+ * U_r or the workspace.  workspace: scao_fused_kronecker_workspace() bytes
+ * (k*n + k*k + m*k floats). */
 /* <- scao.cuda.low_rank_precond_mm (scao/cuda/__init__.py:190-228; kernels
  * scao/cuda/low_rank_ops.cu:239-296).  left != 0: out = (U*s) (U^T G) with U
  * m x k; left == 0: out = (G (U*s)) U^T with U n x k; G and out m x n, all

@@ -2471,8 +2471,9 @@ extern "C" int64_t scao_fused_kronecker_workspace(int64_t m, int64_t n, int64_t 
 
 namespace {
 
-// The four launches of the reference operator over one block, with the
-// block's T, Delta and W in the k*n + k*k + m*k floats at ws.
+// The launches of the reference operator over one block (project, delta in one
+// or two, lift, apply), with the block's T, Delta and W in the k*n + k*k + m*k
+// floats at ws.
 int launch_fused_kronecker(const float* U_l, const float* s_l_inv4, const float* U_r,
                            const float* s_r_inv4, const float* G, int64_t ldG, float* out,
                            int64_t m, int64_t n, int64_t k, float* ws, hipStream_t s) {
@@ -2499,15 +2500,19 @@ int launch_fused_kronecker(const float* U_l, const float* s_l_inv4, const float*
   // (at least 128 per part, up to a workgroup per CU) and P is formed by column
   // chunks.  Their planes of T and P live in `out`, which the last launch
   // overwrites, so the scratch stays T, Delta and W.  An `out` that shares
-  // storage with G or has no room for the planes takes fewer parts or none.
+  // storage with G, U_l, s_l or s_r, which are still read while the planes are
+  // written, or has no room for the planes takes fewer parts or none.
   // 2048 x 2048 at k = 64: projection 337 -> 13 us, P 69 -> 24 us.
   const int64_t strips = (n + SCAO_PROJ_COLS - 1) / SCAO_PROJ_COLS;
   const int cr = k > 128 ? 256 : k > 64 ? 128 : 64;
   const int64_t kt = (k + cr - 1) / cr, pt = (k + 63) / 64;
   const int64_t tp = plane_floats(k * n), pp = plane_floats(k * k);
   int64_t chunks = (n + delta_cols((int)k) - 1) / delta_cols((int)k);
-  const bool apart = (uintptr_t)out >= (uintptr_t)(G + (m - 1) * ldG + n) ||
-                     (uintptr_t)(out + m * n) <= (uintptr_t)G;
+  auto clear_of_out = [&](const float* p, int64_t floats) {
+    return (uintptr_t)out >= (uintptr_t)(p + floats) || (uintptr_t)(out + m * n) <= (uintptr_t)p;
+  };
+  const bool apart = clear_of_out(G, (m - 1) * ldG + n) && clear_of_out(U_l, m * k) &&
+                     clear_of_out(s_l_inv4, k) && clear_of_out(s_r_inv4, k);
   const int64_t room = apart ? m * n : 0;
   if (chunks > 255 || chunks * pp > room) chunks = 0;
   int64_t parts = 1;

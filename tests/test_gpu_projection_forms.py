@@ -52,6 +52,37 @@ def test_fused_operator_forms(hip_device, m, n, k, ld, inplace):
     assert err < 2e-5, err
 
 
+@pytest.mark.parametrize("noalloc", [False, True])
+@pytest.mark.parametrize("shared", ["U_l", "s_l", "s_r"])
+@pytest.mark.parametrize("m,n,k", [(512, 512, 64), (1000, 513, 100)])
+def test_fused_operator_out_shares_an_operand(hip_device, m, n, k, shared, noalloc):
+    """An out that takes the storage of an operand that only the first stages
+    read, at its first and at its last floats: no partial sums go there while
+    the operand is still read.  Tolerance as above."""
+    from scao_amd import _lib as L
+    g = torch.Generator().manual_seed(m + k)
+    ops = dict(U_l=_rand(g, m, k) / m ** 0.5, s_l=torch.rand(k, generator=g) * 3 + 0.1,
+               U_r=_rand(g, n, k) / n ** 0.5, s_r=torch.rand(k, generator=g) * 3 + 0.1,
+               G=_rand(g, m, n))
+    a, b, x = ops["U_l"].double(), ops["U_r"].double(), ops["G"].double()
+    f = ops["s_l"].double()[:, None] * ops["s_r"].double() - 1.0
+    want = x + a @ (f * (a.T @ x @ b)) @ b.T
+    scale = x.abs() + a.abs() @ (f.abs() * (a.abs().T @ x.abs() @ b.abs())) @ b.abs().T
+    for at_end in (False, True):
+        dev = {name: t.to(hip_device) for name, t in ops.items()}
+        out = torch.empty(m, n, device=hip_device)
+        t = dev[shared]
+        part = out.view(-1)[-t.numel():] if at_end else out.view(-1)[:t.numel()]
+        dev[shared] = part.view(t.shape).copy_(t)
+        ptrs = [dev[name].data_ptr() for name in ("U_l", "s_l", "U_r", "s_r", "G")]
+        ws = torch.empty(L.lib().scao_fused_kronecker_workspace(m, n, k) // 4, device=hip_device)
+        name = "scao_fused_kronecker_precond" + ("_noalloc" if noalloc else "")
+        L.call(name, *ptrs, n, out.data_ptr(), m, n, k, *([] if noalloc else [ws.data_ptr()]),
+               L.stream_ptr(hip_device))
+        err = ((out.cpu().double() - want).abs() / scale).max().item()
+        assert err < 2e-5, (shared, at_end, err)
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("shapes,k", [([(96, 300), (257, 511)], 64), ([(1000, 1537)], 40),
                                       ([(640, 768), (129, 257)], 128), ([(512, 520)], 256),
