@@ -38,7 +38,7 @@
 extern "C" {
 #endif
 
-#define SCAO_ABI_VERSION 13
+#define SCAO_ABI_VERSION 14
 
 enum scao_status { SCAO_OK = 0, SCAO_ERR_INVALID = 1, SCAO_ERR_HIP = 2 };
 enum scao_dtype { SCAO_F32 = 0, SCAO_BF16 = 1, SCAO_F16 = 2 };
@@ -229,11 +229,14 @@ int scao_int8_ema_update(int8_t* q, double scale_in, const float* new_val, doubl
 int scao_kron_project(const scao_task* tasks, int ntasks, const scao_leaf_desc* leaves,
                       const scao_param_desc* params, double* slots, int variant, void* stream);
 /* A2  P = T U_r, Delta = (s_l s_r^T - 1) P and nu^2 partial per 64x64 tile of P.
- *     A leaf with column chunks takes two launches: first, with slots NULL
- *     (params is not read), a task per chunk and 64x64 tile, (leaf, a, b +
- *     (chunk << 16)), each forming its share of the tile of P; then its tiles. */
+ *     The tiles of a leaf with column chunks (16 rows x 64 columns) add the
+ *     chunks' shares, which scao_kron_delta_part forms first: a task per chunk
+ *     and 64x64 tile, (leaf, a, b + (chunk << 16)); a chunk that the leaf does
+ *     not have is skipped. */
 int scao_kron_delta(const scao_task* tasks, int ntasks, const scao_leaf_desc* leaves,
                     const scao_param_desc* params, double* slots, void* stream);
+int scao_kron_delta_part(const scao_task* tasks, int ntasks, const scao_leaf_desc* leaves,
+                         void* stream);
 /* A3  W = U_l Delta per 64-row strip. */
 int scao_kron_lift(const scao_task* tasks, int ntasks, const scao_leaf_desc* leaves,
                    void* stream);

@@ -21,7 +21,7 @@ import torch  # noqa: F401  -- loads torch's HIP runtime before ours
 HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.environ.get("SCAO_AMD_LIB", os.path.join(HERE, "_lib", "libscao_amd.so"))
 
-ABI_VERSION = 13
+ABI_VERSION = 14
 SLOT_WIDTH = 3
 FLAT_CHUNK = 4096
 PROJ_COLS = 256
@@ -123,6 +123,7 @@ SIGNATURES = {
     "scao_int8_ema_update": (_I, [_VP, _D, _VP, _D, _I64, _VP, _VP, _VP]),
     "scao_kron_project": (_I, [_VP, _I, _VP, _VP, _VP, _I, _VP]),
     "scao_kron_delta": (_I, [_VP, _I, _VP, _VP, _VP, _VP]),
+    "scao_kron_delta_part": (_I, [_VP, _I, _VP, _VP]),
     "scao_kron_lift": (_I, [_VP, _I, _VP, _VP]),
     "scao_diag_reduce": (_I, [_VP, _I, _VP, _VP, _VP]),
     "scao_step_finalize": (_I, [_VP, _I, _VP, _VP, _VP, _I, _I, _I, _VP]),

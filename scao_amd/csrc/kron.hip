@@ -2215,6 +2215,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
   __shared__ __attribute__((aligned(16))) float Ts[64][TSP];
   const scao_task tk = tasks[blockIdx.x];
   const scao_leaf_desc L = leaves[tk.idx];
+  // a leaf without column chunks has no planes to write
+  if ((unsigned)(tk.b >> 16) >= (unsigned)SCAO_LF_GET_DCHUNK(L.flags)) return;
   delta_part(L, tk.a, tk.b & 0xffff, tk.b >> 16, L.T + plane_floats((int64_t)L.k * L.n),
              L.Delta + plane_floats((int64_t)L.k * L.k), Ts);
 }
@@ -2374,17 +2376,20 @@ extern "C" int scao_kron_delta(const scao_task* tasks, int ntasks, const scao_le
                                const scao_param_desc* params, double* slots, void* stream) {
   SCAO_CHECK_ARG(ntasks >= 0, "scao_kron_delta: ntasks < 0");
   if (ntasks == 0) return SCAO_OK;
-  SCAO_CHECK_ARG(tasks && leaves, "scao_kron_delta: null pointer");
-  if (!slots) {
-    hipLaunchKernelGGL(k_delta_part, dim3(ntasks), dim3(256), 0, (hipStream_t)stream, tasks,
-                       leaves);
-    SCAO_LAUNCH_CHECK("scao_kron_delta");
-    return SCAO_OK;
-  }
-  SCAO_CHECK_ARG(params, "scao_kron_delta: null pointer");
+  SCAO_CHECK_ARG(tasks && leaves && params && slots, "scao_kron_delta: null pointer");
   hipLaunchKernelGGL(k_delta, dim3(ntasks), dim3(256), 0, (hipStream_t)stream, tasks, leaves,
                      params, slots);
   SCAO_LAUNCH_CHECK("scao_kron_delta");
+  return SCAO_OK;
+}
+
+extern "C" int scao_kron_delta_part(const scao_task* tasks, int ntasks,
+                                    const scao_leaf_desc* leaves, void* stream) {
+  SCAO_CHECK_ARG(ntasks >= 0, "scao_kron_delta_part: ntasks < 0");
+  if (ntasks == 0) return SCAO_OK;
+  SCAO_CHECK_ARG(tasks && leaves, "scao_kron_delta_part: null pointer");
+  hipLaunchKernelGGL(k_delta_part, dim3(ntasks), dim3(256), 0, (hipStream_t)stream, tasks, leaves);
+  SCAO_LAUNCH_CHECK("scao_kron_delta_part");
   return SCAO_OK;
 }
 

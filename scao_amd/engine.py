@@ -986,7 +986,7 @@ def _launch_step(ws: Workspace, raw: np.ndarray, n: int, update_norm_ema: bool) 
         if N[f"proj{var}"]:
             _call("scao_kron_project", tp(f"proj{var}"), N[f"proj{var}"], LF, P, SL, var, s)
     if N["dpart"]:
-        _call("scao_kron_delta", tp("dpart"), N["dpart"], LF, 0, 0, s)
+        _call("scao_kron_delta_part", tp("dpart"), N["dpart"], LF, s)
     if N["delta"]:
         _call("scao_kron_delta", tp("delta"), N["delta"], LF, P, SL, s)
         _call("scao_kron_lift", tp("lift"), N["lift"], LF, s)

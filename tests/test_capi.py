@@ -121,6 +121,7 @@ BAD_ARGS = {
     "scao_int8_ema_update": (N, 1.0, N, 0.9, 4, N, N, N),
     "scao_kron_project": (N, -1, N, N, N, 1, N),
     "scao_kron_delta": (N, -1, N, N, N, N),
+    "scao_kron_delta_part": (N, -1, N, N),
     "scao_kron_lift": (N, -1, N, N),
     "scao_diag_reduce": (N, -1, N, N, N),
     "scao_step_finalize": (N, -1, N, N, N, 0, 0, 0, N),
@@ -173,3 +174,18 @@ def test_kron_apply_rejects_variants_it_does_not_have(variant):
     p = 16   # non-null dummies: nothing is launched
     assert lib.scao_kron_apply(p, 1, p, p, p, p, variant, None) == 1
     assert b"bad variant" in lib.scao_last_error()
+
+
+def test_kron_delta_needs_its_slots():
+    """A null pointer among the delta stage's tables is an error, not another
+    kernel."""
+    from scao_amd import _lib as L
+    lib = L.lib()
+    p = 16   # non-null dummies: nothing is launched
+    for args in ((0, p, p, p), (p, 0, p, p), (p, p, 0, p), (p, p, p, 0)):
+        tasks, leaves, params, slots = args
+        assert lib.scao_kron_delta(tasks, 1, leaves, params, slots, None) == 1
+        assert b"null pointer" in lib.scao_last_error()
+    for tasks, leaves in ((0, p), (p, 0)):
+        assert lib.scao_kron_delta_part(tasks, 1, leaves, None) == 1
+        assert b"null pointer" in lib.scao_last_error()
