@@ -242,7 +242,7 @@ int scao_kron_lift(const scao_task* tasks, int ntasks, const scao_leaf_desc* lea
                    void* stream);
 /* Diagonal-mode params: ||g||^2, ||p*decay||^2 and sum g^2/(sqrt(diag)+eps).
  * Here and in scao_diag_apply a task is chunk a of SCAO_FLAT_CHUNK elements, or
- * with b = 1 .. 4 that quarter of it. */
+ * with b = 1 .. 4 that quarter of it; the other flat kernels do not read b. */
 int scao_diag_reduce(const scao_task* tasks, int ntasks, const scao_param_desc* params,
                      double* slots, void* stream);
 /* phase 0: per param ||g||, ||p||, nu, clip; global grad-norm EMA in runtime[0]

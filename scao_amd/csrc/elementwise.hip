@@ -18,14 +18,15 @@ using namespace scao;
 
 namespace {
 
-// element range of a flat task and this thread's 4 groups of 4 elements; with
-// b = 1 .. 4 the task is that quarter of the chunk (one group), which spreads
-// the long per-element chains of the diagonal kernels over more CUs
+// element range of a flat task (chunk a; b is not read) and this thread's 4
+// groups of 4 elements; in a QuarterChunk b = 1 .. 4 makes it that quarter of
+// the chunk (one group), which spreads the long per-element chains of the
+// diagonal kernels over more CUs
 struct Chunk {
   int64_t base, end;
-  __device__ Chunk(const scao_task& tk, int64_t numel) {
-    base = (int64_t)tk.a * SCAO_FLAT_CHUNK + (tk.b ? (tk.b - 1) * (SCAO_FLAT_CHUNK / 4) : 0);
-    end = base + (tk.b ? SCAO_FLAT_CHUNK / 4 : SCAO_FLAT_CHUNK);
+  __device__ Chunk(const scao_task& tk, int64_t numel, int quarter = 0) {
+    base = (int64_t)tk.a * SCAO_FLAT_CHUNK + (quarter ? (quarter - 1) * (SCAO_FLAT_CHUNK / 4) : 0);
+    end = base + (quarter ? SCAO_FLAT_CHUNK / 4 : SCAO_FLAT_CHUNK);
     end = end < numel ? end : numel;
   }
   __device__ int64_t elem(int grp) const { return base + grp * 1024 + threadIdx.x * 4; }
@@ -34,6 +35,10 @@ struct Chunk {
     for (int t = 0; t < 4; ++t) mk |= (e + t < end) ? (1 << t) : 0;
     return mk;
   }
+};
+struct QuarterChunk : Chunk {
+  __device__ QuarterChunk(const scao_task& tk, int64_t numel)
+      : Chunk(tk, numel, tk.b >= 1 && tk.b <= 4 ? tk.b : 0) {}
 };
 
 __device__ __forceinline__ void write_slot(double* slots, int slot, double a, double b, double c) {
@@ -183,7 +188,7 @@ __global__ __launch_bounds__(256) void k_diag_reduce(const scao_task* __restrict
   const scao_task tk = tasks[blockIdx.x];
   const scao_param_desc& P = params[tk.idx];
   const int dt = P.dtype;
-  const Chunk ch(tk, P.numel);
+  const QuarterChunk ch(tk, P.numel);
   const bool decay = P.flags & SCAO_PF_DECAY;
   const bool lars = P.flags & SCAO_PF_LARS;
   double acc[3] = {0.0, 0.0, 0.0};
@@ -224,7 +229,7 @@ __global__ __launch_bounds__(256) void k_diag_apply(const scao_task* __restrict_
   const scao_param_desc& P = params[tk.idx];
   const scao_param_stat S = stat[tk.idx];
   const int dt = P.dtype;
-  const Chunk ch(tk, P.numel);
+  const QuarterChunk ch(tk, P.numel);
   double u2 = 0.0;
 #pragma unroll
   for (int grp = 0; grp < 4; ++grp) {

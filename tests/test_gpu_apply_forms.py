@@ -4,6 +4,7 @@ that start at any element) against the CPU oracle from the same state."""
 
 from __future__ import annotations
 
+import numpy as np
 import pytest
 import torch
 
@@ -101,3 +102,42 @@ def test_phase1_chunks_at_any_element(hip_device, dtype, numel, off):
     assert torch.equal(pa, pb)
     for key in ("exp_avg", "exp_avg_sq", "prev_grad"):
         assert torch.equal(oa.state[pa][key], ob.state[pb][key])
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("phase2", [False, True])
+def test_flat_tasks_do_not_read_b(hip_device, monkeypatch, dtype, phase2):
+    """The Adam and LARS-write tasks are whole chunks whatever their second
+    coordinate holds (a quarter's number is the diagonal kernels' alone): the
+    step equals, bit for bit, the one with zeros there."""
+    from scao_amd import engine as E
+    g = torch.Generator().manual_seed(5)
+    init = [(0.02 * torch.randn(*s, generator=g)).to(dtype).to(hip_device)
+            for s in ((4096 * 3 + 5,), (100, 130))]
+    grads = [(1e-3 * torch.randn(x.shape, generator=g)).to(dtype).to(hip_device) for x in init]
+    cfg = dict(warmup_steps=0 if phase2 else 100, min_precond_updates=0, precond_freq=10 ** 9,
+               sparsity=0.0, noise_std_init=0.0, lookahead_k=0, k_min=8, k_max=8)
+    plain = E._param_tasks
+
+    def marked(it, plan):
+        arrays, *rest = plain(it, plan)
+        arrays = {kind: arr.copy() for kind, arr in arrays.items()}
+        for kind in ("adam", "lars"):
+            if kind in arrays:
+                arrays[kind][:, 2] = 1 + np.arange(len(arrays[kind])) % 7
+        return (arrays, *rest)
+
+    def run():
+        ps = [torch.nn.Parameter(x.clone()) for x in init]
+        opt = scao_amd.SCAO(ps, **cfg)
+        for p, x in zip(ps, grads):
+            p.grad = x
+        opt.step()
+        torch.cuda.synchronize()
+        return [[p.detach()] + [opt.state[p][key] for key in
+                                ("exp_avg", "exp_avg_sq", "exp_avg_diff", "prev_grad")] for p in ps]
+
+    want = run()
+    monkeypatch.setattr(E, "_param_tasks", marked)
+    for a, b in zip(run(), want):
+        assert all(torch.equal(x, y) for x, y in zip(a, b))
