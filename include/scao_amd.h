@@ -247,8 +247,11 @@ int scao_diag_reduce(const scao_task* tasks, int ntasks, const scao_param_desc* 
                      double* slots, void* stream);
 /* phase 0: per param ||g||, ||p||, nu, clip; global grad-norm EMA in runtime[0]
  *          (runtime[1] receives the average) when update_norm_ema != 0.
- * phase 1: per param ||u||, LARS trust and the fp32 step multiplier; with
- *          update_norm_ema the global EMA here instead of in phase 0. */
+ * phase 1: per param ||u||, LARS trust and the fp32 step multiplier; and, when
+ *          update_norm_ema is SCAO_NORM_EMA_PHASE1, the global EMA: for a
+ *          caller that passed 0 in phase 0, it saves a launch.  (Any other
+ *          value is not read here.) */
+#define SCAO_NORM_EMA_PHASE1 2
 int scao_step_finalize(const scao_param_desc* params, int nparams, const double* slots,
                        scao_param_stat* stat, double* runtime, int phase,
                        int update_norm_ema, int norm_count, void* stream);

@@ -31,6 +31,7 @@ APPLY_WIDE_COLS = 256
 APPLY_GROUP = 8
 GRAM_TILE = 128
 LF_NSPLIT_SHIFT, LF_DCHUNK_SHIFT = 8, 16
+NORM_EMA_PHASE1 = 2
 NOALLOC_SCRATCH_BYTES = 16 << 20
 EIG_BAND = 16
 EIG_BANDW = 2 * EIG_BAND + 1

@@ -569,8 +569,9 @@ extern "C" int scao_step_finalize(const scao_param_desc* params, int nparams, co
   if (nparams == 0) return SCAO_OK;
   SCAO_CHECK_ARG(params && slots && stat, "scao_step_finalize: null pointer");
   hipStream_t s = (hipStream_t)stream;
-  SCAO_CHECK_ARG(!update_norm_ema || runtime != nullptr, "scao_step_finalize: null runtime");
-  const int with_global = phase == 1 && update_norm_ema ? 1 : 0;
+  const int with_global = phase == 1 && update_norm_ema == SCAO_NORM_EMA_PHASE1 ? 1 : 0;
+  SCAO_CHECK_ARG(runtime || !(with_global || (phase == 0 && update_norm_ema)),
+                 "scao_step_finalize: null runtime");
   hipLaunchKernelGGL(k_finalize_params, dim3(nparams + with_global), dim3(FIN_T), 0, s, params,
                      nparams, slots, stat, phase, runtime, norm_count);
   SCAO_LAUNCH_CHECK("scao_step_finalize");

@@ -1002,7 +1002,7 @@ def _launch_step(ws: Workspace, raw: np.ndarray, n: int, update_norm_ema: bool) 
     if N["dapply"]:
         _call("scao_diag_apply", tp("dapply"), N["dapply"], P, S, SL, s)
     if N["lars"]:
-        _call("scao_step_finalize", P, n, SL, S, R, 1, norm_ema, n, s)
+        _call("scao_step_finalize", P, n, SL, S, R, 1, norm_ema * L.NORM_EMA_PHASE1, n, s)
         _call("scao_lars_write", tp("lars"), N["lars"], P, S, s)
     ws.finish_params()
 

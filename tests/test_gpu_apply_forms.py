@@ -141,3 +141,33 @@ def test_flat_tasks_do_not_read_b(hip_device, monkeypatch, dtype, phase2):
     monkeypatch.setattr(E, "_param_tasks", marked)
     for a, b in zip(run(), want):
         assert all(torch.equal(x, y) for x, y in zip(a, b))
+
+
+def test_norm_average_is_taken_once(hip_device):
+    """scao_step_finalize's phase 1 takes the grad-norm average only when it is
+    asked for with SCAO_NORM_EMA_PHASE1: a caller that passes its flag to both
+    phases (and no runtime to the second) gets one update."""
+    from scao_amd import _lib as L
+    desc = np.zeros(1, dtype=L.PARAM_DESC)
+    desc["pre_end"] = desc["post_end"] = 1
+    desc["flags"] = L.PF_NORM
+    params = L.upload(desc, hip_device)
+    slots = torch.tensor([4.0, 1.0, 1.0], dtype=torch.float64, device=hip_device)   # ||g|| = 2
+    stat = torch.zeros(L.PARAM_STAT.itemsize, dtype=torch.uint8, device=hip_device)
+    runtime = torch.tensor([1.0, 0.0], dtype=torch.float64, device=hip_device)
+    s = L.stream_ptr(hip_device)
+
+    def finalize(rt, phase, flag):
+        L.call("scao_step_finalize", params.data_ptr(), 1, slots.data_ptr(), stat.data_ptr(), rt,
+               phase, flag, 1, s)
+        return runtime.tolist()
+
+    once = 0.95 * 1.0 + 0.05 * 2.0
+    assert finalize(runtime.data_ptr(), 0, 1) == [once, 2.0]
+    assert finalize(0, 1, 1) == [once, 2.0]
+    assert finalize(runtime.data_ptr(), 1, 1) == [once, 2.0]
+    assert finalize(runtime.data_ptr(), 1, L.NORM_EMA_PHASE1) == [0.95 * once + 0.05 * 2.0, 2.0]
+    with pytest.raises(L.ScaoLibError):
+        finalize(0, 1, L.NORM_EMA_PHASE1)
+    with pytest.raises(L.ScaoLibError):
+        finalize(0, 0, 1)
