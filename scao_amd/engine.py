@@ -132,6 +132,7 @@ class Workspace:
         self.nslots = 0
         self.leaf_dev = None
         self.leaf_index = {}
+        self.splits: list = []   # the blocks' _leaf_splits
         self.upd_offsets = {}
         # parameter-table staging: PARAM_RING slots of (pinned host buffer,
         # device buffer, event recorded after the step that last used them)
@@ -324,132 +325,195 @@ def _leaf_split(leaf, plan: SplitPlan) -> tuple:
     return parts, rows, chunks
 
 
-def _param_tasks(it: PItem, plan: SplitPlan):
+def _leaf_splits(leaves, plan: SplitPlan | None = None) -> list:
+    """_leaf_split of every block of a step, under the step's plan."""
+    if plan is None:
+        plan = _split_plan([lf for lf, *_ in leaves])
+    return [_leaf_split(lf, plan) for lf, *_ in leaves]
+
+
+def _rows(shape, a, b, slot) -> np.ndarray:
+    """Task rows (block 0, a, b, slot) over a grid, the last axis fastest."""
+    out = np.zeros((*shape, 4), dtype=np.int32)
+    out[..., 1], out[..., 2], out[..., 3] = a, b, slot
+    return out.reshape(-1, 4)
+
+
+def _grid(a, b, slot=None) -> np.ndarray:
+    """Task rows over a x b, b fastest; slots counted from ``slot`` or -1."""
+    shape = (len(a), len(b))
+    s = -1 if slot is None else slot + np.arange(shape[0] * shape[1]).reshape(shape)
+    return _rows(shape, a[:, None], b[None, :], s)
+
+
+def _proj_tasks(m, n, k, parts, rows, typed, half, lars):
+    """A block's projection tasks (c0 = 0 owns the norm slots): [(kind, rows)]
+    and the number of slots, one per strip and part."""
+    J, part = np.arange(0, n, L.PROJ_COLS), np.arange(parts)
+    nrows = np.minimum(rows, m - part * rows)
+    whole = ((J[:, None] + L.PROJ_COLS <= n) & (nrows % PROJ_CHUNK == 0)[None, :]
+             if typed else np.zeros((len(J), parts), bool))
+    out = []
+    # 128 or 256 rows of T per whole task where k allows (variant bits 4, 8)
+    cr = 256 if k % 256 == 0 else 128 if k % 128 == 0 else 64
+    for sel, height, var in ((whole, cr, 1 | (half << 4) | {64: 0, 128: 4, 256: 8}[cr]),
+                             (~whole, 64, 0)):
+        jj, pp = np.nonzero(sel)
+        if not len(jj):
+            continue
+        c = np.arange(0, k, height)
+        slots = jj * parts + pp
+        a, b = J[jj][:, None], c[None, :] | (pp[:, None] << 16)
+        if lars:
+            out.append((f"proj{var | 2}", _rows((len(jj), 1), a, b[:, :1], slots[:, None])))
+            if len(c) > 1:
+                out.append((f"proj{var}", _rows((len(jj), len(c) - 1), a, b[:, 1:], -1)))
+        else:
+            out.append((f"proj{var}", _rows(b.shape, a, b, np.where(c[None, :] == 0,
+                                                                    slots[:, None], -1))))
+    return out, len(J) * parts
+
+
+def _delta_tasks(m, n, k, chunks):
+    """A block's delta tasks (k = 0, a diagonal sub-block: its norm partials in
+    64x64 tiles; chunks: shares of P first, then tiles of 16 rows)."""
+    if k == 0:
+        t = _grid(np.arange(0, m, 64), np.arange(0, n, 64), 0)
+        return [("delta", t)], len(t)
+    B = np.arange(0, k, 64)
+    out = []
+    if chunks:
+        shape = (len(B), len(B), chunks)
+        ch = np.arange(chunks) << 16
+        out.append(("dpart", _rows(shape, B[None, :, None], B[:, None, None] | ch, -1)))
+    A = np.arange(0, k, 16 if chunks else 64)
+    t = _rows((len(B), len(A)), A[None, :], B[:, None],
+              np.arange(len(B) * len(A)).reshape(len(B), len(A)))
+    out.append(("delta", t))
+    return out, len(t)
+
+
+def _apply_tasks(m, n, k, fp32, half, var, masked):
+    """A block's lift and apply tasks: strip runs or wide tiles over the
+    interior they tile exactly, masked 64x64 tiles over the right column strip
+    and the bottom row strip."""
+    out = []
+    if k:
+        out.append(("lift", _grid(np.arange(0, m, 64), np.arange(0, k, 64))))
+    # 16-bit data has wide and strip tiles, but no pipelined ones
+    pipe = k >= PIPE_MIN_RANK and k not in STRIP_RANKS
+    ok = k and (fp32 or (half and not pipe))
+    typed = 64 if half else 0
+    strip = ok and k in STRIP_RANKS
+    if strip:
+        tr, sw = (128, 64) if k == 256 else (64, 128)   # the kernel's strip_shape
+    else:
+        tr, sw = L.APPLY_WIDE_ROWS, L.APPLY_WIDE_COLS
+    mw, nw = (m - m % tr, n - n % sw) if ok else (0, 0)
+    if not (mw and nw):
+        mw = nw = 0
+    slot = 0
+    if mw:
+        if strip:
+            wide = var | 4 | 16 | (32 if k == 128 else 0) | typed | (128 if masked else 0)
+            t = np.array(_strip_runs(mw, nw, tr, sw))
+            tiles = np.minimum(L.APPLY_GROUP, (mw - t[:, 0]) // tr)
+        else:
+            wide = var | 4 | (8 if pipe else typed)
+            t = np.array(_wide_tiles(mw, nw, k, pipe))
+            tiles = np.ones(len(t), dtype=np.int64)
+        out.append((f"apply{wide}", _rows((len(t),), t[:, 0], t[:, 1], np.cumsum(tiles) - tiles)))
+        slot = int(tiles.sum())
+    T = L.APPLY_TILE
+    for i0, j0, j1 in ((0, nw, n), (mw, 0, nw)):
+        a, b = np.arange(i0, m, T), np.arange(j0, j1, T)
+        if len(a) and len(b):
+            out.append((f"apply{var}", _grid(a, b, slot)))
+            slot += len(a) * len(b)
+    return out, slot
+
+
+def _flat_tasks(chunks: np.ndarray, quarters, slot) -> np.ndarray:
+    """Flat tasks (parameter 0, chunk, quarter, slot) of a parameter."""
+    return _rows((len(chunks),), chunks, quarters, slot)
+
+
+def _param_tasks(it: PItem, plan: SplitPlan, made: dict):
     """One parameter's share of a step structure, with local indices: block
     indices from 0 (first block of the parameter), parameter index 0, slots
     from 0.  Returns ({type: int32 array (n, 4)}, local slot ranges, slot
-    count, [(leaf, r0, c0)])."""
-    tasks = {}
-
-    def add(kind, t):
-        tasks.setdefault(kind, []).append(t)
-
+    count, [(leaf, r0, c0)]).  Rows are made a block at a time, by array
+    arithmetic (a step has thousands), and once per geometry (``made``): the
+    blocks of a parameter, and of a model's layers, are of a few sizes only."""
+    tasks = {}   # kind -> ([rows], [block], [first slot])
     slot = 0
+
+    def block(fn, *key):
+        got = made.get((fn, key))
+        if got is None:
+            got = made[fn, key] = fn(*key)
+        return got
+
+    def add(li, share):
+        nonlocal slot
+        for kind, rows in share[0]:
+            t = tasks.setdefault(kind, ([], [], []))
+            t[0].append(rows)
+            t[1].append(li)
+            t[2].append(slot)
+        slot += share[1]
+
     leaves = list(it.leaves) if it.phase2 and not it.diag else []
+    nflat = _flat_chunks(it.p.numel())
+    flat = np.arange(nflat)
     if not it.phase2:
-        for c in range(_flat_chunks(it.p.numel())):
-            add("adam", (0, c, 0, slot))
-            slot += 1
+        add(0, ([("adam", _flat_tasks(flat, 0, flat))], nflat))
         rng = (0, slot, slot, slot)
     elif it.diag:
-        # up to a few chunks: quarters, each a task (Chunk in elementwise.hip)
-        n, chunks = it.p.numel(), _flat_chunks(it.p.numel())
-        quarter = L.FLAT_CHUNK // 4
-        parts = ([(c, q + 1) for c in range(chunks) for q in range(4)
-                  if c * L.FLAT_CHUNK + q * quarter < n] if chunks <= DIAG_SPLIT_CHUNKS
-                 else [(c, 0) for c in range(chunks)])
-        for c, q in parts:
-            add("dred", (0, c, q, slot))
-            slot += 1
+        # up to a few chunks: quarters, each a task (QuarterChunk in elementwise.hip)
+        c, q = flat, 0
+        if nflat <= DIAG_SPLIT_CHUNKS:
+            nq = -(-it.p.numel() // (L.FLAT_CHUNK // 4))
+            c, q = np.arange(nq) // 4, np.arange(nq) % 4 + 1
+        add(0, ([("dred", _flat_tasks(c, q, np.arange(len(c))))], len(c)))
         pre_end = slot
-        for c, q in parts:
-            add("dapply", (0, c, q, slot))
-            slot += 1
+        add(0, ([("dapply", _flat_tasks(c, q, np.arange(len(c))))], len(c)))
         rng = (0, pre_end, pre_end, slot)
     else:
-        # projection (chunk 0 owns the norm slots)
-        for li, (leaf, r0, c0l) in enumerate(leaves):
-            if not leaf.use_kronecker:
-                continue
-            m, n = leaf.m, leaf.n
-            k = _leaf_k(leaf)
-            parts, rows, _ = _leaf_split(leaf, plan)
-            # a whole tile's lanes address their rows with a 32-bit byte
-            # offset: 24 row strides + a strip, below 2^32 for rows under 2^25
-            typed = (it.fp32 or it.half) and _cols(it.p) < (1 << 25)
-            for j0 in range(0, n, L.PROJ_COLS):
-                for part in range(parts):
-                    nrows = min(rows, m - part * rows)
-                    whole = typed and j0 + L.PROJ_COLS <= n and nrows % PROJ_CHUNK == 0
-                    # 128 or 256 rows of T per task where k allows (variant bits 4, 8)
-                    cr = 64
-                    if whole and k % 128 == 0:
-                        cr = 256 if k % 256 == 0 else 128
-                    for c0 in range(0, k, cr):
-                        do_p = c0 == 0 and it.lars
-                        var = ((1 | (it.half << 4) if whole else 0) | (2 if do_p else 0)
-                               | (4 if cr == 128 else 0) | (8 if cr == 256 else 0))
-                        b = c0 | (part << 16)
-                        if c0 == 0:
-                            add(f"proj{var}", (li, j0, b, slot))
-                            slot += 1
-                        else:
-                            add(f"proj{var}", (li, j0, b, -1))
-        for li, (leaf, _, _) in enumerate(leaves):
-            if not leaf.use_kronecker:
-                # a diagonal sub-block: its norm partials, 64x64 tiles
-                for a in range(0, leaf.m, 64):
-                    for b in range(0, leaf.n, 64):
-                        add("delta", (li, a, b, slot))
-                        slot += 1
-                continue
-            k = _leaf_k(leaf)
-            chunks = _leaf_split(leaf, plan)[2]
-            for b in range(0, k, 64):
-                for a in range(0, k, 64):
-                    for ch in range(chunks):
-                        add("dpart", (li, a, b | (ch << 16), -1))
-                for a in range(0, k, 16 if chunks else 64):
-                    add("delta", (li, a, b, slot))
-                    slot += 1
+        # a whole tile's lanes address their rows with a 32-bit byte offset:
+        # 24 row strides + a strip, below 2^32 for rows under 2^25
+        typed = (it.fp32 or it.half != 0) and _cols(it.p) < (1 << 25)
+        var = (1 if it.mgrad else 0) | (2 if it.lars else 0)
+        masked, lars = it.masked, it.lars
+        geo = [(lf.m, lf.n, _leaf_k(lf), _leaf_split(lf, plan)) for lf, _, _ in leaves]
+        for li, (m, n, k, (parts, rows, _)) in enumerate(geo):
+            if k:
+                add(li, block(_proj_tasks, m, n, k, parts, rows, typed, it.half, lars))
+        for li, (m, n, k, (_, _, chunks)) in enumerate(geo):
+            add(li, block(_delta_tasks, m, n, k, chunks))
         pre_end = slot
-        for li, (leaf, r0, c0l) in enumerate(leaves):
-            k = _leaf_k(leaf)
-            for i0 in range(0, leaf.m, 64):
-                for d0 in range(0, k, 64):
-                    add("lift", (li, i0, d0, -1))
-            var = (1 if it.mgrad else 0) | (2 if it.lars else 0)
-            # 16-bit data has wide and strip tiles, but no pipelined ones
-            pipe = k >= PIPE_MIN_RANK and k not in STRIP_RANKS
-            ok = leaf.use_kronecker and (it.fp32 or (it.half and not pipe))
-            typed = 64 if it.half else 0
-            m, n, T = leaf.m, leaf.n, L.APPLY_TILE
-            if ok and k in STRIP_RANKS:
-                # runs of strip tiles over the interior they tile exactly
-                sw, tr = (64, 128) if k == 256 else (128, 64)   # the kernel's strip_shape
-                mw, nw = m - m % tr, n - n % sw
-                if not (mw and nw):
-                    mw = nw = 0
-                wide = var | 4 | 16 | (32 if k == 128 else 0) | typed | (128 if it.masked else 0)
-                for i0, j0 in _strip_runs(mw, nw, tr, sw):
-                    add(f"apply{wide}", (li, i0, j0, slot))
-                    slot += min(L.APPLY_GROUP, (mw - i0) // tr)
-            else:
-                # wide 16x256 tiles over the interior that they tile exactly,
-                # masked 64x64 tiles over the right column strip and the
-                # bottom row strip
-                mw = m - m % L.APPLY_WIDE_ROWS if ok else 0
-                nw = n - n % L.APPLY_WIDE_COLS if ok else 0
-                if not (mw and nw):
-                    mw = nw = 0
-                wide = var | 4 | (8 if pipe else typed)
-                for i0, j0 in _wide_tiles(mw, nw, k, pipe):
-                    add(f"apply{wide}", (li, i0, j0, slot))
-                    slot += 1
-            for i0 in range(0, m, T):
-                for j0 in range(nw, n, T):
-                    add(f"apply{var}", (li, i0, j0, slot))
-                    slot += 1
-            for i0 in range(mw, m, T):
-                for j0 in range(0, nw, T):
-                    add(f"apply{var}", (li, i0, j0, slot))
-                    slot += 1
+        for li, (m, n, k, _) in enumerate(geo):
+            add(li, block(_apply_tasks, m, n, k, it.fp32, it.half, var, masked))
         rng = (0, pre_end, pre_end, slot)
     if it.phase2 and it.lars:
-        for c in range(_flat_chunks(it.p.numel())):
-            add("lars", (0, c, 0, -1))
-    arrays = {k: np.array(v, dtype=np.int32).reshape(-1, 4) for k, v in tasks.items()}
+        add(0, ([("lars", _flat_tasks(flat, 0, -1))], 0))
+    arrays = {kind: _place(*t) for kind, t in tasks.items()}
     return arrays, rng, slot, leaves
+
+
+def _place(rows: list, index: list, slot: list) -> np.ndarray:
+    """Groups of task rows as one array, each group's indices and slots (of
+    the rows that own one) moved by its offsets."""
+    if len(rows) == 1:
+        a = rows[0].copy()
+        idx, off = index[0], slot[0]
+    else:
+        a = np.concatenate(rows)
+        idx, off = np.repeat(np.array((index, slot), dtype=np.int32), [len(r) for r in rows],
+                             axis=1)
+    a[:, 0] += idx
+    a[:, 3] += (a[:, 3] >= 0) * off
+    return a
 
 
 def _item_key(it: PItem) -> tuple:
@@ -473,39 +537,35 @@ def _build_structure(items: list[PItem], cache: dict | None = None):
     knobs = (PIPE_MIN_RANK, L2_OPERANDS, L.APPLY_GROUP, plan)
     if cache is not None and len(cache) > 4 * len(items) + 64:
         cache.clear()
-    parts = {k: [] for k in _TASK_TYPES}
-    offs = {k: [] for k in _TASK_TYPES}    # (index offset, slot offset, rows) per part
+    tasks = {}   # kind -> ([rows], [index offset], [slot offset])
+    made = {}    # block geometry -> rows (_param_tasks)
     ranges, leaves = [], []
     slot = 0
     for pi, it in enumerate(items):
         key = (_item_key(it), knobs)
         frag = cache.get(key) if cache is not None else None
         if frag is None:
-            frag = _param_tasks(it, plan)
+            frag = _param_tasks(it, plan, made)
             if cache is not None:
                 cache[key] = frag
         arrays, rng, nslot, lvs = frag
         base = len(leaves)
         for kind, arr in arrays.items():
-            parts[kind].append(arr)
-            offs[kind].append((base if (kind in _LEAF_TASKS or kind.startswith(("proj", "apply")))
-                               else pi, slot, len(arr)))
+            t = tasks.setdefault(kind, ([], [], []))
+            t[0].append(arr)
+            t[1].append(base if (kind in _LEAF_TASKS or kind.startswith(("proj", "apply")))
+                        else pi)
+            t[2].append(slot)
         ranges.append(tuple(x + slot for x in rng))
         leaves.extend((lf, r0, c0, pi) for lf, r0, c0 in lvs)
         slot += nslot
-    arrays = {}
-    for kind in _TASK_TYPES:
-        if parts[kind]:
-            a = np.concatenate(parts[kind])
-            o = np.array(offs[kind], dtype=np.int64)
-            a[:, 0] += np.repeat(o[:, 0], o[:, 2]).astype(np.int32)
-            a[:, 3] += np.where(a[:, 3] >= 0, np.repeat(o[:, 1], o[:, 2]), 0).astype(np.int32)
-        else:
-            a = np.zeros((0, 4), np.int32)
+    arrays = dict.fromkeys(_TASK_TYPES, np.zeros(0, dtype=L.TASK))
+    for kind, t in tasks.items():
+        a = _place(*t)
         if kind.startswith("apply") or kind.startswith("proj"):
             grp = L.APPLY_GROUP if kind.startswith("apply") and int(kind[5:]) & 8 else 1
             a = _xcd_interleave(a, grp)
-        arrays[kind] = np.ascontiguousarray(a, dtype=np.int32).view(L.TASK).reshape(-1)
+        arrays[kind] = np.ascontiguousarray(a).view(L.TASK).reshape(-1)
     return arrays, ranges, slot, leaves
 
 
@@ -636,55 +696,43 @@ def _padded_factors(leaves, ws: Workspace) -> dict:
     return out
 
 
-def _leaf_table(leaves, items: list[PItem], ws: Workspace):
+def _leaf_table(leaves, items: list[PItem], ws: Workspace, splits: list | None = None):
     """Block descriptors plus T/Delta/W scratch for every Phase-2 block (T and
-    Delta followed by the planes of a split reduction, _split_plan)."""
-    plan = _split_plan([lf for lf, *_ in leaves])
-    sizes = []
-    for (leaf, r0, c0, pi) in leaves:
-        k = _leaf_k(leaf)
-        parts, _, chunks = _leaf_split(leaf, plan)
+    Delta followed by the planes of a split reduction; ``splits``: the blocks'
+    _leaf_splits)."""
+    if splits is None:
+        splits = _leaf_splits(leaves)
+    sizes, ks = [], []
+    for (leaf, *_), (parts, _, chunks) in zip(leaves, splits):
+        m, n, k = leaf.m, leaf.n, _leaf_k(leaf)
+        ks.append(k)
         # W, then (strip-apply ranks) its three bf16 planes: 1.5 floats per element
-        wsz = _align4(leaf.m * k) + (_align4((3 * leaf.m * k + 1) // 2) if k in STRIP_RANKS else 0)
-        sizes.append((_align4(k * leaf.n) * (1 + parts if parts > 1 else 1),
+        wsz = _align4(m * k) + (_align4((3 * m * k + 1) // 2) if k in STRIP_RANKS else 0)
+        sizes.append((_align4(k * n) * (1 + parts if parts > 1 else 1),
                       _align4(k * k) * (1 + chunks), wsz))
     total = sum(a + b + c for a, b, c in sizes)
     scratch = ws.buf("leaf_scratch", max(total, 1) * 4)
-    base = scratch.data_ptr()
+    at = scratch.data_ptr()
     pads = _padded_factors(leaves, ws)
-    tab = np.zeros(len(leaves), dtype=L.LEAF_DESC)
-    off = 0
-    for i, ((leaf, r0, c0, pi), (st, sd, sw)) in enumerate(zip(leaves, sizes)):
-        it = items[pi]
-        cols = it.graw.shape[-1] if it.graw.ndim == 2 else to_2d(it.graw)[0].shape[1]
-        e = tab[i]
-        e["off"] = r0 * cols + c0
-        e["ld"] = cols
-        e["param"] = pi
+    rows = []
+    for i, ((leaf, r0, c0, pi), k, (st, sd, sw), (parts, _, chunks)) in enumerate(
+            zip(leaves, ks, sizes, splits)):
+        m, n = leaf.m, leaf.n
+        g = items[pi].graw
+        cols = g.shape[-1] if g.ndim == 2 else to_2d(g)[0].shape[1]
         if not leaf.use_kronecker:
             # diagonal sub-block: its EMA in Sl, the bias factor in dbias
-            e["Sl"] = leaf.diag_ema.data_ptr()
-            e["m"], e["n"], e["k"] = leaf.m, leaf.n, 0
-            e["flags"] = L.LF_DIAG
-            e["dbias"] = getattr(leaf, "_diag_bias_factor", 1.0)
+            rows.append((0, 0, leaf.diag_ema.data_ptr(), 0, 0, 0, 0, r0 * cols + c0, cols, pi,
+                         m, n, 0, L.LF_DIAG, getattr(leaf, "_diag_bias_factor", 1.0), 0))
             continue
-        k = _leaf_k(leaf)
-        if k == leaf.U_l.shape[1]:
-            e["Ul"], e["Ur"] = leaf.U_l.data_ptr(), leaf.U_r.data_ptr()
-            e["Sl"], e["Sr"] = leaf.S_l.data_ptr(), leaf.S_r.data_ptr()
-        else:
-            ul, ur, sl, sr = pads[i]
-            e["Ul"], e["Ur"], e["Sl"], e["Sr"] = (ul.data_ptr(), ur.data_ptr(), sl.data_ptr(),
-                                                  sr.data_ptr())
-        e["T"] = base + 4 * off
-        e["Delta"] = base + 4 * (off + st)
-        e["W"] = base + 4 * (off + st + sd)
-        e["Wb"] = base + 4 * (off + st + sd + _align4(leaf.m * k)) if k in STRIP_RANKS else 0
-        off += st + sd + sw
-        e["m"], e["n"], e["k"] = leaf.m, leaf.n, k
-        parts, _, chunks = _leaf_split(leaf, plan)
-        e["flags"] = (parts << L.LF_NSPLIT_SHIFT) | (chunks << L.LF_DCHUNK_SHIFT)
-    return tab
+        ul, ur, sl, sr = pads.get(i) or (leaf.U_l, leaf.U_r, leaf.S_l, leaf.S_r)
+        T, D, W = at, at + 4 * st, at + 4 * (st + sd)
+        rows.append((ul.data_ptr(), ur.data_ptr(), sl.data_ptr(), sr.data_ptr(), T, D, W,
+                     r0 * cols + c0, cols, pi, m, n, k,
+                     (parts << L.LF_NSPLIT_SHIFT) | (chunks << L.LF_DCHUNK_SHIFT), 0.0,
+                     W + 4 * _align4(m * k) if k in STRIP_RANKS else 0))
+        at += 4 * (st + sd + sw)
+    return np.array(rows, dtype=L.LEAF_DESC)
 
 
 # --------------------------------------------------------------------------
@@ -922,12 +970,12 @@ def run_step(items: list[PItem], ws: Workspace, update_norm_ema: bool,
                     upd_offsets[i] = off
                     off += _align4(it.p.numel())
             ent = ({k: (L.upload(v, dev) if len(v) else None) for k, v in arrays.items()},
-                   {k: len(v) for k, v in arrays.items()}, ranges, nslots, leaves, upd_offsets,
-                   off)
+                   {k: len(v) for k, v in arrays.items()}, ranges, nslots, leaves,
+                   _leaf_splits(leaves), upd_offsets, off)
         ws.recent[skey] = ent
         while len(ws.recent) > RECENT_STRUCTURES:
             ws.recent.pop(next(iter(ws.recent)))
-        (ws.tasks, ws.ntasks, ws.slot_ranges, ws.nslots, ws.leaves, ws.upd_offsets,
+        (ws.tasks, ws.ntasks, ws.slot_ranges, ws.nslots, ws.leaves, ws.splits, ws.upd_offsets,
          ws.upd_total) = ent
         ws.struct_key = skey
         ws.leaf_epoch = -1
@@ -936,7 +984,7 @@ def run_step(items: list[PItem], ws: Workspace, update_norm_ema: bool,
     # the block table holds no gradient pointer: a gradient that moves keeps
     # it valid
     if ws.leaf_epoch != leaf_epoch() or ws.leaf_dev is None:
-        tab = _leaf_table(ws.leaves, items, ws)
+        tab = _leaf_table(ws.leaves, items, ws, ws.splits)
         ws.leaf_dev = L.upload(tab, dev) if len(tab) else None
         ws.leaf_epoch = leaf_epoch()
     raw, classes = _param_table(items, ws.slot_ranges, ws, gsnr)

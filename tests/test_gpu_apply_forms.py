@@ -119,8 +119,8 @@ def test_flat_tasks_do_not_read_b(hip_device, monkeypatch, dtype, phase2):
                sparsity=0.0, noise_std_init=0.0, lookahead_k=0, k_min=8, k_max=8)
     plain = E._param_tasks
 
-    def marked(it, plan):
-        arrays, *rest = plain(it, plan)
+    def marked(*args):
+        arrays, *rest = plain(*args)
         arrays = {kind: arr.copy() for kind, arr in arrays.items()}
         for kind in ("adam", "lars"):
             if kind in arrays:

@@ -4,6 +4,8 @@ keep what each kernel variant promises.  CPU only."""
 
 from __future__ import annotations
 
+import sys
+
 import pytest
 import torch
 
@@ -88,3 +90,61 @@ def test_cut_follows_the_number_of_tasks():
     plan = E._split_plan([lf for it in small for lf, _, _ in it.leaves])
     assert plan.rows == E.SPLIT_MIN_ROWS and plan.chunks
     assert E._split_plan([lf for it in big for lf, _, _ in it.leaves]).rows == 0
+
+
+@pytest.mark.parametrize("shapes", [[(768, 2304), (768, 768)], [(2048, 2048)] * 4])
+def test_structure_costs_no_python_call_per_task(shapes):
+    """A step structure is array arithmetic: the Python calls of building it
+    grow with its blocks (some fifty each, and the helpers of a type), not with
+    its thousands of task rows; the block table takes the splits the structure
+    was built with instead of working them out again."""
+    items = _items(shapes, 64, 2048, False)
+    arrays, _, _, leaves = E._build_structure(items)
+    rows = sum(len(a) for a in arrays.values())
+    calls = 0
+
+    def count(frame, event, arg):
+        nonlocal calls
+        calls += event == "call"
+
+    sys.setprofile(count)
+    try:
+        E._build_structure(items)
+    finally:
+        sys.setprofile(None)
+    assert calls < 600 + 60 * len(leaves) < rows, (calls, rows)
+    splits = E._leaf_splits(leaves)
+    ws = E.Workspace(torch.device("cpu"))
+    want = E._leaf_table(leaves, items, ws)
+    with pytest.MonkeyPatch.context() as mp:
+        mp.setattr(E, "_split_plan", None)
+        mp.setattr(E, "_leaf_split", None)
+        assert E._leaf_table(leaves, items, ws, splits).tobytes() == want.tobytes()
+
+
+@pytest.mark.parametrize("first", [True, False])
+def test_slots_of_mixed_parameters(first):
+    """Parameters with and without LARS, ragged ones among them, in either
+    order: each reduction slot is written once (a strip run writes several)."""
+    shapes = [(100, 300), (512, 768), (33, 257), (640, 512)]
+    for k in (64, 128, 256):
+        items = _items(shapes, k, 512, False)
+        for i, it in enumerate(items):
+            it.lars = (i % 2 == 0) == first
+        arrays, ranges, nslots, leaves = E._build_structure(items)
+        writes = [0] * nslots
+        for kind, arr in arrays.items():
+            var = int(kind[5:]) if kind.startswith("apply") else 0
+            for t in arr:
+                s = int(t["slot"])
+                if s < 0:
+                    continue
+                n = 1
+                if var & 16:
+                    tr = 64 if var & 32 else 128
+                    m = leaves[int(t["idx"])][0].m
+                    n = min(L.APPLY_GROUP, (m - m % tr - int(t["a"])) // tr)
+                for q in range(s, s + n):
+                    writes[q] += 1
+        assert writes == [1] * nslots
+        assert ranges[-1][3] == nslots
