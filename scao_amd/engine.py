@@ -244,9 +244,11 @@ _PROJ_VARIANTS = [0, 2] + [1 | p | w | t for t in (0, 16, 32) for w in (0, 4, 8)
 # | 128: strip tiles whose moments see the filtered gradient without noise
 _APPLY_VARIANTS = ([t | v for t in (0, 4, 12, 20, 52, 68, 84, 116) for v in range(4)]
                    + [128 | t | v for t in (20, 52, 84, 116) for v in (1, 3)])
-_TASK_TYPES = (["adam", "dpart", "delta", "lift", "dred", "dapply", "lars"] +
-               [f"proj{v}" for v in sorted({*range(12), *_PROJ_VARIANTS})] +
-               [f"apply{v}" for v in sorted({*range(64), *_APPLY_VARIANTS})])
+# what _launch_step launches; a structure holds no task of another type
+_LAUNCHED = frozenset(["adam", "dpart", "delta", "lift", "dred", "dapply", "lars"] +
+                      [f"proj{v}" for v in _PROJ_VARIANTS] +
+                      [f"apply{v}" for v in _APPLY_VARIANTS])
+_TASK_TYPES = sorted(_LAUNCHED | {f"proj{v}" for v in range(12)} | {f"apply{v}" for v in range(64)})
 
 
 DIAG_SPLIT_CHUNKS = 64         # 1-D parameters up to this many chunks take quarter tasks
@@ -561,6 +563,8 @@ def _build_structure(items: list[PItem], cache: dict | None = None):
         slot += nslot
     arrays = dict.fromkeys(_TASK_TYPES, np.zeros(0, dtype=L.TASK))
     for kind, t in tasks.items():
+        if kind not in _LAUNCHED:
+            raise RuntimeError(f"no launch takes tasks of type {kind!r}")
         a = _place(*t)
         if kind.startswith("apply") or kind.startswith("proj"):
             grp = L.APPLY_GROUP if kind.startswith("apply") and int(kind[5:]) & 8 else 1

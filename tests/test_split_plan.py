@@ -148,3 +148,19 @@ def test_slots_of_mixed_parameters(first):
                     writes[q] += 1
         assert writes == [1] * nslots
         assert ranges[-1][3] == nslots
+
+
+def test_a_task_type_without_a_launch_is_an_error(monkeypatch):
+    """Tasks filed under a variant that the step does not launch would leave
+    their part of a parameter as it was, silently."""
+    items = _items([(300, 300)], 64, 512, False)
+    E._build_structure(items)
+    plain = E._apply_tasks
+
+    def misfiled(*args):
+        tasks, slots = plain(*args)
+        return [("apply9" if kind == "apply2" else kind, t) for kind, t in tasks], slots
+
+    monkeypatch.setattr(E, "_apply_tasks", misfiled)
+    with pytest.raises(RuntimeError, match="apply9"):
+        E._build_structure(items)
