@@ -17,7 +17,8 @@ pytestmark = pytest.mark.gpu
 # k, shapes: widths on both sides of the tiles of each kernel (16 x 256 wide;
 # 64 x 128 and 128 x 64 strips; 64 x 64 masked), odd row strides, chunks of 4096
 CASES = [(64, [(32, 512), (33, 257), (17, 300)]), (128, [(64, 256), (129, 385)]),
-         (256, [(512, 512), (300, 515)]), (320, [(640, 700)]), (24, [(65, 1003), (4097,), (5,)])]
+         (256, [(512, 512), (300, 515)]), (320, [(640, 700)]), (24, [(65, 1003), (4097,), (5,)]),
+         (320, [(400, 515)])]
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
