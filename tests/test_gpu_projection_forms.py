@@ -139,3 +139,44 @@ def test_step_projection_and_delta(hip_device, dtype, shapes, k):
     for x, st in zip(grads, np.frombuffer(stat, dtype=L.PARAM_STAT)):
         want = x.double().square().sum().item()
         assert abs(float(st["g2"]) - want) <= 1e-6 * want
+
+
+def test_cut_of_the_sums_changes_rounding_only(hip_device):
+    """A step cuts the sums of its projection and delta stages by how many
+    blocks it has, so a parameter steps with other roundings alone than beside
+    308 blocks more: 1e-6 in the 2-norm of its moments (an fp32 sum of 512
+    terms, in one chain or in parts, is within 2^-24 times a few of 512^0.5 of
+    it), and the same bits each time in the same company."""
+    from scao_amd import engine as E
+    g = torch.Generator().manual_seed(2)
+    init = [0.02 * _rand(g, 512, 512), 0.02 * _rand(g, 308 * 256, 256)]
+    grads = [1e-3 * _rand(g, *x.shape) for x in init]
+    factors = [_rand(g, 256, 64) / 16.0 for _ in range(8)]
+    spectra = [1e-3 * (0.1 + torch.rand(64, generator=g)) for _ in range(8)]
+
+    def run(n):
+        params = [torch.nn.Parameter(x.to(hip_device)) for x in init[:n]]
+        opt = scao_amd.SCAO(params, k_min=64, k_max=64, warmup_steps=0, min_precond_updates=0,
+                            precond_freq=10 ** 9, max_precond_dim=256, sparsity=0.0,
+                            noise_std_init=0.0, lookahead_k=0, blend_steps=0)
+        for p, x in zip(params, grads):
+            p.grad = x.to(hip_device)
+            opt._init_state(p, opt.param_groups[0])
+        for i, (leaf, _, _) in enumerate(opt.state[params[0]]["preconditioner"].leaves()):
+            leaf.U_l, leaf.U_r = (factors[2 * i + j].to(hip_device) for j in range(2))
+            leaf.S_l, leaf.S_r = (spectra[2 * i + j].to(hip_device) for j in range(2))
+            leaf._touch()
+        opt.step()
+        torch.cuda.synchronize()
+        st = opt.state[params[0]]
+        plan = E._split_plan([lf for lf, *_ in opt._ws.leaves])
+        return plan, [params[0].detach()] + [st[key] for key in
+                                             ("exp_avg", "exp_avg_sq", "exp_avg_diff")]
+
+    alone, few = run(1)
+    beside, many = run(2)
+    assert alone.rows and alone.chunks and not beside.rows and not beside.chunks
+    for a, b in zip(few, many):
+        assert ((a - b).double().norm() / a.double().norm()).item() < 1e-6
+    for n, first in ((1, few), (2, many)):
+        assert all(torch.equal(a, b) for a, b in zip(first, run(n)[1]))
