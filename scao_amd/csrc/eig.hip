@@ -2381,9 +2381,14 @@ extern "C" int scao_eig_bisect(const double* d, const double* e, int n, int batc
   double* e2 = info + 5 * (int64_t)batch;     // after nneg's batch 8-byte slots
   hipLaunchKernelGGL(k_tri_info, dim3(batch), dim3(256), 0, s, d, e, n, info, nneg, e2);
   SCAO_LAUNCH_CHECK("scao_eig_bisect/info");
-  // few matrices: many lanes per eigenvalue (k_bisect); 8 n / 64 waves for the
-  // negative ones and kq / 4 for the largest leave a SIMD about one wave each
-  // up to some 16 matrices of 2048 rows
+  // few matrices: many lanes per eigenvalue (k_bisect).  Up to 64 K rows of
+  // batch that is the faster form at every size measured, kq = 64 (many lanes /
+  // few, all eigenvalues positive | half of them negative, ms):
+  //    rows    64 K rows of batch          128 K                  256 K
+  //     256   0.46/0.50 | 0.72/0.94   0.81/0.64 | 1.4/1.6    1.6/1.1 | 2.7/2.4
+  //    1024   0.68/1.9  | 1.7/3.1     0.85/1.9  | 2.9/3.6    1.7/1.9 | 5.4/4.7
+  //    4096   2.6/7.3   | 5.9/12.2    2.6/7.4   | 9.8/12.2   2.7/7.4 | 18/16
+  // Past it the lines cross at a batch that follows rows, rank and signs.
   if ((int64_t)batch * n <= 64 * 1024) {
     const int nwave = bisect_waves(kq, 16) + bisect_waves(n - kq, 8);
     hipLaunchKernelGGL((k_bisect<16, 1, 8>), dim3(batch, (nwave + 3) / 4), dim3(256), 0, s, d, e2,

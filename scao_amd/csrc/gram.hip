@@ -990,6 +990,8 @@ extern "C" int scao_eig_diag(const scao_prep_desc* descs, int ndescs, int n, int
   return SCAO_OK;
 }
 
+// More than the kernels use (a maximum per block, at most EMA_BLOCKS floats):
+// the size that callers have always been told.
 extern "C" int64_t scao_int8_ema_scratch_bytes(int64_t n) {
   if (n <= 0) return 0;
   const int64_t parts = (n + SCAO_FLAT_CHUNK - 1) / SCAO_FLAT_CHUNK;

@@ -588,7 +588,8 @@ __device__ __forceinline__ void delta_tile(const scao_leaf_desc& L, float eps, i
 // rounded up to 64 columns (the chunks' shares of P then take as much memory
 // as T), one workgroup each.  64 columns of T at a time are staged through LDS
 // as floats: there the planes of a row-split projection are added in order
-// (b0 = 0 tasks also write the sum to T itself).  Wave w takes rows 16w .. +15
+// (b0 = 0 tasks also write the sum to T, which then holds U_l^T G whatever the
+// cut; no later kernel reads it).  Wave w takes rows 16w .. +15
 // of the tile on six bf16 products per fp32 product and writes them to the
 // chunk's plane; delta_finish adds the chunks.  tplanes and pplanes: the row
 // parts' planes of T and the chunks' planes of P.
@@ -938,7 +939,7 @@ __device__ __forceinline__ void lift_tile(const scao_leaf_desc& L, int i0, int d
   }
 }
 
-// The same tile for k % 128 == 0 on whole, aligned tiles, with the products on
+// The same tile for k % 128 == 0 on whole tiles, with the products on
 // the bf16 matrix cores (mm64_x6): wave w takes the whole 64 x 64 tile over
 // its quarter of k (a multiple of 32), the four partial tiles go through LDS,
 // and wave w adds rows 16w .. 16w + 15 of them in order (((w0 + w1) + w2) + w3)
@@ -2119,8 +2120,11 @@ __device__ __forceinline__ void apply_out_tile(const scao_leaf_desc& L, const fl
 // The same for 64 rows x 256 columns at k = 64, 64 x 64 per wave: a wave keeps
 // its columns' U_r rows in registers for four 16-row tiles, so the operands
 // it reads from L2 (32 KB) are half what the tile streams, against two and a
-// half times for 16 rows.  Worth it where the tiles still cover the CUs:
-// 2048 x 2048 17.6 -> 14.6 us.
+// half times for 16 rows.  Taken from 128 of its tiles, half the CUs, on (whole
+// operator, 64 x 64 tiles / this: 64 tiles 31 / 35 us, 128 36 / 38, 225 58 / 53,
+// 256 (2048 x 2048) 48 / 42, 1024 101 / 79).  Written for the one width: 64
+// registers of U_r rows; at 128 they would be 128 beside the double-buffered W
+// and G.
 __device__ __forceinline__ void apply_out_wide(const scao_leaf_desc& L, const float* G, float* out,
                                                int i0, int j0) {
   const int w = threadIdx.x / 64, l = threadIdx.x % 64;

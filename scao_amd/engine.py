@@ -25,8 +25,8 @@ The curvature refresh (``refresh``) batches every block due for an update:
 Gram -> EMA -> requantise on the GPU (no host round trip for the int8
 scale), then the eigen stage on stacked equal-size matrices
 (``scao_amd.eigen.topk_eigh``: the k_max largest eigenpairs and the sum of
-the clamped spectrum) and the adaptive-rank choice with one host read of all
-ranks.
+the clamped spectrum) and the adaptive-rank choice on the host from one read of
+all spectra.
 """
 
 from __future__ import annotations
@@ -251,7 +251,11 @@ _LAUNCHED = frozenset(["adam", "dpart", "delta", "lift", "dred", "dapply", "lars
 _TASK_TYPES = sorted(_LAUNCHED | {f"proj{v}" for v in range(12)} | {f"apply{v}" for v in range(64)})
 
 
-DIAG_SPLIT_CHUNKS = 64         # 1-D parameters up to this many chunks take quarter tasks
+# 1-D parameters up to this many chunks take quarter tasks: reduce and apply
+# together 23 -> 15 us at one chunk, 25 -> 17 at 64, 26 -> 18 at 128, 36 -> 32 at
+# 512, 88 -> 84 at 2048.  Past 64 chunks the gain is a small share and four slots
+# a chunk would be the finalize kernel's to add.
+DIAG_SPLIT_CHUNKS = 64
 STEP_WIDTHS = (64, 128, 256)   # eigenfactor widths the step kernels are built for
 
 
@@ -291,7 +295,16 @@ def _split_plan(leaves) -> SplitPlan:
     split into parts (the largest that give every CU work: two workgroups of
     the 64-row kernel, one of the wider ones), and P is formed by column
     chunks.  Both write planes that the delta stage adds in order, which costs
-    one more pass over T and P, so a step that fills the chip takes neither."""
+    one more pass over T and P, so a step that fills the chip takes neither:
+    projection and delta stage, whole / cut in us, by the share of the CUs that
+    whole tasks would fill,
+        share                    0.25       0.5        0.6        0.75       1.0
+        1024 x 1024, k = 64    110 / 78   132 / 130  178 / 171  190 / 188  222 / 224
+        2048 x 2048, k = 64    187 / 123  226 / 216  304 / 284  327 / 311  392 / 417
+        2048 x 2048, k = 128   219 / 93   241 / 158  250 / 257  275 / 275  284 / 305
+        4096 x 4096, k = 256   599 / 230  646 / 423  669 / 593  664 / 645  693 / 855
+    Up to 0.6 the cut gains or is even; past it the gain is a few per cent and
+    turns over before 1."""
     tasks = []   # (rows, strips, CU share of a task) per block
     tiles = 0
     for lf in leaves:
@@ -1290,9 +1303,11 @@ def eigen_route(dim: int, diagonal: bool) -> str:
 #     2560    56 /  56    57 /  69
 #     3072    77 /  73    78 /  91
 #     4096   128 / 109   130 / 152
-# One matrix of at least 2048 rows goes to the library (the lines cross near
-# 2560 rows), two go to the solver.  Two of 4096 rows and more keep the
-# library's route, which tests/test_host_logic.py states.
+# One matrix of at least 2048 rows goes to the library, two go to the solver but
+# for two of 4096 rows and more.  The lines cross near 2560 rows for one matrix
+# and not below 4096 for two: one of 2048 to 2560 rows and two of 4096 keep the
+# library, up to a tenth and a sixth slower, because that was their route before
+# the table was measured and tests/test_host_logic.py states it.
 LIBRARY_MIN_DIM = 2048
 LIBRARY_PAIR_DIM = 4096
 
