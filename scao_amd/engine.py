@@ -742,7 +742,8 @@ def _leaf_table(leaves, items: list[PItem], ws: Workspace, splits: list | None =
             rows.append((0, 0, leaf.diag_ema.data_ptr(), 0, 0, 0, 0, r0 * cols + c0, cols, pi,
                          m, n, 0, L.LF_DIAG, getattr(leaf, "_diag_bias_factor", 1.0), 0))
             continue
-        ul, ur, sl, sr = pads.get(i) or (leaf.U_l, leaf.U_r, leaf.S_l, leaf.S_r)
+        ul, ur, sl, sr = ((leaf.U_l, leaf.U_r, leaf.S_l, leaf.S_r) if k == leaf.U_l.shape[1]
+                          else pads[i])
         T, D, W = at, at + 4 * st, at + 4 * (st + sd)
         rows.append((ul.data_ptr(), ur.data_ptr(), sl.data_ptr(), sr.data_ptr(), T, D, W,
                      r0 * cols + c0, cols, pi, m, n, k,
